@@ -54,7 +54,8 @@ def build_lib() -> pathlib.Path:
     LIB_DIR.mkdir(exist_ok=True)
     cc = hipcc()
     objs = []
-    for src, device in (("gemv_kernels.hip", True), ("dmc_hip_runtime.cpp", False), ("npz_ingress.cpp", False)):
+    for src, device in (("gemv_kernels.hip", True), ("gemm_kernels.hip", True),
+                        ("dmc_hip_runtime.cpp", False), ("npz_ingress.cpp", False)):
         obj = OBJ / (src.rsplit(".", 1)[0] + ".o")
         lang = ["-x", "hip"] + DEVICE if device else ["-D__HIP_PLATFORM_AMD__"]
         _run([cc, *COMMON, *lang, "-c", str(CSRC / src), "-o", str(obj)])

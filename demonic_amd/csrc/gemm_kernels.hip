@@ -1,0 +1,457 @@
+// gemm_kernels.hip -- the MFMA "gemm" layout: bf16 weights against 9 and more
+// f32 activation rows (prefill and large decode batches), W [N,K].
+#include "gemv_device.h"
+#include "gemv_launch.h"
+
+#include <algorithm>
+#include <type_traits>
+
+namespace dmc {
+namespace {
+
+// A workgroup of NWV waves owns 32 * NWV weight rows against MT activation
+// rows, so W streams from HBM once per MT rows (the 16-row layouts stream it
+// once per 16).  k advances in chunks of 64: each weight row's chunk is one
+// 128-byte line.  x enters as three bf16 terms (split3), either split by the
+// workgroup on the way into LDS (FUSE) or once per call by
+// split_x_planes_kernel into planes XS [3][M][K].
+//
+// What bounds it: from MT = 64 the matrix cores (3 MFMAs per product), whose
+// clock falls under load (operands that are not zero run this MFMA at 1.94
+// PFLOP/s out of registers, 2.4 with zeros), below that HBM.  Every wave
+// taking its LDS reads, its MFMAs, its stores and a barrier in turn left the
+// matrix cores ~30% busy, since the eight waves do each phase together.  So
+// the operands of the next step are read from LDS while this step's MFMAs
+// run, across the barrier too:
+//   - a chunk is NS steps of (k-block of 32, 16 activation rows): RN MFMA
+//     tiles x 3 terms, 12 to 24 MFMAs, against 3 to 7 operand reads for the
+//     step after it in a second register set;
+//   - one barrier per chunk, ahead of its last step: the chunk after next's
+//     loads were stored to the other LDS buffer the step before, and the last
+//     step's operands are already in registers, so its MFMAs cover the
+//     barrier and the next chunk's first reads;
+//   - the WN x WM grid of waves gives each a near-square tile (64 rows x MT/2),
+//     7 to 10 operand reads per 24 MFMAs; W is shared through LDS like x;
+//   - loads are unconditional and the chunk loop has no exit in its body, so
+//     the compiler counts them instead of draining them (a `break` between
+//     two chunks cost 5-10%).
+// Measured, before (operand reads, MFMAs, stores and a barrier in turn; 64
+// rows at most) / now, us, same box: C2 up m = 512 235 / 164, C2 down m = 2048
+// 911 / 602 (1.2 PFLOP/s of MFMA; a large bf16 matrix product through the
+// vendor library reaches 1.25 on this card), up m = 64 47.2 / 38.3.
+//
+// When the tiles would leave the device short of workgroups, k is split over
+// `slices` workgroups of kc chunks each, whose partial sums go to
+// P[slice][m][n] for gemm_sum_slices_kernel.  Special values, tiny activation
+// rows and the zero rule are as in the other MFMA layouts; with slices the
+// zero rule runs after the sum.
+typedef f32x4 f32x4_u __attribute__((aligned(4)));  // y's rows may start at any float
+constexpr uint32_t kDeadLane = 0x80000000u;   // lane offset past every buffer: zeros, no traffic
+constexpr uint32_t kDeadChunk = 0x7fff0000u;  // scalar offset of a chunk past the last (no 32-bit wrap with kDeadLane)
+
+// The three bf16 terms of eight values by truncation alone: split3's terms for
+// every finite |x| >= 2^-133 and 0.  Of a smaller x nothing is left, and an inf
+// leaves a NaN in mid: rows that hold those are settled after the stream.
+__device__ __forceinline__ void split8_finite(const float (&v)[8], u32x4 (&t)[3]) {
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+        const uint32_t u0 = __float_as_uint(v[2 * q]), u1 = __float_as_uint(v[2 * q + 1]);
+        const float r10 = v[2 * q] - __uint_as_float(u0 & 0xffff0000u);
+        const float r11 = v[2 * q + 1] - __uint_as_float(u1 & 0xffff0000u);
+        const uint32_t b10 = __float_as_uint(r10), b11 = __float_as_uint(r11);
+        const uint32_t b20 = __float_as_uint(r10 - __uint_as_float(b10 & 0xffff0000u));
+        const uint32_t b21 = __float_as_uint(r11 - __uint_as_float(b11 & 0xffff0000u));
+        t[0][q] = (u0 >> 16) | (u1 & 0xffff0000u);
+        t[1][q] = (b10 >> 16) | (b11 & 0xffff0000u);
+        t[2][q] = (b20 >> 16) | (b21 & 0xffff0000u);
+    }
+}
+
+template <int NWV, int MT, bool FUSE>
+__global__ void __launch_bounds__(64 * NWV) __attribute__((amdgpu_waves_per_eu(MT == 16 ? 4 : 2)))
+gemv_rd_mfma_gemm_kernel(const uint16_t *__restrict__ W, const float *__restrict__ X, const uint16_t *__restrict__ XS,
+                         float *__restrict__ Y, float *__restrict__ P, int N, int K, int M, int kc, int gx, int gy,
+                         int xcd) {
+    static_assert(NWV == 4 || NWV == 8, "32 weight rows per wave");
+    static_assert(MT == 16 || MT == 32 || MT == 64 || MT == 128, "activation rows per workgroup");
+    constexpr int kRows = 32 * NWV;
+    constexpr int XT = MT / 16;                    // 16-row activation tiles
+    constexpr int WM = MT >= 64 ? 2 : (MT == 32 && NWV == 8) ? 2 : 1, WN = NWV / WM;
+    constexpr int RN = kRows / 16 / WN, RM = XT / WM;  // MFMA tiles per wave
+    constexpr int NS = 2 * RM;                     // steps per chunk
+    constexpr int XI = (2 * XT + NWV - 1) / NWV;   // x staging items (16 rows x 32 k) per wave
+    const int tid = threadIdx.x;
+    const int lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int i16 = lane & 15;
+    const int g = lane >> 4;
+    const int wn = wave % WN, wm = wave / WN;
+    // The tile from the linear workgroup id (a 1-D grid of gx * gy * slices).
+    // With `xcd` set, workgroup L, which runs on XCD L % 8 (the dispatcher
+    // deals workgroups to the 8 XCDs in turn), takes the L / 8-th tile of
+    // that XCD's contiguous share, activation tiles fastest, so the
+    // workgroups an XCD runs together share weight blocks through its L2;
+    // otherwise tiles go in launch order, consecutive weight blocks to
+    // different XCDs.
+    uint32_t lin = blockIdx.x;
+    if (xcd) {
+        const uint32_t x = lin & 7u, q = gridDim.x >> 3, r = gridDim.x & 7u;
+        lin = x * q + min(x, r) + (lin >> 3);
+    }
+    const int by = (int)(lin % (uint32_t)gy);
+    const int bx = (int)(lin / (uint32_t)gy % (uint32_t)gx);
+    const int bz = (int)(lin / (uint32_t)gy / (uint32_t)gx);
+    const int row0 = bx * kRows;
+    const int nrows = min(kRows, N - row0);
+    const int m0 = by * MT;
+    const int c0 = bz * kc;  // this slice's chunks: [c0, c0 + nch)
+    const int nch = max(0, min(K / 64, c0 + kc) - c0);
+
+    __shared__ __attribute__((aligned(16))) uint8_t wt[2][kRows * 128];  // swizzled 128-byte rows (swz)
+    __shared__ u32x4 xp[2][XT][2][3][64];                                // operand order: conflict-free
+
+    const __amdgpu_buffer_rsrc_t rs = weight_rsrc(W + (int64_t)row0 * K, (uint32_t)((int64_t)nrows * K * 2));
+    const uint32_t plane_bytes = (uint32_t)M * (uint32_t)K * 2u;
+    const __amdgpu_buffer_rsrc_t xrs = FUSE ? weight_rsrc(X, 2u * plane_bytes) : weight_rsrc(XS, 3u * plane_bytes);
+    // W staging: item j of a wave is rows 32 * wave + 8j + lane/8, 16 bytes per lane: whole lines.
+    const int slr = wave * 32 + (lane >> 3);
+    uint32_t woff[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+        woff[j] = (uint32_t)min(slr + 8 * j, nrows - 1) * (uint32_t)K * 2u + (lane & 7) * 16;
+    // x staging: item it = (tile it/2, k-block it%2), 8 elements of row i16 per lane.
+    uint32_t xoff[XI];
+#pragma unroll
+    for (int j = 0; j < XI; ++j) {
+        const int it = wave * XI + j;
+        const int xm = m0 + (it >> 1) * 16 + i16;
+        const uint32_t e = (uint32_t)xm * (uint32_t)K + (it & 1) * 32 + g * 8;
+        xoff[j] = it < 2 * XT && xm < M ? e * (FUSE ? 4u : 2u) : kDeadLane;
+    }
+    struct Regs {
+        u32x4 w[4];
+        u32x4 x[XI][FUSE ? 2 : 3];  // f32 halves, or the three planes
+    };
+    const int s0 = chunk_rotation(bx, nch);
+    auto load = [&](int c, Regs &r) __attribute__((always_inline)) {
+        const bool live = c < nch;
+        const uint32_t cb = (uint32_t)(c0 + rotate_chunk(c, s0, nch)) * 128u;
+        const uint32_t wb = live ? cb : kDeadChunk;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) r.w[j] = load_w16(rs, woff[j], wb);
+#pragma unroll
+        for (int j = 0; j < XI; ++j) {
+#pragma unroll
+            for (int q = 0; q < (FUSE ? 2 : 3); ++q)
+                r.x[j][q] = FUSE ? __builtin_amdgcn_raw_buffer_load_b128(xrs, xoff[j] + 16u * q,
+                                                                         live ? 2u * cb : kDeadChunk, 0)
+                                 : __builtin_amdgcn_raw_buffer_load_b128(xrs, xoff[j],
+                                                                         live ? q * plane_bytes + cb : kDeadChunk, 0);
+        }
+    };
+    uint32_t xmx[XI];  // the largest |x| staged (f32 bits; the hi term's with planes), per lane
+#pragma unroll
+    for (int j = 0; j < XI; ++j) xmx[j] = 0;
+    auto store = [&](const Regs &r, int buf, auto TERMS) __attribute__((always_inline)) {
+        constexpr int terms = decltype(TERMS)::value;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) *reinterpret_cast<u32x4 *>(wt[buf] + swz(slr + 8 * j, lane & 7)) = r.w[j];
+#pragma unroll
+        for (int j = 0; j < XI; ++j) {
+            const int it = wave * XI + j;
+            if (it >= 2 * XT) break;  // wave-uniform
+            u32x4 t[3];
+            if constexpr (FUSE) {
+                float v[8];
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    v[e] = __uint_as_float(r.x[j][0][e]);
+                    v[4 + e] = __uint_as_float(r.x[j][1][e]);
+                }
+                if constexpr (terms == 1) {
+                    split8(v, t[0], t[1], t[2]);
+                } else {
+                    split8_finite(v, t);
+#pragma unroll
+                    for (int e = 0; e < 8; ++e) xmx[j] = max(xmx[j], __float_as_uint(v[e]) & 0x7fffffffu);
+                }
+            } else {
+#pragma unroll
+                for (int q = 0; q < 3; ++q) t[q] = r.x[j][q];
+                if constexpr (terms == 3) {
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) xmx[j] = max_mag(xmx[j], t[0][e]);
+                }
+            }
+#pragma unroll
+            for (int q = 0; q < terms; ++q) xp[buf][it >> 1][it & 1][q][lane] = t[q];
+        }
+    };
+
+    f32x4 acc[RM][RN];
+    u32x4 a[2][RN], xo[2][3];  // operands: weights per k-block, x per step
+    auto read_a = [&](int buf, int kb) __attribute__((always_inline)) {
+#pragma unroll
+        for (int j = 0; j < RN; ++j)
+            a[kb][j] = *reinterpret_cast<const u32x4 *>(wt[buf] + swz((wn * RN + j) * 16 + i16, kb * 4 + g));
+    };
+    auto read_x = [&](int buf, int kb, int mf, int set) __attribute__((always_inline)) {
+#pragma unroll
+        for (int q = 0; q < 3; ++q) xo[set][q] = xp[buf][wm * RM + mf][kb][q][lane];
+    };
+    // LDS only: the global loads in flight stay in flight.
+    auto lds_barrier = [] { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); };
+
+    // Chunk c is in LDS buffer BUF and its first step's operands in registers;
+    // chunk c + 1 is in `r`, loaded a chunk ago.
+    Regs r;
+    auto chunk = [&](int c, auto BUF, auto TERMS) __attribute__((always_inline)) {
+        constexpr int buf = decltype(BUF)::value;
+#pragma unroll
+        for (int s = 0; s < NS; ++s) {
+            const int kb = s / RM, mf = s % RM;
+            if (s + 1 < NS) {
+                if ((s + 1) % RM == 0) read_a(buf, (s + 1) / RM);
+                read_x(buf, (s + 1) / RM, (s + 1) % RM, (s + 1) & 1);
+            }
+            if (s == NS - 2) {
+                store(r, buf ^ 1, TERMS);
+                load(c + 2, r);
+            }
+            if (s == NS - 1) {
+                lds_barrier();
+                read_a(buf ^ 1, 0);
+                read_x(buf ^ 1, 0, 0, 0);
+            }
+#pragma unroll
+            for (int q = 0; q < decltype(TERMS)::value; ++q)
+#pragma unroll
+                for (int j = 0; j < RN; ++j) acc[mf][j] = mfma_bf16(a[kb][j], xo[s & 1][q], acc[mf][j]);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    };
+    auto stream = [&](auto TERMS) __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < RM; ++i)
+#pragma unroll
+            for (int j = 0; j < RN; ++j) acc[i][j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+        load(0, r);
+        store(r, 0, TERMS);
+        load(1, r);
+        lds_barrier();
+        read_a(0, 0);
+        read_x(0, 0, 0, 0);
+        int c = 0;
+        for (; c + 1 < nch; c += 2) {
+            chunk(c, std::integral_constant<int, 0>{}, TERMS);
+            chunk(c + 1, std::integral_constant<int, 1>{}, TERMS);
+        }
+        if (c < nch) chunk(c, std::integral_constant<int, 0>{}, TERMS);
+    };
+    stream(std::integral_constant<int, 3>{});
+
+    // The activation rows' largest magnitudes (this slice's k), in LDS bytes
+    // that the stream is done with.
+    uint32_t *const xmax_s = reinterpret_cast<uint32_t *>(&xp[0][0][0][0][0]);
+    __syncthreads();
+    for (int i = tid; i < MT; i += 64 * NWV) xmax_s[i] = 0;
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < XI; ++j) {
+        const int it = wave * XI + j;
+        if (it < 2 * XT) atomicMax(&xmax_s[(it >> 1) * 16 + i16], FUSE ? xmx[j] : hi_max(xmx[j]) << 16);
+    }
+    __syncthreads();
+    // Outputs: lane l holds weight rows 4(l/16) + v of a tile, activation row
+    // l%16.  They are stored as they are; the rare ones that the sums do not
+    // settle (a tiny row, an exact zero, a value that is not finite) are redone.
+    float *const out = (P ? P + (int64_t)bz * M * N : Y) + row0;
+    bool rare = false;
+    uint32_t big[RM];  // bit 4j + v: the output is not finite
+#pragma unroll
+    for (int mf = 0; mf < RM; ++mf) {
+        const int ml = (wm * RM + mf) * 16 + i16;
+        big[mf] = 0;
+        if (m0 + ml >= M) continue;
+        rare |= xmax_s[ml] != 0 && xmax_s[ml] < kTinyHiBits << 16;
+        float *const o = out + (int64_t)(m0 + ml) * N;
+#pragma unroll
+        for (int j = 0; j < RN; ++j) {
+            const int n = (wn * RN + j) * 16 + g * 4;
+            if ((N & 3) == 0) {
+                if (n < nrows) *reinterpret_cast<f32x4_u *>(o + n) = acc[mf][j];
+            } else {
+#pragma unroll
+                for (int v = 0; v < 4; ++v)
+                    if (n + v < nrows) o[n + v] = acc[mf][j][v];
+            }
+#pragma unroll
+            for (int v = 0; v < 4; ++v) {
+                rare |= !P && n + v < nrows && acc[mf][j][v] == 0.0f;
+                if (n + v < nrows && !(fabsf(acc[mf][j][v]) < __builtin_inff())) big[mf] |= 1u << (4 * j + v);
+            }
+        }
+    }
+    if (__builtin_amdgcn_ballot_w64(rare) != 0) {
+#pragma nounroll
+        for (int f = 0; f < RM * RN * 4; ++f) {
+            const int mf = f / (RN * 4), n = (wn * RN + f / 4 % RN) * 16 + g * 4 + f % 4;
+            const int ml = (wm * RM + mf) * 16 + i16;
+            const bool live = m0 + ml < M && n < nrows;
+            const uint32_t xm = xmax_s[ml];
+            const float *const xr = X + (int64_t)min(m0 + ml, M - 1) * K;
+            const uint16_t *const wr = W + (int64_t)(row0 + min(n, nrows - 1)) * K;
+            float *const o = out + (int64_t)(m0 + ml) * N + n;
+            const bool tiny = live && xm != 0 && xm < kTinyHiBits << 16;
+            const bool zero = live && !tiny && !P && *o == 0.0f;
+            if (tiny) *o = reference_chain(wr + 64 * c0, xr + 64 * c0, 64 * nch);  // this slice's chain
+            if (zero && xm == 0) *o = 0.0f;  // an activation row of +-0
+            // Zeros of the other rows: +0 where the weight row holds only +-0, else the chain.
+            for (int gq = 0; gq < 4; ++gq) {
+                const bool ask = zero && xm != 0 && g == gq;
+                const uint64_t who = __builtin_amdgcn_ballot_w64(ask);
+                if (who == 0) continue;
+                const bool nz = wave_row_nonzero(readlane_ptr(wr, __builtin_ctzll(who)), K / 8, 0x7fff7fffu);
+                if (ask) *o = nz ? reference_chain(wr, xr, K) : 0.0f;
+            }
+        }
+    }
+    // Outputs that are not finite: a weight or an activation is inf or NaN
+    // (then every output of its row is inf or NaN in the reference), or a sum
+    // overflowed.  Their class may be wrong: mid and lo are 0 against an inf
+    // weight (NaN where the reference has inf), and the split of an inf leaves
+    // a NaN.  The hi term alone by split3's rule, nonzero for every nonzero x
+    // and carrying its inf or NaN, has the reference's classes, so the tile is
+    // streamed again with it and those outputs take its result where that is
+    // not finite either.  (Screening W in the loop and clearing such weights
+    // for mid and lo cost 12-18% of it, for weights that hold none.)
+    uint32_t *const any_s = xmax_s + MT;
+    bool mine = false;
+#pragma unroll
+    for (int mf = 0; mf < RM; ++mf) mine |= big[mf] != 0;
+    if (tid == 0) *any_s = 0;
+    __syncthreads();
+    if (mine) *any_s = 1;
+    __syncthreads();
+    const bool again = *any_s != 0;
+    __syncthreads();
+    if (!again) return;
+    stream(std::integral_constant<int, 1>{});
+#pragma unroll
+    for (int mf = 0; mf < RM; ++mf) {
+        float *const o = out + (int64_t)(m0 + (wm * RM + mf) * 16 + i16) * N;
+#pragma unroll
+        for (int j = 0; j < RN; ++j)
+#pragma unroll
+            for (int v = 0; v < 4; ++v)
+                if ((big[mf] >> (4 * j + v) & 1u) && !(fabsf(acc[mf][j][v]) < __builtin_inff()))
+                    o[(wn * RN + j) * 16 + g * 4 + v] = acc[mf][j][v];
+    }
+}
+
+// x [M,K] f32 -> its three bf16 terms as planes XS[q][M][K] (split3 of each
+// element).  count = M*K, a multiple of 8; 16-byte aligned.  Grid-stride.
+__global__ void __launch_bounds__(256)
+split_x_planes_kernel(const float *__restrict__ X, uint16_t *__restrict__ XS, int64_t count) {
+    for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < count / 8; i += (int64_t)gridDim.x * 256) {
+        const float4 a = reinterpret_cast<const float4 *>(X)[2 * i];
+        const float4 b = reinterpret_cast<const float4 *>(X)[2 * i + 1];
+        const float v[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
+        u32x4 hi, md, lo;
+        split8(v, hi, md, lo);
+        reinterpret_cast<u32x4 *>(XS)[i] = hi;
+        reinterpret_cast<u32x4 *>(XS + count)[i] = md;
+        reinterpret_cast<u32x4 *>(XS + 2 * count)[i] = lo;
+    }
+}
+
+// y[m][n] = P[0][m][n] + P[1][m][n] + ... in slice order, then the zero rule
+// of settle_zeros for one output: an exact zero is +0 when the activation row
+// or the weight row holds only +-0, else the reference chain's value.  Q
+// outputs per thread (4 where N is a multiple of 4, so that they share an
+// activation row): 16-byte loads, up to 8 slices' in flight.
+template <int Q>
+__global__ void __launch_bounds__(256)
+gemm_sum_slices_kernel(const float *__restrict__ P, int slices, float *__restrict__ Y, const uint16_t *__restrict__ W,
+                       const float *__restrict__ X, int M, int N, int K) {
+    typedef float vec __attribute__((ext_vector_type(Q), aligned(4)));
+    const int64_t count = (int64_t)M * N;
+    for (int64_t i = Q * ((int64_t)blockIdx.x * 256 + threadIdx.x); i < count; i += Q * (int64_t)gridDim.x * 256) {
+        vec s = *reinterpret_cast<const vec *>(P + i);
+#pragma unroll 8
+        for (int j = 1; j < slices; ++j) s += *reinterpret_cast<const vec *>(P + j * count + i);
+        bool zero = false;
+#pragma unroll
+        for (int e = 0; e < Q; ++e) zero |= s[e] == 0.0f;
+        if (zero) {
+            const int m = (int)(i / N), n = (int)(i - (int64_t)m * N);
+            const uint32_t *xr = reinterpret_cast<const uint32_t *>(X + (int64_t)m * K);
+            uint32_t xo = 0;
+            for (int k = 0; k < K; ++k) xo |= xr[k] & 0x7fffffffu;
+#pragma unroll
+            for (int e = 0; e < Q; ++e) {
+                if (s[e] != 0.0f) continue;
+                const uint16_t *w = W + (int64_t)(n + e) * K;
+                const uint32_t *wr = reinterpret_cast<const uint32_t *>(w);
+                uint32_t wo = 0;
+                for (int k = 0; xo && k < K / 2; ++k) wo |= wr[k] & 0x7fff7fffu;
+                s[e] = wo ? reference_chain(w, X + (int64_t)m * K, K) : 0.0f;
+            }
+        }
+        *reinterpret_cast<vec *>(Y + i) = s;
+    }
+}
+
+unsigned grid_for(int64_t blocks) { return (unsigned)std::max<int64_t>(1, std::min<int64_t>(blocks, 4096)); }
+
+}  // namespace
+
+hipError_t launch_sum_slices(const float *part, int slices, const RdProblem &p, hipStream_t s) {
+#define DMC_SUM(Q)                                                                                            \
+    hipLaunchKernelGGL(gemm_sum_slices_kernel<Q>, dim3(grid_for((p.m * p.n / Q + 255) / 256)), dim3(256), 0, s, part, \
+                       slices, p.y, p.w, p.x, (int)p.m, (int)p.n, (int)p.k)
+    if (p.n % 4 == 0) DMC_SUM(4);
+    else DMC_SUM(1);
+#undef DMC_SUM
+    return hipGetLastError();
+}
+
+hipError_t launch_gemm(const RdProblem &p, const RdPlan &pl, void *workspace, hipStream_t s) {
+    // The workspace holds x's planes (unless the kernel splits x itself) and
+    // the slice partials (when k is split): a fused single-slice plan needs
+    // none and may be given none.
+    const bool needs_ws = !pl.xfuse || pl.kslices > 1;
+    const int mt = pl.mt * pl.mtiles;
+    if ((needs_ws && !workspace) || pl.kslices < 1 || pl.kslices > 65535 ||
+        (int64_t)pl.kslices * pl.kchunks < p.k / 64 || pl.rpw != 32 * pl.waves || pl.grid_x * pl.rpw < p.n)
+        return hipErrorInvalidValue;
+    uint16_t *xs = pl.xfuse ? nullptr : static_cast<uint16_t *>(workspace);
+    const size_t planes = pl.xfuse ? 0 : ((size_t)3 * p.m * p.k * 2 + 255) / 256 * 256;
+    float *part = pl.kslices > 1 ? reinterpret_cast<float *>(static_cast<char *>(workspace) + planes) : nullptr;
+    const int64_t count = p.m * p.k;
+    if (!pl.xfuse)
+        hipLaunchKernelGGL(split_x_planes_kernel, dim3(grid_for((count / 8 + 255) / 256)), dim3(256), 0, s, p.x, xs,
+                           count);
+    const int64_t gy = (p.m + mt - 1) / mt;
+    const int64_t wgs = pl.grid_x * gy * (int64_t)pl.kslices;
+    if (wgs > INT32_MAX) return hipErrorInvalidValue;
+    // The XCD-grouped tile order where activation tiles share weight
+    // blocks (DMC_HIP_GEMM_XCD: 0 never, 2 always).
+    const int xenv = env_int("DMC_HIP_GEMM_XCD", 1);
+    const int xcd = xenv == 2 || (xenv == 1 && gy > 1) ? 1 : 0;
+#define DMC_GEMM(NW, MT, F)                                                                                   \
+    if (pl.waves == NW && mt == MT && pl.xfuse == F)                                                          \
+        hipLaunchKernelGGL((gemv_rd_mfma_gemm_kernel<NW, MT, F>), dim3((unsigned)wgs), dim3(64 * NW), 0, s, p.w, \
+                           p.x, xs, p.y, part, (int)p.n, (int)p.k, (int)p.m, pl.kchunks, (int)pl.grid_x, (int)gy, \
+                           xcd);                                                                              \
+    else
+    DMC_GEMM(8, 16, true) DMC_GEMM(8, 16, false) DMC_GEMM(8, 32, true) DMC_GEMM(8, 32, false)
+    DMC_GEMM(8, 64, true) DMC_GEMM(8, 64, false) DMC_GEMM(8, 128, true) DMC_GEMM(8, 128, false)
+    DMC_GEMM(4, 32, true) DMC_GEMM(4, 32, false) DMC_GEMM(4, 64, true) DMC_GEMM(4, 64, false)
+    return hipErrorInvalidValue;
+#undef DMC_GEMM
+    if (pl.kslices > 1) return launch_sum_slices(part, pl.kslices, p, s);
+    return hipGetLastError();
+}
+
+}  // namespace dmc

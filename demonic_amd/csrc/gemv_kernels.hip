@@ -23,6 +23,7 @@
 //    (compiled with -fno-gpu-flush-denormals-to-zero, no fast-math, no fp
 //    contraction), packed-fp32 disabled.  Fixed reduction order: bit-identical
 //    results run to run.
+#include "gemv_device.h"
 #include "gemv_launch.h"
 
 #include <algorithm>
@@ -166,175 +167,6 @@ __device__ __forceinline__ void wave_sums(const float (&a)[V], Store store) {
             }
         }
     }
-}
-
-// 128-bit weight loads through a buffer resource, marked nontemporal: weights
-// are streamed once per launch, so they should not displace x or y in the
-// caches.  (Measured on MI355X: ~8% more bandwidth than plain global loads.)
-typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
-
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t weight_rsrc(const void *base, uint32_t bytes) {
-    return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(base), (short)0, (int)bytes, 0x00020000);
-}
-
-constexpr int kLoadNT = 2;  // cache-policy bits of a buffer load: nt
-
-__device__ __forceinline__ u32x4 load_w16(__amdgpu_buffer_rsrc_t r, uint32_t byte_off) {
-    return __builtin_amdgcn_raw_buffer_load_b128(r, byte_off, 0, kLoadNT);
-}
-
-// The same with a wave-uniform part of the offset in the instruction's scalar
-// offset.  Measured on gfx950: the range check covers the sum of both offsets
-// (per dword), like a single offset.  Keeping a loop's row offset scalar and
-// the lane's offset loop-invariant leaves no per-load vector address
-// arithmetic, whose temporaries the register allocator otherwise places in
-// registers just freed by a load -- and the compiler then waits for that
-// load's whole batch before the next one may issue.
-__device__ __forceinline__ u32x4 load_w16(__amdgpu_buffer_rsrc_t r, uint32_t lane_off, uint32_t uniform_off) {
-    return __builtin_amdgcn_raw_buffer_load_b128(r, lane_off, uniform_off, kLoadNT);
-}
-
-__device__ __forceinline__ float widen_lo(uint32_t w) { return __uint_as_float(w << 16); }
-__device__ __forceinline__ float widen_hi(uint32_t w) { return __uint_as_float(w & 0xffff0000u); }
-
-// ---- zero outputs of the FMA kernels ------------------------------------------
-//
-// The FMA kernels split k, so an output is a sum of partial chains.  When that
-// sum comes out exactly 0 it can differ from the reference chain (fmaf over
-// ascending k from +0, jit.rs:29655-29670): a run of underflowing products of
-// both signs leaves the chain at the zero of the last one's sign, where a sum
-// of reordered partials is -0 only if every partial is; and reordered partials
-// can cancel exactly where the chain keeps a subnormal residue.  Neither can
-// happen when every product is an exact zero (some factor +-0): the chain then
-// never leaves +0, and neither does the split sum (lanes with elements start
-// at +0, idle ones add -0).  So a zero output is settled by the reference's
-// rule: +0 when no product has two nonzero factors -- an all-zero activation
-// row, an all-zero weight row, or factors that never meet -- and otherwise
-// the chain itself (underflow or exact cancellation, which takes crafted
-// data).  The common path costs one compare and one ballot per output.
-
-// The reference chain for one output: K products x[k] * w[k * wstep], any
-// alignment (2- and 4-byte loads; the rare path only).
-__device__ float chain_strided(const uint16_t *__restrict__ w, int64_t wstep, const float *__restrict__ x, int K) {
-    float acc = 0.0f;
-    int k = 0;
-    for (; k + 4 <= K; k += 4) {
-        const uint16_t *p = w + (int64_t)k * wstep;
-        const uint32_t b0 = p[0], b1 = p[wstep], b2 = p[2 * wstep], b3 = p[3 * wstep];
-        const float x0 = x[k], x1 = x[k + 1], x2 = x[k + 2], x3 = x[k + 3];
-        acc = fmaf(x0, __uint_as_float(b0 << 16), acc);
-        acc = fmaf(x1, __uint_as_float(b1 << 16), acc);
-        acc = fmaf(x2, __uint_as_float(b2 << 16), acc);
-        acc = fmaf(x3, __uint_as_float(b3 << 16), acc);
-    }
-    for (; k < K; ++k) acc = fmaf(x[k], __uint_as_float((uint32_t)w[(int64_t)k * wstep] << 16), acc);
-    return acc;
-}
-
-template <class T>
-__device__ __forceinline__ const T *readlane_ptr(const T *p, int j) {
-    const uint64_t v = reinterpret_cast<uint64_t>(p);
-    const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)v, j);
-    const uint32_t hi = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(v >> 32), j);
-    return reinterpret_cast<const T *>(((uint64_t)hi << 32) | lo);
-}
-
-// Wave-uniform: does some k have x[k] and (w == nullptr, or w[k * wstep])
-// nonzero?  Contiguous rows (wstep <= 1, K <= 2^28): 16-byte buffer loads at
-// the rows' own 4- and 2-byte alignments (exact on gfx950), 8 elements per
-// lane per load, 4096 per round -- one round for K <= 4096.  The weight range
-// ends exactly after element K-1: a load's dword that runs past it comes back
-// as zeros (element K-1 itself when it shares such a dword), so element K-1
-// is also read alone, 2 bytes, and nothing past the row is ever read.
-// Strided columns: one element per lane per load, 64 * 32 per round.  All
-// loads of a round are in flight together; the scan stops at the first round
-// that finds a product.
-__device__ bool wave_any_product(const float *x, const uint16_t *w, int64_t wstep, int K) {
-    const int lane = threadIdx.x & 63;
-    if (K <= 0) return false;
-    if (wstep <= 1 && K <= (1 << 28)) {
-        constexpr int U = 8;
-        const uintptr_t wb = reinterpret_cast<uintptr_t>(w);
-        const __amdgpu_buffer_rsrc_t xr = weight_rsrc(x, (uint32_t)K * 4u);
-        const uintptr_t w0 = wb & ~(uintptr_t)3;
-        const uint32_t wd = (uint32_t)(wb - w0);  // 0 or 2
-        const __amdgpu_buffer_rsrc_t wr =
-            weight_rsrc(reinterpret_cast<const void *>(w ? w0 : reinterpret_cast<uintptr_t>(x)),
-                        w ? wd + 2u * (uint32_t)K : 0u);
-        const uint32_t wl = w ? (uint32_t)__builtin_amdgcn_raw_buffer_load_b16(wr, wd + 2u * (K - 1), 0, 0) : 1u;
-        const uint32_t xl = __float_as_uint(x[K - 1]) & 0x7fffffffu;
-        bool first = true;
-        for (int k0 = 0; k0 < K; k0 += 512 * U) {
-            u32x4 xa[U], xc[U], wv[U];
-#pragma unroll
-            for (int u = 0; u < U; ++u) {
-                const uint32_t e = (uint32_t)(k0 + (u * 64 + lane) * 8);
-                xa[u] = __builtin_amdgcn_raw_buffer_load_b128(xr, e * 4u, 0, 0);
-                xc[u] = __builtin_amdgcn_raw_buffer_load_b128(xr, e * 4u + 16u, 0, 0);
-                wv[u] = w ? __builtin_amdgcn_raw_buffer_load_b128(wr, wd + e * 2u, 0, 0) : u32x4{~0u, ~0u, ~0u, ~0u};
-            }
-            uint32_t hit = first && (wl & 0x7fffu) != 0 && xl != 0 ? 1u : 0u;
-            first = false;
-#pragma unroll
-            for (int u = 0; u < U; ++u) {
-                const int e = k0 + (u * 64 + lane) * 8;
-#pragma unroll
-                for (int i = 0; i < 8; ++i) {
-                    const uint32_t xv = (i < 4 ? xa[u][i] : xc[u][i - 4]) & 0x7fffffffu;
-                    const uint32_t wv16 = (wv[u][i >> 1] >> (16 * (i & 1))) & 0x7fffu;
-                    hit |= (e + i < K && xv != 0 && wv16 != 0) ? 1u : 0u;
-                }
-            }
-            if (__builtin_amdgcn_ballot_w64(hit != 0) != 0) return true;
-        }
-        return false;
-    }
-    constexpr int U = 32;
-    for (int k0 = 0; k0 < K; k0 += 64 * U) {
-        uint32_t xb[U], wb[U];
-#pragma unroll
-        for (int u = 0; u < U; ++u) {
-            const int k = min(k0 + u * 64 + lane, K - 1);
-            xb[u] = __float_as_uint(x[k]) & 0x7fffffffu;
-            wb[u] = w ? (uint32_t)w[(int64_t)k * wstep] & 0x7fffu : 1u;
-        }
-        uint32_t hit = 0;
-#pragma unroll
-        for (int u = 0; u < U; ++u) hit |= (k0 + u * 64 + lane < K && xb[u] != 0 && wb[u] != 0) ? 1u : 0u;
-        if (__builtin_amdgcn_ballot_w64(hit != 0) != 0) return true;
-    }
-    return false;
-}
-
-// The zero rule for the outputs this wave holds, one per lane: `zero` marks a
-// lane whose output s is exactly 0 and is stored; x is its activation row,
-// w its first weight, wstep the elements between consecutive k.  All 64 lanes
-// call it (wave-uniform control flow): rows are scanned by the whole wave,
-// one output at a time, and the chains (if any) run one per lane.
-__device__ float settle_zero(float s, bool zero, const float *x, const uint16_t *w, int64_t wstep, int K) {
-    uint64_t pend = __builtin_amdgcn_ballot_w64(zero);
-    if (pend == 0) return s;
-    const int lane = threadIdx.x & 63;
-    // activation rows that hold only +-0, each distinct row scanned once (a
-    // lone zero output skips this: its product scan covers its row)
-    bool xnz = true;
-    if (pend & (pend - 1)) while (pend) {
-        const int j = __builtin_ctzll(pend);
-        const float *xj = readlane_ptr(x, j);
-        const bool nz = wave_any_product(xj, nullptr, 0, K);
-        const bool same = zero && x == xj;
-        if (same) xnz = nz;
-        pend &= ~__builtin_amdgcn_ballot_w64(same);
-    }
-    // outputs whose products all have a zero factor
-    bool chain = false;
-    for (uint64_t todo = __builtin_amdgcn_ballot_w64(zero && xnz); todo; todo &= todo - 1) {
-        const int j = __builtin_ctzll(todo);
-        const bool hit = wave_any_product(readlane_ptr(x, j), readlane_ptr(w, j), wstep, K);
-        if (lane == j) chain = hit;
-    }
-    if (zero) s = chain ? chain_strided(w, wstep, x, K) : 0.0f;
-    return s;
 }
 
 // The column-stream kernels and the row-dot kernels that keep x in registers
@@ -1191,230 +1023,6 @@ gemv_rd_unaligned_kernel(const uint16_t *__restrict__ W, const float *__restrict
     }
 }
 
-// ---- RD skinny M on MFMA: W [N,K] x X [M,K], K % 64 == 0 ---------------------------
-//
-// From M = 2 the FMA path loses to the matrix cores (M fmas per weight element,
-// MT activation rows of registers; on the LM-head shape M = 2 takes 174-183 us
-// there against 161-166 here, M = 3 212-240 against 166-173), so the
-// products go to v_mfma_f32_16x16x32_bf16: A = a 16-row weight tile, B = x^T
-// for 16 activation rows.  x is f32, so it enters as three bf16 terms,
-// x == hi + mid + lo, each taken by truncation: every residual is exact in
-// f32 and keeps at most 8 significant bits, so the split is exact for
-// |x| >= 2^-110 (below that the error is < 2^-133 absolute).  Measured on
-// gfx950 this MFMA multiplies exactly, sums a block's 32 products and the
-// accumulator with one rounding, keeps bf16/f32 subnormals, and follows IEEE
-// for inf and NaN -- so each output is the exact dot product up to 3
-// roundings per 32 k, more accurate than the reference's sequential fma chain.
-//
-// Special values keep the reference's classes (fmaf(x, w, acc) semantics):
-//   x = +-inf or NaN: hi carries it (a NaN is kept quiet), mid = lo = 0;
-//   x != 0 tiny: hi is never 0, so inf * x stays inf;
-//   w = +-inf or NaN: multiplies hi only -- the mid and lo MFMAs see 0 there,
-//     because inf * (mid == 0) would be NaN where the reference has inf.
-//
-// Zeros: the MFMA rounds a nonzero sum smaller than half the least f32
-// subnormal to +0 whatever its sign, where the reference's fmaf gives the
-// signed zero (every product underflowing negative ends at -0).  So an output
-// that comes out exactly zero is settled by the reference's own rule: +0 when
-// its activation row or its weight row holds only zeros (every product is an
-// exact zero and the chain never leaves +0), otherwise the chain itself,
-// fmaf over ascending k from +0 (rare: underflow or exact cancellation).
-
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-typedef float f32x4 __attribute__((ext_vector_type(4)));
-
-__device__ __forceinline__ f32x4 mfma_bf16(const u32x4 &a, const u32x4 &b, const f32x4 &c) {
-    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b),
-                                                   c, 0, 0, 0);
-}
-
-// Bits 0xffff in each 16-bit half of d whose bf16 exponent is all ones.
-__device__ __forceinline__ uint32_t inf_nan_mask(uint32_t d) {
-    const uint32_t t = ((d & 0x7f807f80u) + 0x00800080u) & 0x80008000u;
-    return (t >> 15) * 0xffffu;
-}
-
-typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
-
-// Running per-half maximum of bf16 magnitudes: a half holding an inf or NaN
-// reaches 0x7f80.  Two instructions per dword (and, packed max); the exact
-// per-element mask is computed only when a wave's screen fires.
-__device__ __forceinline__ uint32_t max_mag(uint32_t acc, uint32_t d) {
-    return __builtin_bit_cast(uint32_t, __builtin_elementwise_max(__builtin_bit_cast(u16x2, acc),
-                                                                  __builtin_bit_cast(u16x2, d & 0x7fff7fffu)));
-}
-
-__device__ __forceinline__ bool wave_has_inf_nan(uint32_t mx) {
-    const bool mine = (mx & 0xffffu) >= 0x7f80u || (mx >> 16) >= 0x7f80u;
-    return __builtin_amdgcn_ballot_w64(mine) != 0;
-}
-
-// The three bf16 terms of one f32.
-__device__ __forceinline__ void split3(float v, uint32_t &h, uint32_t &m, uint32_t &l) {
-    // Selects, not branches: every lane of the rows16 layout splits 16 values per line.
-    const uint32_t u = __float_as_uint(v);
-    const bool fin = (u & 0x7f800000u) != 0x7f800000u;
-    const uint32_t t = u >> 16;
-    const uint32_t nan_q = !fin && (u & 0x007fffffu) ? 0x0040u : 0u;                 // NaN: stay NaN after truncation
-    const uint32_t keep = fin && (t & 0x7fffu) == 0 && (u & 0x7fffffffu) != 0 ? 1u : 0u;  // |x| < 2^-133: hi nonzero
-    h = t | nan_q | keep;
-    const float r1 = fin ? v - __uint_as_float(h << 16) : 0.0f;
-    m = __float_as_uint(r1) >> 16;
-    const float r2 = r1 - __uint_as_float(m << 16);
-    l = __float_as_uint(r2) >> 16;
-}
-
-// Four values at once, two per dword of each plane.  Where all four are
-// finite with |x| = 0 or |x| >= 2^-133 (bf16's least subnormal), split3's
-// rule is truncation alone (no NaN quieting, no kept tiny bit, no inf
-// residual), taken here without its selects: 4 operations a value and the
-// packing instead of about 15.  The test is two reductions over the
-// magnitudes (|x| - 1 wraps 0 to the top); a lane that fails it (an inf, a
-// NaN or a tiny value among its four) takes split3.
-__device__ __forceinline__ void split4(const float *v, uint32_t *hi, uint32_t *mid, uint32_t *lo) {
-    uint32_t amax = 0, amin1 = 0xffffffffu;
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-        const uint32_t a = __float_as_uint(v[e]) & 0x7fffffffu;
-        amax = max(amax, a);
-        amin1 = min(amin1, a - 1u);
-    }
-    if (amax < 0x7f800000u && amin1 >= 0x0000ffffu) {
-#pragma unroll
-        for (int q = 0; q < 2; ++q) {
-            const uint32_t u0 = __float_as_uint(v[2 * q]), u1 = __float_as_uint(v[2 * q + 1]);
-            const float r10 = v[2 * q] - __uint_as_float(u0 & 0xffff0000u);
-            const float r11 = v[2 * q + 1] - __uint_as_float(u1 & 0xffff0000u);
-            const uint32_t b10 = __float_as_uint(r10), b11 = __float_as_uint(r11);
-            const uint32_t b20 = __float_as_uint(r10 - __uint_as_float(b10 & 0xffff0000u));
-            const uint32_t b21 = __float_as_uint(r11 - __uint_as_float(b11 & 0xffff0000u));
-            hi[q] = (u0 >> 16) | (u1 & 0xffff0000u);
-            mid[q] = (b10 >> 16) | (b11 & 0xffff0000u);
-            lo[q] = (b20 >> 16) | (b21 & 0xffff0000u);
-        }
-        return;
-    }
-#pragma unroll
-    for (int q = 0; q < 2; ++q) {
-        uint32_t h0, m0, l0, h1, m1, l1;
-        split3(v[2 * q], h0, m0, l0);
-        split3(v[2 * q + 1], h1, m1, l1);
-        hi[q] = h0 | (h1 << 16);
-        mid[q] = m0 | (m1 << 16);
-        lo[q] = l0 | (l1 << 16);
-    }
-}
-
-// Eight values: two halves of four.
-__device__ __forceinline__ void split8(const float *v, u32x4 &hi, u32x4 &mid, u32x4 &lo) {
-#pragma unroll
-    for (int h = 0; h < 2; ++h) {
-        uint32_t hq[2], mq[2], lq[2];
-        split4(v + 4 * h, hq, mq, lq);
-        hi[2 * h] = hq[0], hi[2 * h + 1] = hq[1];
-        mid[2 * h] = mq[0], mid[2 * h + 1] = mq[1];
-        lo[2 * h] = lq[0], lo[2 * h + 1] = lq[1];
-    }
-}
-
-// The reference chain for one output: fmaf over ascending k from +0 (K a
-// multiple of 8, rows 16-byte aligned).
-__device__ float reference_chain(const uint16_t *__restrict__ w, const float *__restrict__ x, int K) {
-    float acc = 0.0f;
-    for (int k = 0; k < K; k += 8) {
-        const u32x4 wv = *reinterpret_cast<const u32x4 *>(w + k);
-        const float4 xa = *reinterpret_cast<const float4 *>(x + k);
-        const float4 xb = *reinterpret_cast<const float4 *>(x + k + 4);
-        const float xv[8] = {xa.x, xa.y, xa.z, xa.w, xb.x, xb.y, xb.z, xb.w};
-#pragma unroll
-        for (int e = 0; e < 8; ++e) {
-            const uint32_t bits = e & 1 ? wv[e >> 1] & 0xffff0000u : wv[e >> 1] << 16;
-            acc = fmaf(xv[e], __uint_as_float(bits), acc);
-        }
-    }
-    return acc;
-}
-
-// Tiny activation rows.  split3 is exact for |x| >= 2^-110: below that the
-// third term falls under bf16's least subnormal (2^-133) and x loses its low
-// bits.  That matters only when a whole activation row is that small -- then
-// every product loses up to 2^-133 / |x| of itself (a row of |x| ~ 1e-37
-// would be off by ~2^-10) -- while in a row with larger entries the lost
-// bits are below 2^-33 of the largest one.  So each MFMA kernel keeps, per
-// lane, the largest bf16 magnitude of the hi terms it split (hi keeps the
-// order of |x| against 2^-100, and is nonzero for every nonzero x), takes
-// the maximum per activation row over its workgroup's k range, and gives a
-// row whose maximum is nonzero but below 2^-100 (bf16 0x0d80) the reference
-// chain over that k range instead of its MFMA sums: bit for bit the
-// reference's value when k is not split, else the slice's part of it.  Rare
-// path: no real activation row is this small.
-constexpr uint32_t kTinyHiBits = 0x0d80u;
-
-__device__ __forceinline__ uint32_t hi_max(uint32_t mx) { return max(mx & 0xffffu, mx >> 16); }
-__device__ __forceinline__ bool tiny_row(uint32_t mx) { return mx != 0 && mx < kTinyHiBits; }
-
-// Wave-uniform: does the row hold an element other than +-0?  (bytes: 16 * n16)
-__device__ bool wave_row_nonzero(const void *row, int n16, uint32_t mask) {
-    const u32x4 *p = reinterpret_cast<const u32x4 *>(row);
-    uint32_t acc = 0;
-    for (int c = threadIdx.x & 63; c < n16; c += 64) {
-        const u32x4 v = p[c];
-        acc |= (v[0] | v[1] | v[2] | v[3]) & mask;
-    }
-    return __builtin_amdgcn_ballot_w64(acc != 0) != 0;
-}
-
-// One wave's outputs after the zero rule above.  Lane l holds s[t][r] for
-// weight row base[t] + 4(l/16) + r of W and activation row m of X; `live`
-// marks the ones it stores.  All 64 lanes call this; the rows are walked
-// wave-uniformly.  Rare path: entered only when some output is exactly zero.
-template <int T>
-__device__ void settle_zeros(f32x4 (&s)[T], const bool (&live)[T][4], const int (&base)[T], const uint16_t *W,
-                             const float *X, int K, int m) {
-    const int g = (threadIdx.x & 63) >> 4;
-    bool zero[T][4];
-    bool any = false;
-#pragma unroll
-    for (int t = 0; t < T; ++t)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            zero[t][r] = live[t][r] && s[t][r] == 0.0f;
-            any |= zero[t][r];
-        }
-    if (__builtin_amdgcn_ballot_w64(any) == 0) return;
-    // Is this lane's activation row nonzero?  Lanes j = 0..15 hold every row
-    // the wave has.
-    bool xnz = false;
-    for (int j = 0; j < 16; ++j) {
-        const int mj = __builtin_amdgcn_readlane(m, j);
-        if (__builtin_amdgcn_ballot_w64(any && m == mj) != 0) {
-            const bool nz = wave_row_nonzero(X + (int64_t)mj * K, K / 4, 0x7fffffffu);
-            if (m == mj) xnz = nz;
-        }
-    }
-    // Zero outputs become +0, or the chain's value where both rows are nonzero.
-    bool chain[T][4];
-#pragma unroll
-    for (int t = 0; t < T; ++t)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            chain[t][r] = false;
-            if (zero[t][r]) s[t][r] = 0.0f;
-            for (int gq = 0; gq < 4; ++gq) {
-                const bool ask = zero[t][r] && xnz && g == gq;
-                if (__builtin_amdgcn_ballot_w64(ask) == 0) continue;
-                const int row = base[t] + 4 * gq + r;
-                const bool nz = wave_row_nonzero(W + (int64_t)row * K, K / 8, 0x7fff7fffu);
-                if (ask) chain[t][r] = nz;
-            }
-        }
-#pragma unroll
-    for (int t = 0; t < T; ++t)
-#pragma unroll
-        for (int r = 0; r < 4; ++r)
-            if (chain[t][r]) s[t][r] = reference_chain(W + (int64_t)(base[t] + 4 * g + r) * K, X + (int64_t)m * K, K);
-}
-
 // Fourth MFMA layout ("wide"): what bounds the MFMA kernels on MI355X is the
 // bytes every vector load moves into the CU -- activation re-reads cost as
 // much as weight bytes, even from L2 -- and the MFMA operand pattern (16 rows
@@ -1430,29 +1038,6 @@ __device__ void settle_zeros(f32x4 (&s)[T], const bool (&live)[T][4], const int 
 // Loads run two chunks ahead in registers.
 constexpr int kWideRows = 256;
 constexpr int kWidePitch = 128;
-
-// Weight and x tiles in LDS hold rows of 128 bytes, 8 pieces of 16, back to
-// back, with piece p of row r stored at position p ^ ((r / 2) mod 8).  A
-// tile is written 8 rows x 128 bytes per instruction (each pair of rows then
-// covers the 64 banks once) and read 16 rows x one piece (the rows' pieces
-// land on 16 different groups of 4 banks).  The earlier 144-byte pitch kept
-// the reads apart but let each pair of rows written together meet on 4 banks
-// (11-24% of the MFMA kernels' LDS cycles lost to conflicts).
-__device__ __forceinline__ int swz(int r, int p) { return r * 128 + ((p ^ ((r >> 1) & 7)) << 4); }
-
-// Chunk order of the MFMA layouts.  A workgroup streams its weight rows
-// one 128-byte column of lines (64 k) at a time; with every workgroup at
-// the same k the whole device reads addresses that differ only above the
-// row pitch, which for power-of-two rows (K = 4096: 8 KiB) meets a few HBM
-// channels at a time.  Workgroup b therefore starts at chunk 5b mod n and
-// wraps: on C4's W [128256, 4096] the read pattern alone streams in 150 us
-// rotated against 178 in step (a plain read of the same bytes: 145).  The
-// MFMA sums are taken in that order; the zero rule and the tiny-row chains
-// recompute in k order, so only rounding inside the bound changes.
-__device__ __forceinline__ int chunk_rotation(uint32_t b, int n) {
-    return n > 0 ? (int)((b * 5u) % (uint32_t)n) : 0;
-}
-__device__ __forceinline__ int rotate_chunk(int c, int s0, int n) { return c + s0 >= n ? c + s0 - n : c + s0; }
 
 __global__ void __launch_bounds__(512)
 gemv_rd_mfma_wide_kernel(const uint16_t *__restrict__ W, const float *__restrict__ X, float *__restrict__ Y, int N,
@@ -1592,339 +1177,6 @@ gemv_rd_mfma_wide_kernel(const uint16_t *__restrict__ W, const float *__restrict
 #pragma unroll
         for (int r = 0; r < 4; ++r)
             if (live[t][r]) Y[(int64_t)(m0 + i16) * N + row0 + base[t] + g * 4 + r] = acc[t][r];
-}
-
-// Sixth MFMA layout ("gemm"), for 9 activation rows and up (prefill-sized M
-// among them): the wide layout with MB tiles of 16 activation rows per
-// workgroup instead of one.  Every
-// weight tile a wave stages in LDS meets all 16 * MB activation rows, so W
-// streams from HBM once per 16 * MB rows (the 16-row layouts stream it once
-// per 16).  x arrives already split: split_x_planes_kernel writes its three
-// bf16 terms once per call as planes [3][M][K], and each chunk's operands are
-// copied into LDS (no per-workgroup split).  FUSE (16-row activation tiles):
-// each workgroup loads its chunks of x as f32 and splits them itself on the
-// way into LDS instead, which saves the split launch; at 16 activation rows
-// the repeated split is a few dozen values per thread.  When 256-row by 16*MB-row tiles
-// would leave the device short of workgroups, k is split over `slices`
-// workgroups, each covering kc chunks of 64, whose partial sums go to
-// P[slice][m][n] for gemm_sum_slices_kernel.  Numerics, special values and
-// the zero rule are the wide layout's, tile by tile; with slices the zero
-// rule runs after the sum.
-template <int MB, bool FUSE, int NWV>
-__global__ void __launch_bounds__(64 * NWV)
-gemv_rd_mfma_gemm_kernel(const uint16_t *__restrict__ W, const float *__restrict__ X, const uint16_t *__restrict__ XS,
-                         float *__restrict__ Y, float *__restrict__ P, int N, int K, int M, int kc, int gx, int gy,
-                         int xcd) {
-    static_assert(MB >= 1 && MB <= 4, "16 to 64 activation rows per workgroup");
-    static_assert(NWV == 4 || NWV == 8, "32 weight rows per wave");
-    constexpr int kRows = 32 * NWV;                  // weight rows per workgroup
-    constexpr int kXItems = 128 * MB;                // x staging items (tile, k-block, operand lane)
-    constexpr int kXPer = (kXItems + 64 * NWV - 1) / (64 * NWV);  // items per thread
-    constexpr int D = 2;  // register sets of the chunk ring (3 and 4 measured no faster)
-    const int tid = threadIdx.x;
-    const int lane = tid & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int i16 = lane & 15;
-    const int g = lane >> 4;
-    // The tile from the linear workgroup id (a 1-D grid of gx * gy * slices).
-    // With `xcd` set, workgroup L, which runs on XCD L % 8 (the dispatcher
-    // deals workgroups to the 8 XCDs in turn), takes the L / 8-th tile of
-    // that XCD's contiguous share, activation tiles fastest, so the
-    // workgroups an XCD runs together share weight blocks through its L2
-    // (C2 shapes at several activation tiles: 2-3% faster than weight blocks
-    // fastest); otherwise tiles go in launch order, consecutive weight
-    // blocks to different XCDs.
-    uint32_t lin = blockIdx.x;
-    if (xcd) {
-        const uint32_t x = lin & 7u, q = gridDim.x >> 3, r = gridDim.x & 7u;
-        lin = x * q + min(x, r) + (lin >> 3);
-    }
-    const int by = (int)(lin % (uint32_t)gy);
-    const int bx = (int)(lin / (uint32_t)gy % (uint32_t)gx);
-    const int bz = (int)(lin / (uint32_t)gy / (uint32_t)gx);
-    const int row0 = bx * kRows;
-    const int nrows = min(kRows, N - row0);
-    const int m0 = by * 16 * MB;
-    const int c0 = bz * kc;                              // this slice's chunks: [c0, c1)
-    const int c1 = min(K / 64, c0 + kc);
-    const int nchunks = max(0, c1 - c0);
-
-    __shared__ __attribute__((aligned(16))) uint8_t wt[kRows * kWidePitch];  // 32 KiB at 8 waves
-    __shared__ u32x4 xpl[2][MB][2][3][64];                                   // MB x 12 KiB
-    __shared__ uint32_t xmax_s[16 * MB];  // per activation row: the largest hi-term magnitude (tiny rows)
-    uint8_t *const wtw = wt + wave * 32 * kWidePitch;                            // this wave's 32 rows
-    if (tid < 16 * MB) xmax_s[tid] = 0;
-
-    const __amdgpu_buffer_rsrc_t rs = weight_rsrc(W + (int64_t)row0 * K, (uint32_t)((int64_t)nrows * K * 2));
-    // Staging: load j (0..3) covers the wave's rows 8j + lane/8, bytes 16*(lane%8) of the chunk.
-    const int scol = (lane & 7) * 16;
-    const int slr = lane >> 3;
-    uint32_t soff[4];
-#pragma unroll
-    for (int j = 0; j < 4; ++j)
-        soff[j] = (uint32_t)min(wave * 32 + slr + 8 * j, nrows - 1) * (uint32_t)K * 2u + scol;
-    // x items it = tid + 64*NWV*j (j < kXPer), those below 128*MB: (tile xt =
-    // it/128, k-block b = it/64 % 2, operand lane = lane): the lane's 8
-    // elements of each of the three planes (FUSE: its 8 f32 values, split in
-    // `store`), by unconditional buffer loads (rows past M load from past the
-    // range: zeros).
-    bool xthread[kXPer];
-    int xt[kXPer], xb[kXPer];
-    uint32_t xoff[kXPer];
-    const uint32_t plane_bytes = (uint32_t)M * (uint32_t)K * 2u;
-    const __amdgpu_buffer_rsrc_t xrs = FUSE ? weight_rsrc(X, 2u * plane_bytes) : weight_rsrc(XS, 3u * plane_bytes);
-#pragma unroll
-    for (int j = 0; j < kXPer; ++j) {
-        const int it = tid + 64 * NWV * j;
-        xthread[j] = it < kXItems;
-        xt[j] = xthread[j] ? it >> 7 : 0;
-        xb[j] = (it >> 6) & 1;
-        const int xm = m0 + xt[j] * 16 + (lane & 15);
-        const uint32_t xelem = (uint32_t)xm * (uint32_t)K + xb[j] * 32 + (lane >> 4) * 8;
-        xoff[j] = xthread[j] && xm < M ? xelem * (FUSE ? 4u : 2u) : kOutOfRange;
-    }
-
-    constexpr int XQ = FUSE ? 2 : 3;  // x registers per item and chunk: f32 halves, or the three planes
-    struct Regs {
-        u32x4 w[4];
-        u32x4 x[kXPer][XQ];
-    };
-    const int s0 = chunk_rotation(bx, nchunks);
-    auto load = [&](int c, Regs &r) {
-        const uint32_t cb = (uint32_t)(c0 + rotate_chunk(c, s0, nchunks)) * 128u;
-#pragma unroll
-        for (int j = 0; j < 4; ++j) r.w[j] = load_w16(rs, soff[j] + cb);
-#pragma unroll
-        for (int j = 0; j < kXPer; ++j) {
-            if constexpr (FUSE) {
-#pragma unroll
-                for (int q = 0; q < 2; ++q)
-                    r.x[j][q] = __builtin_amdgcn_raw_buffer_load_b128(xrs, xoff[j], 2u * cb + 16u * q, 0);
-            } else {
-#pragma unroll
-                for (int q = 0; q < 3; ++q)
-                    r.x[j][q] = __builtin_amdgcn_raw_buffer_load_b128(xrs, xoff[j], q * plane_bytes + cb, 0);
-            }
-        }
-    };
-    uint32_t xmx[kXPer];
-#pragma unroll
-    for (int j = 0; j < kXPer; ++j) xmx[j] = 0;
-    auto store = [&](const Regs &r, int xbuf) {
-#pragma unroll
-        for (int j = 0; j < 4; ++j) *reinterpret_cast<u32x4 *>(wtw + swz(slr + 8 * j, lane & 7)) = r.w[j];
-#pragma unroll
-        for (int j = 0; j < kXPer; ++j) {
-            if (!xthread[j]) continue;
-            if constexpr (FUSE) {
-                const float v[8] = {__uint_as_float(r.x[j][0][0]), __uint_as_float(r.x[j][0][1]),
-                                    __uint_as_float(r.x[j][0][2]), __uint_as_float(r.x[j][0][3]),
-                                    __uint_as_float(r.x[j][1][0]), __uint_as_float(r.x[j][1][1]),
-                                    __uint_as_float(r.x[j][1][2]), __uint_as_float(r.x[j][1][3])};
-                u32x4 hi, md, lo;
-                split8(v, hi, md, lo);
-#pragma unroll
-                for (int e = 0; e < 4; ++e) xmx[j] = max_mag(xmx[j], hi[e]);
-                xpl[xbuf][xt[j]][xb[j]][0][lane] = hi;
-                xpl[xbuf][xt[j]][xb[j]][1][lane] = md;
-                xpl[xbuf][xt[j]][xb[j]][2][lane] = lo;
-            } else {
-#pragma unroll
-                for (int e = 0; e < 4; ++e) xmx[j] = max_mag(xmx[j], r.x[j][0][e]);
-#pragma unroll
-                for (int q = 0; q < 3; ++q) xpl[xbuf][xt[j]][xb[j]][q][lane] = r.x[j][q];
-            }
-        }
-    };
-
-    f32x4 acc[MB][2];
-#pragma unroll
-    for (int mt = 0; mt < MB; ++mt) acc[mt][0] = acc[mt][1] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-    // One k-block of 32: the hi term with the raw weights, md and lo with
-    // inf/NaN lanes cleared when the wave's block holds any.
-    auto block = [&](const u32x4 (&a)[2], const u32x4 (&xo)[MB][3]) {
-        u32x4 a2[2];
-        uint32_t mx = 0;
-#pragma unroll
-        for (int t = 0; t < 2; ++t)
-#pragma unroll
-            for (int v = 0; v < 4; ++v) mx = max_mag(mx, a[t][v]);
-        const bool any_special = wave_has_inf_nan(mx);
-#pragma unroll
-        for (int t = 0; t < 2; ++t) {
-            a2[t] = a[t];
-            if (any_special) {
-#pragma unroll
-                for (int v = 0; v < 4; ++v) a2[t][v] &= ~inf_nan_mask(a2[t][v]);
-            }
-        }
-#pragma unroll
-        for (int mt = 0; mt < MB; ++mt)
-#pragma unroll
-            for (int t = 0; t < 2; ++t) {
-                acc[mt][t] = mfma_bf16(a[t], xo[mt][0], acc[mt][t]);
-                acc[mt][t] = mfma_bf16(a2[t], xo[mt][1], acc[mt][t]);
-                acc[mt][t] = mfma_bf16(a2[t], xo[mt][2], acc[mt][t]);
-            }
-    };
-    auto read_ops = [&](int xbuf, int b, u32x4 (&a)[2], u32x4 (&xo)[MB][3]) {
-#pragma unroll
-        for (int t = 0; t < 2; ++t)
-            a[t] = *reinterpret_cast<const u32x4 *>(wtw + swz(t * 16 + i16, b * 4 + g));
-#pragma unroll
-        for (int mt = 0; mt < MB; ++mt)
-#pragma unroll
-            for (int q = 0; q < 3; ++q) xo[mt][q] = xpl[xbuf][mt][b][q][lane];
-    };
-    // With 64-row tiles both k-blocks' operands are read from LDS up front,
-    // so the second block's reads are in flight during the first block's
-    // MFMAs (C2 up / down at m = 512: 233 / 239 us against 245 / 241).  With
-    // fewer tiles the extra registers would cost a workgroup per CU (m = 64:
-    // 67 / 68 us against 61 / 63), so each block's operands are read just
-    // before it.
-    auto compute = [&](int xbuf) {
-        if constexpr (MB == 4) {
-            u32x4 a[2][2], xo[2][MB][3];
-            read_ops(xbuf, 0, a[0], xo[0]);
-            read_ops(xbuf, 1, a[1], xo[1]);
-            block(a[0], xo[0]);
-            block(a[1], xo[1]);
-        } else {
-#pragma unroll
-            for (int b = 0; b < 2; ++b) {
-                u32x4 a[2], a2[2];
-                uint32_t mx = 0;
-#pragma unroll
-                for (int t = 0; t < 2; ++t) {
-                    a[t] = *reinterpret_cast<const u32x4 *>(wtw + swz(t * 16 + i16, b * 4 + g));
-#pragma unroll
-                    for (int v = 0; v < 4; ++v) mx = max_mag(mx, a[t][v]);
-                }
-                const bool any_special = wave_has_inf_nan(mx);
-#pragma unroll
-                for (int t = 0; t < 2; ++t) {
-                    a2[t] = a[t];
-                    if (any_special) {
-#pragma unroll
-                        for (int v = 0; v < 4; ++v) a2[t][v] &= ~inf_nan_mask(a2[t][v]);
-                    }
-                }
-#pragma unroll
-                for (int mt = 0; mt < MB; ++mt) {
-                    const u32x4 hi = xpl[xbuf][mt][b][0][lane], md = xpl[xbuf][mt][b][1][lane],
-                                lo = xpl[xbuf][mt][b][2][lane];
-#pragma unroll
-                    for (int t = 0; t < 2; ++t) {
-                        acc[mt][t] = mfma_bf16(a[t], hi, acc[mt][t]);
-                        acc[mt][t] = mfma_bf16(a2[t], md, acc[mt][t]);
-                        acc[mt][t] = mfma_bf16(a2[t], lo, acc[mt][t]);
-                    }
-                }
-            }
-        }
-    };
-
-    // A ring of D register sets: at step c chunk c is in LDS (x planes in
-    // buffer c&1), chunks c+1 .. c+D-1 are in flight to their sets, and the
-    // set chunk c arrived in (already in LDS) takes chunk c+D.
-    Regs r[D];
-#pragma unroll
-    for (int u = 0; u < D; ++u)
-        if (u < nchunks) load(u, r[u]);
-    if (nchunks > 0) store(r[0], 0);
-    __syncthreads();
-    for (int cb = 0; cb < nchunks; cb += D) {
-#pragma unroll
-        for (int u = 0; u < D; ++u) {
-            const int c = cb + u;
-            if (c >= nchunks) break;
-            if (c + D < nchunks) load(c + D, r[u]);
-            compute(c & 1);
-            if (c + 1 < nchunks) store(r[(u + 1) % D], (c + 1) & 1);
-            __syncthreads();
-        }
-    }
-
-#pragma unroll
-    for (int j = 0; j < kXPer; ++j)
-        if (xthread[j]) atomicMax(&xmax_s[xt[j] * 16 + (lane & 15)], hi_max(xmx[j]));
-    __syncthreads();
-    const int base[2] = {wave * 32, wave * 32 + 16};
-#pragma unroll
-    for (int mt = 0; mt < MB; ++mt) {
-        const int m = m0 + mt * 16 + i16;
-        bool live[2][4];
-#pragma unroll
-        for (int t = 0; t < 2; ++t)
-#pragma unroll
-            for (int rr = 0; rr < 4; ++rr) live[t][rr] = m < M && base[t] + g * 4 + rr < nrows;
-        const bool tiny = m < M && tiny_row(xmax_s[mt * 16 + i16]);
-        if (__builtin_amdgcn_ballot_w64(tiny) != 0) {  // this slice's chain (all of k without slices)
-#pragma unroll
-            for (int t = 0; t < 2; ++t)
-#pragma unroll
-                for (int rr = 0; rr < 4; ++rr)
-                    if (tiny && live[t][rr])
-                        acc[mt][t][rr] = reference_chain(W + (int64_t)(row0 + base[t] + g * 4 + rr) * K + 64 * c0,
-                                                         X + (int64_t)m * K + 64 * c0, 64 * nchunks);
-        }
-        if (P) {  // a k slice: the partial sums, for gemm_sum_slices_kernel
-            float *ps = P + (int64_t)bz * M * N + (int64_t)m * N + row0;
-#pragma unroll
-            for (int t = 0; t < 2; ++t)
-#pragma unroll
-                for (int rr = 0; rr < 4; ++rr)
-                    if (live[t][rr]) ps[base[t] + g * 4 + rr] = acc[mt][t][rr];
-            continue;
-        }
-        settle_zeros(acc[mt], live, base, W + (int64_t)row0 * K, X + (int64_t)(m0 + mt * 16) * K, K, i16);
-#pragma unroll
-        for (int t = 0; t < 2; ++t)
-#pragma unroll
-            for (int rr = 0; rr < 4; ++rr)
-                if (live[t][rr]) Y[(int64_t)m * N + row0 + base[t] + g * 4 + rr] = acc[mt][t][rr];
-    }
-}
-
-// x [M,K] f32 -> its three bf16 terms as planes XS[q][M][K] (split3 of each
-// element), for the gemm layout.  count = M*K, a multiple of 8; 16-byte
-// aligned.  Grid-stride.
-__global__ void __launch_bounds__(256)
-split_x_planes_kernel(const float *__restrict__ X, uint16_t *__restrict__ XS, int64_t count) {
-    for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < count / 8; i += (int64_t)gridDim.x * 256) {
-        const float4 a = reinterpret_cast<const float4 *>(X)[2 * i];
-        const float4 b = reinterpret_cast<const float4 *>(X)[2 * i + 1];
-        const float v[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
-        u32x4 hi, md, lo;
-        split8(v, hi, md, lo);
-        reinterpret_cast<u32x4 *>(XS)[i] = hi;
-        reinterpret_cast<u32x4 *>(XS + count)[i] = md;
-        reinterpret_cast<u32x4 *>(XS + 2 * count)[i] = lo;
-    }
-}
-
-// y[m][n] = P[0][m][n] + P[1][m][n] + ... in slice order, then the zero rule
-// of settle_zeros for one output: an exact zero is +0 when the activation row
-// or the weight row holds only +-0, else the reference chain's value.
-__global__ void __launch_bounds__(256)
-gemm_sum_slices_kernel(const float *__restrict__ P, int slices, float *__restrict__ Y, const uint16_t *__restrict__ W,
-                       const float *__restrict__ X, int M, int N, int K) {
-    const int64_t count = (int64_t)M * N;
-    for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < count; i += (int64_t)gridDim.x * 256) {
-        float s = P[i];
-#pragma unroll 8
-        for (int j = 1; j < slices; ++j) s += P[j * count + i];
-        if (s == 0.0f) {
-            const int m = (int)(i / N), n = (int)(i - (int64_t)m * N);
-            const uint32_t *xr = reinterpret_cast<const uint32_t *>(X + (int64_t)m * K);
-            const uint32_t *wr = reinterpret_cast<const uint32_t *>(W + (int64_t)n * K);
-            uint32_t xo = 0, wo = 0;
-            for (int k = 0; k < K; ++k) xo |= xr[k] & 0x7fffffffu;
-            for (int k = 0; k < K / 2; ++k) wo |= wr[k] & 0x7fff7fffu;
-            s = (xo && wo) ? reference_chain(W + (int64_t)n * K, X + (int64_t)m * K, K) : 0.0f;
-        }
-        Y[i] = s;
-    }
 }
 
 // Fifth MFMA layout ("rows16"), for a few activation rows: 16 weight rows per
@@ -3095,13 +2347,6 @@ int mt_for(int64_t m) {
     return 16;
 }
 
-bool aligned(const void *p, size_t a) { return (reinterpret_cast<uintptr_t>(p) % a) == 0; }
-
-int env_int(const char *name, int dflt) {
-    const char *v = getenv(name);
-    return (v && *v) ? atoi(v) : dflt;
-}
-
 template <int VEC, int ROWS, int MT>
 hipError_t rd_go(const RdProblem &p, const RdPlan &pl, hipStream_t s) {
     hipLaunchKernelGGL((gemv_rd_kernel<VEC, ROWS, MT>), dim3((unsigned)pl.grid_x, (unsigned)pl.grid_y),
@@ -3632,22 +2877,50 @@ RdPlan plan_rd(const RdProblem &p, int num_cus) {
             // m = 256: 124 / 125 against 140 / 135), except up at m = 192,
             // whose 168 tiles leave a third of the CUs idle (112 us on three
             // slices against 124 on one).
-            const int64_t tiles = ((p.n + mp.rpw - 1) / mp.rpw) * ((p.m + mp.mt - 1) / mp.mt);
             const int64_t nchunks = p.k / 64;
             const int64_t per_cu =
                 std::max(1, env_int("DMC_HIP_GEMM_PER_CU", mp.mt == 16 || mp.waves == 4 ? 2 : 1));
-            int64_t want = std::max<int64_t>(1, per_cu * cus / tiles);
-            if (tiles < cus && tiles * want * 10 < cus * 7) want = std::max<int64_t>(1, 2 * per_cu * cus / tiles);
-            // A slice of fewer than 8 chunks pays its pipeline fill and output
-            // too often: halve the split (C2 down at m = 12 / 16 on 16-row
-            // tiles: 35.0 / 37.2 us on 16 slices of 14 chunks against 37.3 /
-            // 40.4 on 32 of 7).
-            const int64_t min_chunks = std::max(1, env_int("DMC_HIP_GEMM_MIN_CHUNKS", 8));
-            while (want > 1 && (nchunks + want - 1) / want < min_chunks) want = (want + 1) / 2;
-            want = std::min<int64_t>({want, nchunks, (int64_t)env_int("DMC_HIP_GEMM_MAX_SLICES", 64)});
-            want = std::max<int64_t>(want, 1);
-            mp.kchunks = (int)((nchunks + want - 1) / want);
-            mp.kslices = (int)((nchunks + mp.kchunks - 1) / mp.kchunks);
+            const int64_t gx = (p.n + mp.rpw - 1) / mp.rpw;
+            const int fenv = env_int("DMC_HIP_GEMM_FUSE", 1);  // 0: never; 2: always
+            // The split for workgroups of `pair` activation tiles, and its time in us.
+            auto split = [&](int pair, RdPlan &o) {
+                const int64_t wgm = (int64_t)mp.mt * pair;
+                const int64_t tiles = gx * ((p.m + wgm - 1) / wgm);
+                int64_t want = std::max<int64_t>(1, per_cu * cus / tiles);
+                if (tiles < cus && tiles * want * 10 < cus * 7) want = std::max<int64_t>(1, 2 * per_cu * cus / tiles);
+                // A slice of fewer than 8 chunks pays its pipeline fill and output
+                // too often: halve the split (C2 down at m = 12 / 16 on 16-row
+                // tiles: 35.0 / 37.2 us on 16 slices of 14 chunks against 37.3 /
+                // 40.4 on 32 of 7).
+                const int64_t min_chunks = std::max(1, env_int("DMC_HIP_GEMM_MIN_CHUNKS", 8));
+                while (want > 1 && (nchunks + want - 1) / want < min_chunks) want = (want + 1) / 2;
+                want = std::min<int64_t>({want, nchunks, (int64_t)env_int("DMC_HIP_GEMM_MAX_SLICES", 64)});
+                want = std::max<int64_t>(want, 1);
+                o.mtiles = pair;
+                o.kchunks = (int)((nchunks + want - 1) / want);
+                o.kslices = (int)((nchunks + o.kchunks - 1) / o.kchunks);
+                o.xfuse = fenv == 2 || (fenv == 1 && (mp.mt == 16 || gx * p.m <= (pair == 2 ? 65536 : 8192)));
+                const int64_t rounds = (tiles * o.kslices + per_cu * cus - 1) / (per_cu * cus);
+                const double chunk = pair == 2 ? 2.65 : o.xfuse ? 1.55 : 1.75;
+                return (double)rounds * o.kchunks * chunk + 4 +
+                       (o.kslices > 1 ? 5 + 0.42e-6 * ((double)o.kslices * p.m * p.n * 4) : 0);
+            };
+            // 64-row tiles: one or two per workgroup (two take 2.65 us per 64-k
+            // chunk against 1.55, 1.75 with x's planes, but split k further
+            // where they leave CUs idle), whichever the sum of rounds x chunks
+            // x that time and the slice pass (5 us and 0.42 per MB of partials)
+            // puts ahead.  Measured, one / two, us: C2 up m = 65 / 128 / 192 /
+            // 256 / 512 / 1024 62.4 / 66.0 / 94.3 / 109 / 206 / 398 against 54.6
+            // / 60.5 / 92.1 / 96.0 / 165 / 320; C2 down m = 128 / 160 / 512 /
+            // 1024 62.7 / 78.4 / 183 / 389 against 60.8 / 87.6 / 170 / 307;
+            // [4096,4096] m = 128 / 256 / 512 / 1024 32.3 / 41.8 / 62.1 / 114
+            // against 34.6 / 44.3 / 59.6 / 99; [8192,1024] m = 512 / 1024 37.4 /
+            // 69.9 against 44.9 / 50.0.  DMC_HIP_GEMM_PAIR: 1 or 2 tiles always.
+            const int penv = env_int("DMC_HIP_GEMM_PAIR", 0);
+            const bool can_pair = mp.mt == 64 && mp.waves == 8 && (p.m > 64 || penv == 2) && penv != 1;
+            RdPlan one = mp, two = mp;
+            const double t1 = split(1, one);
+            mp = can_pair && (split(2, two) < t1 || penv == 2) ? two : one;
             // Workgroups split their own chunks of x (no planes, no split
             // launch) at 16-row tiles (C2 down at m = 16: the split launch cost
             // 3-4 us of 37), and at 32 and 64 while the repeated split stays
@@ -3657,9 +2930,9 @@ RdPlan plan_rd(const RdProblem &p, int num_cus) {
             // 50.7 / 75.1 / 120.1 / 218.7 (16 column blocks); up m = 32 / 64 /
             // 128 37.9 / 55.4 / 80.0 against 36.2 / 51.1 / 79.4, but m = 256 /
             // 512 122.2 / 230.8 against 126.0 / 248.0 (56 column blocks).
-            const int fenv = env_int("DMC_HIP_GEMM_FUSE", 1);  // 0: never; 2: always
-            const int64_t gx = (p.n + mp.rpw - 1) / mp.rpw;
-            mp.xfuse = fenv == 2 || (fenv == 1 && (mp.mt == 16 || gx * p.m <= 8192));
+            // Two 64-row tiles per workgroup read and split twice as much x per
+            // weight, and both in the kernel hold up to gx * m = 65536 (C2 up m =
+            // 512 181 / 170, down m = 2048 626 / 562).
             const size_t planes = mp.xfuse ? 0 : ((size_t)3 * p.m * p.k * 2 + 255) / 256 * 256;
             mp.workspace_bytes = planes + (mp.kslices > 1 ? (size_t)mp.kslices * p.m * p.n * 4 : 0);
         } else if (mp.mkind == 6) {
@@ -3957,42 +3230,7 @@ hipError_t launch_rd(const RdProblem &p, const RdPlan &pl, void *workspace, hipS
                                (int)p.m);
             return hipGetLastError();
         }
-        if (pl.mkind == 8) {
-            // The workspace holds x's planes (unless the kernel splits x
-            // itself) and the slice partials (when k is split): a fused
-            // single-slice plan needs none and may be given none.
-            const bool needs_ws = !pl.xfuse || pl.kslices > 1;
-            if ((needs_ws && !workspace) || (pl.mt != 16 && pl.mt != 32 && pl.mt != 64) || pl.kslices < 1 ||
-                pl.kslices > 65535 || (int64_t)pl.kslices * pl.kchunks < p.k / 64 || pl.rpw != 32 * pl.waves)
-                return hipErrorInvalidValue;
-            uint16_t *xs = pl.xfuse ? nullptr : static_cast<uint16_t *>(workspace);
-            const size_t planes = pl.xfuse ? 0 : ((size_t)3 * p.m * p.k * 2 + 255) / 256 * 256;
-            float *part = pl.kslices > 1 ? reinterpret_cast<float *>(static_cast<char *>(workspace) + planes) : nullptr;
-            const int64_t count = p.m * p.k;
-            if (!pl.xfuse)
-                hipLaunchKernelGGL(split_x_planes_kernel, dim3(stride_grid((count / 8 + 255) / 256)), dim3(256), 0,
-                                   s, p.x, xs, count);
-            const int64_t wgs = pl.grid_x * pl.grid_y * (int64_t)pl.kslices;
-            if (wgs > INT32_MAX) return hipErrorInvalidValue;
-            // The XCD-grouped tile order where activation tiles share weight
-            // blocks (DMC_HIP_GEMM_XCD: 0 never, 2 always).
-            const int xenv = env_int("DMC_HIP_GEMM_XCD", 1);
-            const int xcd = xenv == 2 || (xenv == 1 && pl.grid_y > 1) ? 1 : 0;
-#define DMC_GEMM(MB, F, NW)                                                                                  \
-    if (pl.mt == 16 * MB && pl.xfuse == F && pl.waves == NW)                                                 \
-        hipLaunchKernelGGL((gemv_rd_mfma_gemm_kernel<MB, F, NW>), dim3((unsigned)wgs), dim3(64 * NW), 0, s, p.w,  \
-                           p.x, xs, p.y, part, (int)p.n, (int)p.k, (int)p.m, pl.kchunks, (int)pl.grid_x,          \
-                           (int)pl.grid_y, xcd);                                                              \
-    else
-            DMC_GEMM(1, true, 8) DMC_GEMM(1, false, 8) DMC_GEMM(2, false, 8) DMC_GEMM(4, false, 8)
-            DMC_GEMM(2, false, 4) DMC_GEMM(4, false, 4) DMC_GEMM(2, true, 8) DMC_GEMM(4, true, 8)
-            DMC_GEMM(2, true, 4) DMC_GEMM(4, true, 4) return hipErrorInvalidValue;
-#undef DMC_GEMM
-            if (pl.kslices > 1)
-                hipLaunchKernelGGL(gemm_sum_slices_kernel, dim3(stride_grid((p.m * p.n + 255) / 256)), dim3(256), 0,
-                                   s, part, pl.kslices, p.y, p.w, p.x, (int)p.m, (int)p.n, (int)p.k);
-            return hipGetLastError();
-        }
+        if (pl.mkind == 8) return launch_gemm(p, pl, workspace, s);
         if (pl.mkind == 7) {
             const int tiles = pl.rpw / 16;
             const int ks = pl.kslices;
@@ -4009,9 +3247,7 @@ hipError_t launch_rd(const RdProblem &p, const RdPlan &pl, void *workspace, hipS
             DMC_R16(4, 1) DMC_R16(4, 2) DMC_R16(4, 4) DMC_R16(8, 1) DMC_R16(8, 2) DMC_R16(8, 4)
             DMC_R16(16, 1) DMC_R16(16, 2) DMC_R16(16, 4) return hipErrorInvalidValue;
 #undef DMC_R16
-            if (ks > 1)
-                hipLaunchKernelGGL(gemm_sum_slices_kernel, dim3(stride_grid((p.m * p.n + 255) / 256)), dim3(256), 0,
-                                   s, part, ks, p.y, p.w, p.x, (int)p.m, (int)p.n, (int)p.k);
+            if (ks > 1) return launch_sum_slices(part, ks, p, s);
             return hipGetLastError();
         }
         return hipErrorInvalidValue;

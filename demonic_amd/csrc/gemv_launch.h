@@ -70,6 +70,7 @@ struct RdPlan {
     // gemm layout (mkind 8): k split over `kslices` workgroups of `kchunks`
     // 64-element chunks each; workspace for x's bf16 planes and the partials
     int kslices = 1, kchunks = 0;
+    int mtiles = 1;  // gemm layout: activation tiles of `mt` rows per workgroup (1 or 2)
     bool xfuse = false;  // gemm layout, 16-row activation tiles: x split inside the kernel (no planes)
     // streaming over misaligned rows: windows cover k < kmain, and the 1..8
     // elements [kmain, k) are each row's short tail (0: kmain = k)
@@ -131,6 +132,10 @@ CsPlan plan_cs(const CsProblem &p, int num_cus);
 // when plan.slices > 1).  Returns hipSuccess or the launch error.
 hipError_t launch_rd(const RdProblem &p, const RdPlan &plan, void *workspace, hipStream_t stream);
 hipError_t launch_rd_group(const RdGroup &g, const RdPlan &plan, hipStream_t stream);
+// The gemm layout (plan.mkind == 8), and the sum of k-slice partials
+// part[slice][m][n] into p.y in slice order with the zero rule.
+hipError_t launch_gemm(const RdProblem &p, const RdPlan &plan, void *workspace, hipStream_t stream);
+hipError_t launch_sum_slices(const float *part, int slices, const RdProblem &p, hipStream_t stream);
 
 hipError_t launch_cs(const CsProblem &p, const CsPlan &plan, void *workspace, hipStream_t stream);
 
