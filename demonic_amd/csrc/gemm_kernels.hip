@@ -312,7 +312,8 @@ gemv_rd_mfma_gemm_kernel(const uint16_t *__restrict__ W, const float *__restrict
                 const uint64_t who = __builtin_amdgcn_ballot_w64(ask);
                 if (who == 0) continue;
                 const bool nz = wave_row_nonzero(readlane_ptr(wr, __builtin_ctzll(who)), K / 8, 0x7fff7fffu);
-                if (ask) *o = nz ? reference_chain(wr, xr, K) : 0.0f;
+                const float v = wave_chains(ask && nz, 0.0f, wr, 1, xr, K);
+                if (ask) *o = v;
             }
         }
     }
@@ -376,26 +377,38 @@ gemm_sum_slices_kernel(const float *__restrict__ P, int slices, float *__restric
                        const float *__restrict__ X, int M, int N, int K) {
     typedef float vec __attribute__((ext_vector_type(Q), aligned(4)));
     const int64_t count = (int64_t)M * N;
-    for (int64_t i = Q * ((int64_t)blockIdx.x * 256 + threadIdx.x); i < count; i += Q * (int64_t)gridDim.x * 256) {
+    for (int64_t i0 = Q * ((int64_t)blockIdx.x * 256 + threadIdx.x / 64 * 64); i0 < count;
+         i0 += Q * (int64_t)gridDim.x * 256) {  // wave-uniform
+        const int64_t own = i0 + Q * (threadIdx.x & 63);
+        const int64_t i = own < count ? own : count - Q;  // lanes past the end repeat the last outputs
         vec s = *reinterpret_cast<const vec *>(P + i);
 #pragma unroll 8
         for (int j = 1; j < slices; ++j) s += *reinterpret_cast<const vec *>(P + j * count + i);
         bool zero = false;
 #pragma unroll
         for (int e = 0; e < Q; ++e) zero |= s[e] == 0.0f;
-        if (zero) {
+        // Rare: the wave settles its lanes' zeros together, each activation row scanned once.
+        if (__builtin_amdgcn_ballot_w64(zero) != 0) {
             const int m = (int)(i / N), n = (int)(i - (int64_t)m * N);
-            const uint32_t *xr = reinterpret_cast<const uint32_t *>(X + (int64_t)m * K);
-            uint32_t xo = 0;
-            for (int k = 0; k < K; ++k) xo |= xr[k] & 0x7fffffffu;
+            bool xnz = false;
+            for (uint64_t todo = __builtin_amdgcn_ballot_w64(zero); todo;) {
+                const int mj = __builtin_amdgcn_readlane(m, __builtin_ctzll(todo));
+                const bool nz = wave_row_nonzero(X + (int64_t)mj * K, K / 4, 0x7fffffffu);
+                const bool same = zero && m == mj;
+                if (same) xnz = nz;
+                todo &= ~__builtin_amdgcn_ballot_w64(same);
+            }
 #pragma unroll
             for (int e = 0; e < Q; ++e) {
-                if (s[e] != 0.0f) continue;
-                const uint16_t *w = W + (int64_t)(n + e) * K;
-                const uint32_t *wr = reinterpret_cast<const uint32_t *>(w);
-                uint32_t wo = 0;
-                for (int k = 0; xo && k < K / 2; ++k) wo |= wr[k] & 0x7fff7fffu;
-                s[e] = wo ? reference_chain(w, X + (int64_t)m * K, K) : 0.0f;
+                const bool z = s[e] == 0.0f;
+                const uint16_t *const w = W + (int64_t)(n + e) * K;
+                bool chain = false;
+                for (uint64_t todo = __builtin_amdgcn_ballot_w64(z && xnz); todo; todo &= todo - 1) {
+                    const int j = __builtin_ctzll(todo);
+                    const bool nz = wave_row_nonzero(readlane_ptr(w, j), K / 8, 0x7fff7fffu);
+                    if ((int)(threadIdx.x & 63) == j) chain = nz;
+                }
+                s[e] = wave_chains(chain, z ? 0.0f : s[e], w, 1, X + (int64_t)m * K, K);
             }
         }
         *reinterpret_cast<vec *>(Y + i) = s;

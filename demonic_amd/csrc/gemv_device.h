@@ -148,6 +148,80 @@ __device__ bool wave_any_product(const float *x, const uint16_t *w, int64_t wste
     return false;
 }
 
+// The reference chain of one output by a whole wave (w, wstep, x, K wave-
+// uniform; wstep <= 1 means packed weights): the lanes load 512 elements at a
+// time, 8 each, the next 512 while these are summed, and the accumulator goes
+// from lane to lane, 8 dependent fmas and one readlane per lane.  A lane on
+// its own waits for memory every 8 elements: the chain of one output of
+// K = 14336 took 560 us that way, against 45 us here.  An exact zero from
+// ordinary data (full cancellation) is rare per output, ~3e-8, but a prefill
+// has millions of outputs: a few calls in a hundred at 1M, one in four at 8M.
+// Elements past K multiply +0 by -0: adding -0 keeps the accumulator.
+__device__ __attribute__((noinline)) float wave_chain(const uint16_t *w, int64_t wstep, const float *x, int K) {
+    const int lane = threadIdx.x & 63;
+    if (K <= 0) return 0.0f;
+    const bool packed = wstep <= 1 && K <= (1 << 28);
+    const uintptr_t wb = reinterpret_cast<uintptr_t>(w);
+    const uint32_t wd = packed ? (uint32_t)(wb & 3) : 0;  // 0 or 2
+    const __amdgpu_buffer_rsrc_t xr = weight_rsrc(x, packed ? (uint32_t)K * 4u : 0u);
+    const __amdgpu_buffer_rsrc_t wr =
+        weight_rsrc(reinterpret_cast<const void *>(wb - wd), packed ? wd + 2u * (uint32_t)K : 0u);
+    const uint32_t wlast = w[(int64_t)(K - 1) * wstep];  // its dword may straddle the range's end
+    struct Block {
+        float x[8], w[8];
+    };
+    auto load = [&](int k0, Block &b) {
+        const int e0 = k0 + lane * 8;
+        if (packed) {
+            const u32x4 xa = __builtin_amdgcn_raw_buffer_load_b128(xr, (uint32_t)e0 * 4u, 0, 0);
+            const u32x4 xc = __builtin_amdgcn_raw_buffer_load_b128(xr, (uint32_t)e0 * 4u + 16u, 0, 0);
+            const u32x4 wv = __builtin_amdgcn_raw_buffer_load_b128(wr, wd + (uint32_t)e0 * 2u, 0, 0);
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                b.x[e] = __uint_as_float(e < 4 ? xa[e] : xc[e - 4]);
+                uint32_t bits = (wv[e >> 1] >> (16 * (e & 1))) & 0xffffu;
+                bits = e0 + e == K - 1 ? wlast : bits;
+                b.w[e] = __uint_as_float((e0 + e < K ? bits : 0x8000u) << 16);
+            }
+        } else {
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                const int k = min(e0 + e, K - 1);
+                b.x[e] = e0 + e < K ? x[k] : 0.0f;
+                b.w[e] = __uint_as_float((e0 + e < K ? (uint32_t)w[(int64_t)k * wstep] : 0x8000u) << 16);
+            }
+        }
+    };
+    float acc = 0.0f;
+    Block cur, next;
+    load(0, cur);
+    for (int k0 = 0; k0 < K; k0 += 512) {
+        load(min(k0 + 512, K), next);
+        const int n = min(64, (K - k0 + 7) / 8);
+        for (int l = 0; l < n; ++l) {
+            float t = acc;
+#pragma unroll
+            for (int e = 0; e < 8; ++e) t = fmaf(cur.x[e], cur.w[e], t);
+            acc = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(t), l));
+        }
+        cur = next;
+    }
+    return acc;
+}
+
+// The chains of the lanes that ask for one (w, x per lane): a few one after
+// another by the whole wave, many one per lane.
+__device__ __forceinline__ float wave_chains(bool ask, float s, const uint16_t *w, int64_t wstep, const float *x, int K) {
+    uint64_t todo = __builtin_amdgcn_ballot_w64(ask);
+    if (__builtin_popcountll(todo) > 6) return ask ? chain_strided(w, wstep, x, K) : s;
+    for (; todo; todo &= todo - 1) {
+        const int j = __builtin_ctzll(todo);
+        const float v = wave_chain(readlane_ptr(w, j), wstep, readlane_ptr(x, j), K);
+        if ((int)(threadIdx.x & 63) == j) s = v;
+    }
+    return s;
+}
+
 // The zero rule for the outputs this wave holds, one per lane: `zero` marks a
 // lane whose output s is exactly 0 and is stored; x is its activation row,
 // w its first weight, wstep the elements between consecutive k.  All 64 lanes
@@ -175,8 +249,7 @@ __device__ float settle_zero(float s, bool zero, const float *x, const uint16_t 
         const bool hit = wave_any_product(readlane_ptr(x, j), readlane_ptr(w, j), wstep, K);
         if (lane == j) chain = hit;
     }
-    if (zero) s = chain ? chain_strided(w, wstep, x, K) : 0.0f;
-    return s;
+    return wave_chains(chain, zero ? 0.0f : s, w, wstep, x, K);
 }
 
 // ---- RD skinny M on MFMA: W [N,K] x X [M,K], K % 64 == 0 ---------------------------
@@ -400,7 +473,7 @@ __device__ void settle_zeros(f32x4 (&s)[T], const bool (&live)[T][4], const int 
     for (int t = 0; t < T; ++t)
 #pragma unroll
         for (int r = 0; r < 4; ++r)
-            if (chain[t][r]) s[t][r] = reference_chain(W + (int64_t)(base[t] + 4 * g + r) * K, X + (int64_t)m * K, K);
+            s[t][r] = wave_chains(chain[t][r], s[t][r], W + (int64_t)(base[t] + 4 * g + r) * K, 1, X + (int64_t)m * K, K);
 }
 
 // Weight and x tiles in LDS hold rows of 128 bytes, 8 pieces of 16, back to

@@ -1,13 +1,14 @@
 """GPU parity of the gemm layout's tiles (MFMA, many activation rows): one and
-two 64-row activation tiles per workgroup at the edges of both, with special
-values in the weights and in the activations, which send a tile through its
-second, hi-term pass."""
+two 64-row activation tiles per workgroup at the edges of both, special values
+in the weights and in the activations (which send a tile through its second,
+hi-term pass), and outputs whose exact zero sends one wave through the
+reference chain."""
 import numpy as np
 import pytest
 
 import oracle
 from demonic_amd import workloads as W
-from parity import check_or_bound
+from parity import check, check_bound, check_or_bound
 from test_gpu_parity import case, run_rd
 
 pytestmark = pytest.mark.gpu
@@ -31,3 +32,22 @@ def test_one_and_two_activation_tiles(hip, m, k, n, pair, fuse, monkeypatch):
     y_ref = oracle.matmul_bf16_t(x, w)
     assert y_ref[5, 13] == 0 and np.isposinf(y_ref[2, 9])
     check_or_bound(run_rd(hip, x, w), y_ref, x, W.bf16_to_f32(w), f"gemm pair={pair} fuse={fuse} {m}x{k}x{n}")
+
+
+@pytest.mark.parametrize("slices", [1, 4])
+def test_a_lone_cancelling_output_takes_the_chain(hip, slices, monkeypatch):
+    """One output in 80 x 300 whose sum is exactly zero, K long enough for
+    several rounds of the wave's chain: the reference's bits."""
+    m, k, n = 80, 3008, 300
+    monkeypatch.setenv("DMC_HIP_RD_MFMA_KIND", "8")
+    monkeypatch.setenv("DMC_HIP_GEMM_MAX_SLICES", str(slices))
+    x, w = case(m, k, n, seed=5, scale=0.02)
+    x[70] = 1
+    w[200, : k // 2], w[200, k // 2:] = 0x3F80, 0xBF80
+    y_ref = oracle.matmul_bf16_t(x, w)
+    assert y_ref[70, 200] == 0
+    y = run_rd(hip, x, w)
+    assert y[70, 200].view(np.uint32) == y_ref[70, 200].view(np.uint32)
+    check(y, y_ref, what="lone zero")
+    for r in (0, 70, 79):
+        check_bound(y[r], y_ref[r], x[r], W.bf16_to_f32(w), what=f"lone zero row {r}")
