@@ -1,5 +1,5 @@
-// gemm_kernels.hip -- the MFMA "gemm" layout: bf16 weights against 9 and more
-// f32 activation rows (prefill and large decode batches), W [N,K].
+// gemm_kernels.hip -- the MFMA "gemm" layout: bf16 weights against several to
+// thousands of f32 activation rows (prefill and large decode batches).
 #include "gemv_device.h"
 #include "gemv_launch.h"
 
@@ -40,6 +40,25 @@ namespace {
 // 911 / 602 (1.2 PFLOP/s of MFMA; a large bf16 matrix product through the
 // vendor library reaches 1.25 on this card), up m = 64 47.2 / 38.3.
 //
+// Where W lies (SRC): packed rows [N,K], K a multiple of 64, 16-byte aligned
+// (kSrcPacked); rows [N,K] of any length and alignment (kSrcRows); columns, W [K,N]
+// (kSrcCols).  Only the way of a chunk into the weight tile differs:
+//   - kSrcRows reads the same 16-byte pieces at the rows' own 2-byte alignment
+//     (exact on gfx950, checked per dword), and clears what lies past K in the
+//     last chunk, in W (the next row's start, which may be an inf) and in x;
+//   - kSrcCols reads 8 k rows of 512 bytes per wave, 4 columns per lane, and turns
+//     each lane's 8 x 4 block with 16 byte permutes into 4 pieces of 8 k.
+// A dword that runs past the matrix reads as zeros, and with K (kSrcCols: N) odd
+// the matrix's last element shares one: it is read alone and put in.
+//
+// The kSrcRows and kSrcCols forms replace FMA kernels whose sums are spread over many
+// lanes, 3 to 7 times closer to the exact value than one MFMA chain over all of
+// k (each MFMA rounds the running sum; measured, K = 4096: 1.1e-7 against
+// 7e-7).  They keep that: every k-block of 32 is summed from zero (lo, mid, hi:
+// one rounding at full size), the blocks are added up in f32, and those sums
+// once more every `fold` chunks, these and the k slices with the rounding
+// errors of their sums kept.
+//
 // When the tiles would leave the device short of workgroups, k is split over
 // `slices` workgroups of kc chunks each, whose partial sums go to
 // P[slice][m][n] for gemm_sum_slices_kernel.  Special values, tiny activation
@@ -47,6 +66,7 @@ namespace {
 // zero rule runs after the sum.
 typedef f32x4 f32x4_u __attribute__((aligned(4)));  // y's rows may start at any float
 constexpr uint32_t kDeadLane = 0x80000000u;   // lane offset past every buffer: zeros, no traffic
+enum Src { kSrcPacked, kSrcRows, kSrcCols };
 constexpr uint32_t kDeadChunk = 0x7fff0000u;  // scalar offset of a chunk past the last (no 32-bit wrap with kDeadLane)
 
 // The three bf16 terms of eight values by truncation alone: split3's terms for
@@ -67,12 +87,43 @@ __device__ __forceinline__ void split8_finite(const float (&v)[8], u32x4 (&t)[3]
     }
 }
 
-template <int NWV, int MT, bool FUSE>
-__global__ void __launch_bounds__(64 * NWV) __attribute__((amdgpu_waves_per_eu(MT == 16 ? 4 : 2)))
-gemv_rd_mfma_gemm_kernel(const uint16_t *__restrict__ W, const float *__restrict__ X, const uint16_t *__restrict__ XS,
-                         float *__restrict__ Y, float *__restrict__ P, int N, int K, int M, int kc, int gx, int gy,
-                         int xcd) {
+// The weight tile's swizzle for columns: a lane's pieces go to rows 4 apart
+// there (swz spreads rows 1 apart), so row bit 4 takes part too.
+__device__ __forceinline__ int swz_cols(int r, int p) {
+    return r * 128 + ((p ^ (((r >> 1) ^ (r >> 4 & 1)) & 7)) << 4);
+}
+
+// Does some weight of a row (wstep 1) or a column (wstep N) differ from +-0?  Wave-uniform; the rare path.
+__device__ bool wave_weights_nonzero(const uint16_t *w, int64_t wstep, int K) {
+    constexpr int U = 16;
+    for (int k0 = 0; k0 < K; k0 += 64 * U) {
+        uint32_t hit = 0;
+#pragma unroll
+        for (int u = 0; u < U; ++u) hit |= w[(int64_t)min(k0 + u * 64 + (int)(threadIdx.x & 63), K - 1) * wstep];
+        if (__builtin_amdgcn_ballot_w64((hit & 0x7fffu) != 0) != 0) return true;
+    }
+    return false;
+}
+
+// s += p, and what the rounding of that sum lost.
+__device__ __forceinline__ float add_exact(float &s, float p) {
+    const float t = s + p, b = t - s;
+    const float e = (s - (t - b)) + (p - b);
+    s = t;
+    return e;
+}
+// (Sums that are not finite have no meaningful loss.)
+__device__ __forceinline__ float add_lost(float s, float e) { return fabsf(s) < __builtin_inff() ? s + e : s; }
+
+template <int NWV, int MT, int SRC, bool FUSE>
+__global__ void __launch_bounds__(64 * NWV) __attribute__((amdgpu_waves_per_eu(MT == 16 && SRC == kSrcPacked ? 4 : 2)))
+gemv_mfma_gemm_kernel(const uint16_t *__restrict__ W, const float *__restrict__ X, const uint16_t *__restrict__ XS,
+                      float *__restrict__ Y, float *__restrict__ P, int N, int K, int M, int kc, int gx, int gy,
+                      int xcd, int64_t w_batch, int64_t x_batch) {
     static_assert(NWV == 4 || NWV == 8, "32 weight rows per wave");
+    static_assert(SRC == kSrcPacked || (NWV == 8 && FUSE), "the general forms split x themselves, on 8 waves");
+    static_assert(SRC == kSrcPacked || MT <= 64, "register budget");
+    constexpr bool kTwoLevel = SRC != kSrcPacked;
     static_assert(MT == 16 || MT == 32 || MT == 64 || MT == 128, "activation rows per workgroup");
     constexpr int kRows = 32 * NWV;
     constexpr int XT = MT / 16;                    // 16-row activation tiles
@@ -105,20 +156,38 @@ gemv_rd_mfma_gemm_kernel(const uint16_t *__restrict__ W, const float *__restrict
     const int nrows = min(kRows, N - row0);
     const int m0 = by * MT;
     const int c0 = bz * kc;  // this slice's chunks: [c0, c0 + nch)
-    const int nch = max(0, min(K / 64, c0 + kc) - c0);
+    const int nck = SRC == kSrcPacked ? K / 64 : (K + 63) / 64;  // chunks of k in all
+    const int nch = max(0, min(nck, c0 + kc) - c0);
+    if (SRC == kSrcCols) {  // batch slice blockIdx.y (P: [z][slice][m][n])
+        W += blockIdx.y * w_batch;
+        X += blockIdx.y * x_batch;
+        Y += (int64_t)blockIdx.y * M * N;
+        if (P) P += (int64_t)blockIdx.y * (gridDim.x / (uint32_t)(gx * gy)) * M * N;
+    }
+    const int64_t wstep = SRC == kSrcCols ? N : 1;                      // elements between a weight row's k
+    const uint16_t *const wrow0 = SRC == kSrcCols ? W + row0 : W + (int64_t)row0 * K;
+    const int64_t wpitch = SRC == kSrcCols ? 1 : K;                     // ... and between weight rows
+    auto tile_at = [](int r, int p) { return SRC == kSrcCols ? swz_cols(r, p) : swz(r, p); };
 
     __shared__ __attribute__((aligned(16))) uint8_t wt[2][kRows * 128];  // swizzled 128-byte rows (swz)
     __shared__ u32x4 xp[2][XT][2][3][64];                                // operand order: conflict-free
 
-    const __amdgpu_buffer_rsrc_t rs = weight_rsrc(W + (int64_t)row0 * K, (uint32_t)((int64_t)nrows * K * 2));
+    // kSrcRows: up to 16 bytes of the row after the block, so that only the matrix's own end cuts a dword.
+    const __amdgpu_buffer_rsrc_t rs =
+        SRC == kSrcCols   ? weight_rsrc(W, (uint32_t)((int64_t)K * N * 2))
+        : SRC == kSrcRows ? weight_rsrc(wrow0, (uint32_t)min((int64_t)nrows * K * 2 + 16, (int64_t)(N - row0) * K * 2))
+                       : weight_rsrc(wrow0, (uint32_t)((int64_t)nrows * K * 2));
     const uint32_t plane_bytes = (uint32_t)M * (uint32_t)K * 2u;
     const __amdgpu_buffer_rsrc_t xrs = FUSE ? weight_rsrc(X, 2u * plane_bytes) : weight_rsrc(XS, 3u * plane_bytes);
-    // W staging: item j of a wave is rows 32 * wave + 8j + lane/8, 16 bytes per lane: whole lines.
+    // W staging: item j of a wave is rows 32 * wave + 8j + lane/8, 16 bytes per lane: whole lines
+    // (kSrcCols: k rows 8 * wave + 2j and + 1, columns 4 * lane of each).
     const int slr = wave * 32 + (lane >> 3);
     uint32_t woff[4];
 #pragma unroll
     for (int j = 0; j < 4; ++j)
-        woff[j] = (uint32_t)min(slr + 8 * j, nrows - 1) * (uint32_t)K * 2u + (lane & 7) * 16;
+        woff[j] = SRC == kSrcCols ? (uint32_t)(row0 + 4 * lane) * 2u
+                               : (uint32_t)min(slr + 8 * j, nrows - 1) * (uint32_t)K * 2u + (lane & 7) * 16;
+    const uint32_t wlast = SRC == kSrcPacked ? 0 : W[(int64_t)N * K - 1];  // the matrix's last element
     // x staging: item it = (tile it/2, k-block it%2), 8 elements of row i16 per lane.
     uint32_t xoff[XI];
 #pragma unroll
@@ -138,7 +207,21 @@ gemv_rd_mfma_gemm_kernel(const uint16_t *__restrict__ W, const float *__restrict
         const uint32_t cb = (uint32_t)(c0 + rotate_chunk(c, s0, nch)) * 128u;
         const uint32_t wb = live ? cb : kDeadChunk;
 #pragma unroll
-        for (int j = 0; j < 4; ++j) r.w[j] = load_w16(rs, woff[j], wb);
+        for (int j = 0; j < 4; ++j) {
+            if constexpr (SRC == kSrcCols) {
+                const uint32_t k = (uint32_t)(c0 + rotate_chunk(c, s0, nch)) * 64u + wave * 8 + 2 * j;
+#pragma unroll
+                for (int h = 0; h < 2; ++h) {
+                    const auto v = __builtin_amdgcn_raw_buffer_load_b64(
+                        rs, woff[j], live ? (k + h) * (uint32_t)N * 2u : kDeadChunk, kLoadNT);
+                    r.w[j][2 * h] = v[0];
+                    r.w[j][2 * h + 1] = v[1];
+                }
+            } else {
+                // (kSrcRows: not nontemporal, since a row's chunk spans two lines, each half another chunk's.)
+                r.w[j] = __builtin_amdgcn_raw_buffer_load_b128(rs, woff[j], wb, SRC == kSrcRows ? 0 : kLoadNT);
+            }
+        }
 #pragma unroll
         for (int j = 0; j < XI; ++j) {
 #pragma unroll
@@ -152,10 +235,56 @@ gemv_rd_mfma_gemm_kernel(const uint16_t *__restrict__ W, const float *__restrict
     uint32_t xmx[XI];  // the largest |x| staged (f32 bits; the hi term's with planes), per lane
 #pragma unroll
     for (int j = 0; j < XI; ++j) xmx[j] = 0;
-    auto store = [&](const Regs &r, int buf, auto TERMS) __attribute__((always_inline)) {
+    // Chunk c's staged registers into LDS buffer `buf`.
+    auto store = [&](Regs &r, int c, int buf, auto TERMS) __attribute__((always_inline)) {
         constexpr int terms = decltype(TERMS)::value;
+        if constexpr (SRC != kSrcPacked) {
+            const int at = c < nch ? c0 + rotate_chunk(c, s0, nch) : -1;
+            if (at == nck - 1) {  // the last chunk of k: wave-uniform, one in nck
+                int kt = K - 64 * at;  // its elements
+                asm volatile("" : "+s"(kt));  // keep the masks below out of the loop's registers
+                if constexpr (SRC == kSrcRows) {
 #pragma unroll
-        for (int j = 0; j < 4; ++j) *reinterpret_cast<u32x4 *>(wt[buf] + swz(slr + 8 * j, lane & 7)) = r.w[j];
+                    for (int j = 0; j < 4; ++j) {
+                        const int left = kt - (lane & 7) * 8;  // of this piece
+                        const bool end = (K & 1) && row0 + slr + 8 * j == N - 1 && left >= 1 && left <= 8;
+#pragma unroll
+                        for (int v = 0; v < 4; ++v) {
+                            if (end && (left - 1) >> 1 == v) r.w[j][v] = wlast;
+                            r.w[j][v] &= (2 * v < left ? 0xffffu : 0u) | (2 * v + 1 < left ? 0xffff0000u : 0u);
+                        }
+                    }
+                } else if (N & 1) {
+#pragma unroll
+                    for (int j = 0; j < 4; ++j)
+#pragma unroll
+                        for (int v = 0; v < 4; ++v)
+                            if (wave * 8 + 2 * j + (v >> 1) == kt - 1 && row0 + 4 * lane + 2 * (v & 1) == N - 1)
+                                r.w[j][v] = wlast;
+                }
+#pragma unroll
+                for (int j = 0; j < XI; ++j) {
+                    const int left = kt - ((wave * XI + j) & 1) * 32 - g * 8;
+#pragma unroll
+                    for (int e = 0; e < 8; ++e)
+                        if (e >= left) r.x[j][e >> 2][e & 3] = 0;
+                }
+            }
+        }
+        if constexpr (SRC == kSrcCols) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {  // column 4 * lane + e: this wave's 8 k, two per dword
+                u32x4 piece;
+#pragma unroll
+                for (int v = 0; v < 4; ++v)
+                    piece[v] = __builtin_amdgcn_perm(r.w[v][2 + (e >> 1)], r.w[v][e >> 1],
+                                                     e & 1 ? 0x07060302u : 0x05040100u);
+                *reinterpret_cast<u32x4 *>(wt[buf] + tile_at(4 * lane + e, wave)) = piece;
+            }
+        } else {
+#pragma unroll
+            for (int j = 0; j < 4; ++j) *reinterpret_cast<u32x4 *>(wt[buf] + tile_at(slr + 8 * j, lane & 7)) = r.w[j];
+        }
 #pragma unroll
         for (int j = 0; j < XI; ++j) {
             const int it = wave * XI + j;
@@ -189,11 +318,15 @@ gemv_rd_mfma_gemm_kernel(const uint16_t *__restrict__ W, const float *__restrict
     };
 
     f32x4 acc[RM][RN];
+    // kTwoLevel: the sums of all (with their rounding errors) and of the
+    // current `fold` chunks.
+    float total[kTwoLevel ? RM : 1][RN][4], lost[kTwoLevel ? RM : 1][RN][4], part[kTwoLevel ? RM : 1][RN][4];
+    const int fold = kTwoLevel ? max(1, (int)(0.5f * sqrtf(2.0f * nch) + 0.5f)) : 0;
     u32x4 a[2][RN], xo[2][3];  // operands: weights per k-block, x per step
     auto read_a = [&](int buf, int kb) __attribute__((always_inline)) {
 #pragma unroll
         for (int j = 0; j < RN; ++j)
-            a[kb][j] = *reinterpret_cast<const u32x4 *>(wt[buf] + swz((wn * RN + j) * 16 + i16, kb * 4 + g));
+            a[kb][j] = *reinterpret_cast<const u32x4 *>(wt[buf] + tile_at((wn * RN + j) * 16 + i16, kb * 4 + g));
     };
     auto read_x = [&](int buf, int kb, int mf, int set) __attribute__((always_inline)) {
 #pragma unroll
@@ -215,7 +348,7 @@ gemv_rd_mfma_gemm_kernel(const uint16_t *__restrict__ W, const float *__restrict
                 read_x(buf, (s + 1) / RM, (s + 1) % RM, (s + 1) & 1);
             }
             if (s == NS - 2) {
-                store(r, buf ^ 1, TERMS);
+                store(r, c + 1, buf ^ 1, TERMS);
                 load(c + 2, r);
             }
             if (s == NS - 1) {
@@ -223,30 +356,83 @@ gemv_rd_mfma_gemm_kernel(const uint16_t *__restrict__ W, const float *__restrict
                 read_a(buf ^ 1, 0);
                 read_x(buf ^ 1, 0, 0, 0);
             }
+            constexpr int terms = decltype(TERMS)::value;
+            if constexpr (kTwoLevel) {
+                f32x4 blk[RN];
 #pragma unroll
-            for (int q = 0; q < decltype(TERMS)::value; ++q)
+                for (int j = 0; j < RN; ++j) blk[j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-                for (int j = 0; j < RN; ++j) acc[mf][j] = mfma_bf16(a[kb][j], xo[s & 1][q], acc[mf][j]);
+                for (int q = terms - 1; q >= 0; --q)
+#pragma unroll
+                    for (int j = 0; j < RN; ++j) blk[j] = mfma_bf16(a[kb][j], xo[s & 1][q], blk[j]);
+                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int j = 0; j < RN; ++j)
+#pragma unroll
+                    for (int v = 0; v < 4; ++v) {
+                        part[mf][j][v] += blk[j][v];
+                        asm volatile("" : "+v"(part[mf][j][v]));  // here, not after the chunk (registers)
+                    }
+            } else {
+#pragma unroll
+                for (int q = 0; q < terms; ++q)
+#pragma unroll
+                    for (int j = 0; j < RN; ++j) acc[mf][j] = mfma_bf16(a[kb][j], xo[s & 1][q], acc[mf][j]);
+            }
             __builtin_amdgcn_sched_barrier(0);
         }
+    };
+    auto fold_parts = [&]() __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < RM; ++i)
+#pragma unroll
+            for (int j = 0; j < RN; ++j)
+#pragma unroll
+                for (int v = 0; v < 4; ++v) {
+                    lost[i][j][v] += add_exact(total[i][j][v], part[i][j][v]);
+                    part[i][j][v] = 0.0f;
+                }
     };
     auto stream = [&](auto TERMS) __attribute__((always_inline)) {
 #pragma unroll
         for (int i = 0; i < RM; ++i)
 #pragma unroll
-            for (int j = 0; j < RN; ++j) acc[i][j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+            for (int j = 0; j < RN; ++j) {
+                if constexpr (kTwoLevel) {
+#pragma unroll
+                    for (int v = 0; v < 4; ++v) total[i][j][v] = lost[i][j][v] = part[i][j][v] = 0.0f;
+                } else {
+                    acc[i][j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+                }
+            }
         load(0, r);
-        store(r, 0, TERMS);
+        store(r, 0, 0, TERMS);
         load(1, r);
         lds_barrier();
         read_a(0, 0);
         read_x(0, 0, 0, 0);
         int c = 0;
+        int until = fold;
         for (; c + 1 < nch; c += 2) {
             chunk(c, std::integral_constant<int, 0>{}, TERMS);
             chunk(c + 1, std::integral_constant<int, 1>{}, TERMS);
+            if constexpr (kTwoLevel) {
+                if (c + 2 >= until) {
+                    fold_parts();
+                    until = c + 2 + fold;
+                }
+            }
         }
         if (c < nch) chunk(c, std::integral_constant<int, 0>{}, TERMS);
+        if constexpr (kTwoLevel) {
+            fold_parts();
+#pragma unroll
+            for (int i = 0; i < RM; ++i)
+#pragma unroll
+                for (int j = 0; j < RN; ++j)
+#pragma unroll
+                    for (int v = 0; v < 4; ++v) acc[i][j][v] = add_lost(total[i][j][v], lost[i][j][v]);
+        }
     };
     stream(std::integral_constant<int, 3>{});
 
@@ -266,12 +452,10 @@ gemv_rd_mfma_gemm_kernel(const uint16_t *__restrict__ W, const float *__restrict
     // l%16.  They are stored as they are; the rare ones that the sums do not
     // settle (a tiny row, an exact zero, a value that is not finite) are redone.
     float *const out = (P ? P + (int64_t)bz * M * N : Y) + row0;
-    bool rare = false;
-    uint32_t big[RM];  // bit 4j + v: the output is not finite
+    bool rare = false, big = false;  // big: some output is not finite
 #pragma unroll
     for (int mf = 0; mf < RM; ++mf) {
         const int ml = (wm * RM + mf) * 16 + i16;
-        big[mf] = 0;
         if (m0 + ml >= M) continue;
         rare |= xmax_s[ml] != 0 && xmax_s[ml] < kTinyHiBits << 16;
         float *const o = out + (int64_t)(m0 + ml) * N;
@@ -288,7 +472,7 @@ gemv_rd_mfma_gemm_kernel(const uint16_t *__restrict__ W, const float *__restrict
 #pragma unroll
             for (int v = 0; v < 4; ++v) {
                 rare |= !P && n + v < nrows && acc[mf][j][v] == 0.0f;
-                if (n + v < nrows && !(fabsf(acc[mf][j][v]) < __builtin_inff())) big[mf] |= 1u << (4 * j + v);
+                big |= n + v < nrows && !(fabsf(acc[mf][j][v]) < __builtin_inff());
             }
         }
     }
@@ -300,19 +484,24 @@ gemv_rd_mfma_gemm_kernel(const uint16_t *__restrict__ W, const float *__restrict
             const bool live = m0 + ml < M && n < nrows;
             const uint32_t xm = xmax_s[ml];
             const float *const xr = X + (int64_t)min(m0 + ml, M - 1) * K;
-            const uint16_t *const wr = W + (int64_t)(row0 + min(n, nrows - 1)) * K;
+            const uint16_t *const wr = wrow0 + min(n, nrows - 1) * wpitch;
             float *const o = out + (int64_t)(m0 + ml) * N + n;
             const bool tiny = live && xm != 0 && xm < kTinyHiBits << 16;
             const bool zero = live && !tiny && !P && *o == 0.0f;
-            if (tiny) *o = reference_chain(wr + 64 * c0, xr + 64 * c0, 64 * nch);  // this slice's chain
+            if (tiny)  // this slice's chain
+                *o = SRC == kSrcPacked ? reference_chain(wr + 64 * c0, xr + 64 * c0, 64 * nch)
+                                    : chain_strided(wr + 64 * c0 * wstep, wstep, xr + 64 * c0,
+                                                    min(64 * nch, K - 64 * c0));
             if (zero && xm == 0) *o = 0.0f;  // an activation row of +-0
             // Zeros of the other rows: +0 where the weight row holds only +-0, else the chain.
             for (int gq = 0; gq < 4; ++gq) {
                 const bool ask = zero && xm != 0 && g == gq;
                 const uint64_t who = __builtin_amdgcn_ballot_w64(ask);
                 if (who == 0) continue;
-                const bool nz = wave_row_nonzero(readlane_ptr(wr, __builtin_ctzll(who)), K / 8, 0x7fff7fffu);
-                const float v = wave_chains(ask && nz, 0.0f, wr, 1, xr, K);
+                const uint16_t *const wu = readlane_ptr(wr, __builtin_ctzll(who));
+                const bool nz = SRC == kSrcPacked ? wave_row_nonzero(wu, K / 8, 0x7fff7fffu)
+                                               : wave_weights_nonzero(wu, wstep, K);
+                const float v = wave_chains(ask && nz, 0.0f, wr, wstep, xr, K);
                 if (ask) *o = v;
             }
         }
@@ -327,12 +516,9 @@ gemv_rd_mfma_gemm_kernel(const uint16_t *__restrict__ W, const float *__restrict
     // not finite either.  (Screening W in the loop and clearing such weights
     // for mid and lo cost 12-18% of it, for weights that hold none.)
     uint32_t *const any_s = xmax_s + MT;
-    bool mine = false;
-#pragma unroll
-    for (int mf = 0; mf < RM; ++mf) mine |= big[mf] != 0;
     if (tid == 0) *any_s = 0;
     __syncthreads();
-    if (mine) *any_s = 1;
+    if (big) *any_s = 1;
     __syncthreads();
     const bool again = *any_s != 0;
     __syncthreads();
@@ -340,13 +526,17 @@ gemv_rd_mfma_gemm_kernel(const uint16_t *__restrict__ W, const float *__restrict
     stream(std::integral_constant<int, 1>{});
 #pragma unroll
     for (int mf = 0; mf < RM; ++mf) {
-        float *const o = out + (int64_t)(m0 + (wm * RM + mf) * 16 + i16) * N;
+        const int ml = (wm * RM + mf) * 16 + i16;
+        if (m0 + ml >= M) continue;
 #pragma unroll
         for (int j = 0; j < RN; ++j)
 #pragma unroll
-            for (int v = 0; v < 4; ++v)
-                if ((big[mf] >> (4 * j + v) & 1u) && !(fabsf(acc[mf][j][v]) < __builtin_inff()))
-                    o[(wn * RN + j) * 16 + g * 4 + v] = acc[mf][j][v];
+            for (int v = 0; v < 4; ++v) {
+                const int n = (wn * RN + j) * 16 + g * 4 + v;
+                float *const o = out + (int64_t)(m0 + ml) * N + n;
+                if (n < nrows && !(fabsf(*o) < __builtin_inff()) && !(fabsf(acc[mf][j][v]) < __builtin_inff()))
+                    *o = acc[mf][j][v];
+            }
     }
 }
 
@@ -371,19 +561,45 @@ split_x_planes_kernel(const float *__restrict__ X, uint16_t *__restrict__ XS, in
 // or the weight row holds only +-0, else the reference chain's value.  Q
 // outputs per thread (4 where N is a multiple of 4, so that they share an
 // activation row): 16-byte loads, up to 8 slices' in flight.
-template <int Q>
+// PACKED: W as in kSrcPacked, else rows (wstep 1) or columns (wstep N, batch slice
+// blockIdx.y) of any size.
+template <int Q, bool PACKED>
 __global__ void __launch_bounds__(256)
 gemm_sum_slices_kernel(const float *__restrict__ P, int slices, float *__restrict__ Y, const uint16_t *__restrict__ W,
-                       const float *__restrict__ X, int M, int N, int K) {
+                       const float *__restrict__ X, int M, int N, int K, int64_t wstep, int64_t w_batch,
+                       int64_t x_batch) {
     typedef float vec __attribute__((ext_vector_type(Q), aligned(4)));
     const int64_t count = (int64_t)M * N;
+    if (!PACKED) {
+        P += (int64_t)blockIdx.y * slices * count;
+        Y += (int64_t)blockIdx.y * count;
+        W += blockIdx.y * w_batch;
+        X += blockIdx.y * x_batch;
+    }
     for (int64_t i0 = Q * ((int64_t)blockIdx.x * 256 + threadIdx.x / 64 * 64); i0 < count;
          i0 += Q * (int64_t)gridDim.x * 256) {  // wave-uniform
         const int64_t own = i0 + Q * (threadIdx.x & 63);
         const int64_t i = own < count ? own : count - Q;  // lanes past the end repeat the last outputs
         vec s = *reinterpret_cast<const vec *>(P + i);
+        float lost[Q] = {};  // !PACKED: what the sum's roundings lost
 #pragma unroll 8
-        for (int j = 1; j < slices; ++j) s += *reinterpret_cast<const vec *>(P + j * count + i);
+        for (int j = 1; j < slices; ++j) {
+            const vec p = *reinterpret_cast<const vec *>(P + j * count + i);
+            if (PACKED) {
+                s += p;
+            } else {
+#pragma unroll
+                for (int e = 0; e < Q; ++e) {
+                    float t = s[e];
+                    lost[e] += add_exact(t, p[e]);
+                    s[e] = t;
+                }
+            }
+        }
+        if (!PACKED) {
+#pragma unroll
+            for (int e = 0; e < Q; ++e) s[e] = add_lost(s[e], lost[e]);
+        }
         bool zero = false;
 #pragma unroll
         for (int e = 0; e < Q; ++e) zero |= s[e] == 0.0f;
@@ -393,7 +609,8 @@ gemm_sum_slices_kernel(const float *__restrict__ P, int slices, float *__restric
             bool xnz = false;
             for (uint64_t todo = __builtin_amdgcn_ballot_w64(zero); todo;) {
                 const int mj = __builtin_amdgcn_readlane(m, __builtin_ctzll(todo));
-                const bool nz = wave_row_nonzero(X + (int64_t)mj * K, K / 4, 0x7fffffffu);
+                const float *const xr = X + (int64_t)mj * K;
+                const bool nz = PACKED ? wave_row_nonzero(xr, K / 4, 0x7fffffffu) : wave_any_product(xr, nullptr, 0, K);
                 const bool same = zero && m == mj;
                 if (same) xnz = nz;
                 todo &= ~__builtin_amdgcn_ballot_w64(same);
@@ -401,14 +618,15 @@ gemm_sum_slices_kernel(const float *__restrict__ P, int slices, float *__restric
 #pragma unroll
             for (int e = 0; e < Q; ++e) {
                 const bool z = s[e] == 0.0f;
-                const uint16_t *const w = W + (int64_t)(n + e) * K;
+                const uint16_t *const w = W + (int64_t)(n + e) * (wstep == 1 ? K : 1);
                 bool chain = false;
                 for (uint64_t todo = __builtin_amdgcn_ballot_w64(z && xnz); todo; todo &= todo - 1) {
                     const int j = __builtin_ctzll(todo);
-                    const bool nz = wave_row_nonzero(readlane_ptr(w, j), K / 8, 0x7fff7fffu);
+                    const uint16_t *const wu = readlane_ptr(w, j);
+                    const bool nz = PACKED ? wave_row_nonzero(wu, K / 8, 0x7fff7fffu) : wave_weights_nonzero(wu, wstep, K);
                     if ((int)(threadIdx.x & 63) == j) chain = nz;
                 }
-                s[e] = wave_chains(chain, z ? 0.0f : s[e], w, 1, X + (int64_t)m * K, K);
+                s[e] = wave_chains(chain, z ? 0.0f : s[e], w, wstep, X + (int64_t)m * K, K);
             }
         }
         *reinterpret_cast<vec *>(Y + i) = s;
@@ -420,11 +638,14 @@ unsigned grid_for(int64_t blocks) { return (unsigned)std::max<int64_t>(1, std::m
 }  // namespace
 
 hipError_t launch_sum_slices(const float *part, int slices, const RdProblem &p, hipStream_t s) {
-#define DMC_SUM(Q)                                                                                            \
-    hipLaunchKernelGGL(gemm_sum_slices_kernel<Q>, dim3(grid_for((p.m * p.n / Q + 255) / 256)), dim3(256), 0, s, part, \
-                       slices, p.y, p.w, p.x, (int)p.m, (int)p.n, (int)p.k)
-    if (p.n % 4 == 0) DMC_SUM(4);
-    else DMC_SUM(1);
+    const bool packed = p.k % 64 == 0 && aligned(p.w, 16) && aligned(p.x, 16);
+#define DMC_SUM(Q, PK)                                                                                         \
+    hipLaunchKernelGGL((gemm_sum_slices_kernel<Q, PK>), dim3(grid_for((p.m * p.n / Q + 255) / 256)), dim3(256), 0, s, \
+                       part, slices, p.y, p.w, p.x, (int)p.m, (int)p.n, (int)p.k, (int64_t)1, (int64_t)0, (int64_t)0)
+    if (p.n % 4 == 0 && packed) DMC_SUM(4, true);
+    else if (p.n % 4 == 0) DMC_SUM(4, false);
+    else if (packed) DMC_SUM(1, true);
+    else DMC_SUM(1, false);
 #undef DMC_SUM
     return hipGetLastError();
 }
@@ -435,8 +656,12 @@ hipError_t launch_gemm(const RdProblem &p, const RdPlan &pl, void *workspace, hi
     // none and may be given none.
     const bool needs_ws = !pl.xfuse || pl.kslices > 1;
     const int mt = pl.mt * pl.mtiles;
+    const bool packed = pl.vec == 8 && p.k % 64 == 0;
     if ((needs_ws && !workspace) || pl.kslices < 1 || pl.kslices > 65535 ||
-        (int64_t)pl.kslices * pl.kchunks < p.k / 64 || pl.rpw != 32 * pl.waves || pl.grid_x * pl.rpw < p.n)
+        (int64_t)pl.kslices * pl.kchunks < (p.k + 63) / 64 || pl.rpw != 32 * pl.waves || pl.grid_x * pl.rpw < p.n ||
+        p.ldw != p.k || p.ldx != p.k || p.ldy != p.n || p.k < 1 || (int64_t)pl.rpw * p.k * 2 + 16 > INT32_MAX ||
+        (packed ? !aligned(p.w, 16) || !aligned(p.x, 16)
+                : !pl.xfuse || pl.waves != 8 || p.m * p.k * 4 > INT32_MAX || !aligned(p.w, 2) || !aligned(p.x, 4)))
         return hipErrorInvalidValue;
     uint16_t *xs = pl.xfuse ? nullptr : static_cast<uint16_t *>(workspace);
     const size_t planes = pl.xfuse ? 0 : ((size_t)3 * p.m * p.k * 2 + 255) / 256 * 256;
@@ -452,15 +677,17 @@ hipError_t launch_gemm(const RdProblem &p, const RdPlan &pl, void *workspace, hi
     // blocks (DMC_HIP_GEMM_XCD: 0 never, 2 always).
     const int xenv = env_int("DMC_HIP_GEMM_XCD", 1);
     const int xcd = xenv == 2 || (xenv == 1 && gy > 1) ? 1 : 0;
-#define DMC_GEMM(NW, MT, F)                                                                                   \
-    if (pl.waves == NW && mt == MT && pl.xfuse == F)                                                          \
-        hipLaunchKernelGGL((gemv_rd_mfma_gemm_kernel<NW, MT, F>), dim3((unsigned)wgs), dim3(64 * NW), 0, s, p.w, \
+#define DMC_GEMM(NW, MT, SRC, F)                                                                              \
+    if (pl.waves == NW && mt == MT && packed == (SRC == kSrcPacked) && pl.xfuse == F)                            \
+        hipLaunchKernelGGL((gemv_mfma_gemm_kernel<NW, MT, SRC, F>), dim3((unsigned)wgs), dim3(64 * NW), 0, s, p.w, \
                            p.x, xs, p.y, part, (int)p.n, (int)p.k, (int)p.m, pl.kchunks, (int)pl.grid_x, (int)gy, \
-                           xcd);                                                                              \
+                           xcd, (int64_t)0, (int64_t)0);                                                      \
     else
-    DMC_GEMM(8, 16, true) DMC_GEMM(8, 16, false) DMC_GEMM(8, 32, true) DMC_GEMM(8, 32, false)
-    DMC_GEMM(8, 64, true) DMC_GEMM(8, 64, false) DMC_GEMM(8, 128, true) DMC_GEMM(8, 128, false)
-    DMC_GEMM(4, 32, true) DMC_GEMM(4, 32, false) DMC_GEMM(4, 64, true) DMC_GEMM(4, 64, false)
+    DMC_GEMM(8, 16, kSrcPacked, true) DMC_GEMM(8, 16, kSrcPacked, false) DMC_GEMM(8, 32, kSrcPacked, true)
+    DMC_GEMM(8, 32, kSrcPacked, false) DMC_GEMM(8, 64, kSrcPacked, true) DMC_GEMM(8, 64, kSrcPacked, false)
+    DMC_GEMM(8, 128, kSrcPacked, true) DMC_GEMM(8, 128, kSrcPacked, false) DMC_GEMM(4, 32, kSrcPacked, true)
+    DMC_GEMM(4, 32, kSrcPacked, false) DMC_GEMM(4, 64, kSrcPacked, true) DMC_GEMM(4, 64, kSrcPacked, false)
+    DMC_GEMM(8, 16, kSrcRows, true) DMC_GEMM(8, 32, kSrcRows, true) DMC_GEMM(8, 64, kSrcRows, true)
     return hipErrorInvalidValue;
 #undef DMC_GEMM
     if (pl.kslices > 1) return launch_sum_slices(part, pl.kslices, p, s);

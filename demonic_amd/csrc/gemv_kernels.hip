@@ -2663,6 +2663,34 @@ static bool plan_unaligned(const RdProblem &p, int vec, int64_t cus, RdPlan &sp)
     return true;
 }
 
+// The gemm layout's split of k over workgroups of `pair` activation tiles of
+// pl.mt rows (pl.waves, pl.rpw set), whether they split x themselves, and the
+// time that gives in us.  (Why: at the callers.)
+static double gemm_split(int64_t m, int64_t n, int64_t k, int64_t cus, int pair, int wg_per_cu, RdPlan &pl) {
+    const int64_t nchunks = (k + 63) / 64;
+    const int64_t per_cu = std::max(1, env_int("DMC_HIP_GEMM_PER_CU", wg_per_cu));
+    const int64_t gx = (n + pl.rpw - 1) / pl.rpw, wgm = (int64_t)pl.mt * pair;
+    const int64_t tiles = gx * ((m + wgm - 1) / wgm);
+    int64_t want = std::max<int64_t>(1, per_cu * cus / tiles);
+    if (tiles < cus && tiles * want * 10 < cus * 7) want = std::max<int64_t>(1, 2 * per_cu * cus / tiles);
+    // A slice of fewer than 8 chunks pays its pipeline fill and output too
+    // often: halve the split (C2 down at m = 12 / 16 on 16-row tiles: 35.0 /
+    // 37.2 us on 16 slices of 14 chunks against 37.3 / 40.4 on 32 of 7).
+    const int64_t min_chunks = std::max(1, env_int("DMC_HIP_GEMM_MIN_CHUNKS", 8));
+    while (want > 1 && (nchunks + want - 1) / want < min_chunks) want = (want + 1) / 2;
+    want = std::min<int64_t>({want, nchunks, (int64_t)env_int("DMC_HIP_GEMM_MAX_SLICES", 64)});
+    want = std::max<int64_t>(want, 1);
+    pl.mtiles = pair;
+    pl.kchunks = (int)((nchunks + want - 1) / want);
+    pl.kslices = (int)((nchunks + pl.kchunks - 1) / pl.kchunks);
+    const int fenv = env_int("DMC_HIP_GEMM_FUSE", 1);  // 0: never; 2: always
+    pl.xfuse = fenv == 2 || (fenv == 1 && (pl.mt == 16 || gx * m <= (pair == 2 ? 65536 : 8192)));
+    const int64_t rounds = (tiles * pl.kslices + per_cu * cus - 1) / (per_cu * cus);
+    const double chunk = pair == 2 ? 2.65 : pl.xfuse ? 1.55 : 1.75;
+    return (double)rounds * pl.kchunks * chunk + 4 +
+           (pl.kslices > 1 ? 5 + 0.42e-6 * ((double)pl.kslices * m * n * 4) : 0);
+}
+
 RdPlan plan_rd(const RdProblem &p, int num_cus) {
     RdPlan pl{};
     // Widest load the row alignment allows: every row start, every activation
@@ -2877,34 +2905,6 @@ RdPlan plan_rd(const RdProblem &p, int num_cus) {
             // m = 256: 124 / 125 against 140 / 135), except up at m = 192,
             // whose 168 tiles leave a third of the CUs idle (112 us on three
             // slices against 124 on one).
-            const int64_t nchunks = p.k / 64;
-            const int64_t per_cu =
-                std::max(1, env_int("DMC_HIP_GEMM_PER_CU", mp.mt == 16 || mp.waves == 4 ? 2 : 1));
-            const int64_t gx = (p.n + mp.rpw - 1) / mp.rpw;
-            const int fenv = env_int("DMC_HIP_GEMM_FUSE", 1);  // 0: never; 2: always
-            // The split for workgroups of `pair` activation tiles, and its time in us.
-            auto split = [&](int pair, RdPlan &o) {
-                const int64_t wgm = (int64_t)mp.mt * pair;
-                const int64_t tiles = gx * ((p.m + wgm - 1) / wgm);
-                int64_t want = std::max<int64_t>(1, per_cu * cus / tiles);
-                if (tiles < cus && tiles * want * 10 < cus * 7) want = std::max<int64_t>(1, 2 * per_cu * cus / tiles);
-                // A slice of fewer than 8 chunks pays its pipeline fill and output
-                // too often: halve the split (C2 down at m = 12 / 16 on 16-row
-                // tiles: 35.0 / 37.2 us on 16 slices of 14 chunks against 37.3 /
-                // 40.4 on 32 of 7).
-                const int64_t min_chunks = std::max(1, env_int("DMC_HIP_GEMM_MIN_CHUNKS", 8));
-                while (want > 1 && (nchunks + want - 1) / want < min_chunks) want = (want + 1) / 2;
-                want = std::min<int64_t>({want, nchunks, (int64_t)env_int("DMC_HIP_GEMM_MAX_SLICES", 64)});
-                want = std::max<int64_t>(want, 1);
-                o.mtiles = pair;
-                o.kchunks = (int)((nchunks + want - 1) / want);
-                o.kslices = (int)((nchunks + o.kchunks - 1) / o.kchunks);
-                o.xfuse = fenv == 2 || (fenv == 1 && (mp.mt == 16 || gx * p.m <= (pair == 2 ? 65536 : 8192)));
-                const int64_t rounds = (tiles * o.kslices + per_cu * cus - 1) / (per_cu * cus);
-                const double chunk = pair == 2 ? 2.65 : o.xfuse ? 1.55 : 1.75;
-                return (double)rounds * o.kchunks * chunk + 4 +
-                       (o.kslices > 1 ? 5 + 0.42e-6 * ((double)o.kslices * p.m * p.n * 4) : 0);
-            };
             // 64-row tiles: one or two per workgroup (two take 2.65 us per 64-k
             // chunk against 1.55, 1.75 with x's planes, but split k further
             // where they leave CUs idle), whichever the sum of rounds x chunks
@@ -2919,8 +2919,9 @@ RdPlan plan_rd(const RdProblem &p, int num_cus) {
             const int penv = env_int("DMC_HIP_GEMM_PAIR", 0);
             const bool can_pair = mp.mt == 64 && mp.waves == 8 && (p.m > 64 || penv == 2) && penv != 1;
             RdPlan one = mp, two = mp;
-            const double t1 = split(1, one);
-            mp = can_pair && (split(2, two) < t1 || penv == 2) ? two : one;
+            const int wg_per_cu = mp.mt == 16 || mp.waves == 4 ? 2 : 1;
+            const double t1 = gemm_split(p.m, p.n, p.k, cus, 1, wg_per_cu, one);
+            mp = can_pair && (gemm_split(p.m, p.n, p.k, cus, 2, wg_per_cu, two) < t1 || penv == 2) ? two : one;
             // Workgroups split their own chunks of x (no planes, no split
             // launch) at 16-row tiles (C2 down at m = 16: the split launch cost
             // 3-4 us of 37), and at 32 and 64 while the repeated split stays
@@ -3008,6 +3009,39 @@ RdPlan plan_rd(const RdProblem &p, int num_cus) {
         mp.grid_x = (p.n + mp.rpw - 1) / mp.rpw;
         mp.grid_y = (p.m + mp.mt - 1) / mp.mt;
         return mp;
+    }
+
+    // Rows of any other length or alignment: the gemm layout's general form
+    // (x split in the kernel, 16, 32 or 64 activation rows per workgroup, one
+    // workgroup per CU).  It streams W once per 64 rows where the general
+    // kernel does once per 8 with loads of the rows' alignment (the streaming
+    // kernel, K a multiple of 8, once per 4).  Same box, these / here, us:
+    // [11008,4097] m = 2 / 3 / 5 / 16 / 33 / 300 49.5 / 52 / 103 / 180 / 500 /
+    // 3115 against 25.0 / 25.0 / 25.1 / 26.2 / 37.3 / 122; [11008,4104] m = 4
+    // 39.2 / 23.8; [4096,4104] m = 16 / 33 51.9 / 113 against 16.6 / 25.6.
+    // Small products stay, where the fixed cost (~13 us with the slice pass)
+    // decides: K odd, up to 2^25 multiply-adds ([2001,1001] m = 16 12.7
+    // against 14.7; [4000,2052] m = 5, above, 19.4 / 14.3); K a multiple of 8,
+    // up to 2^26 ([11008,1000] m = 3 8.1 against 13.4, [1000,4104] m = 16 19.0
+    // / 18.3), and two rows ([11008,4104] 22.1 / 24).
+    const int rows_env = env_int("DMC_HIP_RD_GEMM_ROWS", 1);  // 0: never; 2: wherever it applies
+    if (rows_env != 0 && mfma_min_m > 0 && p.k >= 1 && p.ldw == p.k && p.ldx == p.k && p.ldy == p.n &&
+        (int64_t)kWideRows * p.k * 2 + 16 <= INT32_MAX && p.m * p.k * 4 <= INT32_MAX &&
+        (rows_env == 2 || (p.m >= (pl.vec == 8 ? 3 : 2) && p.m * p.n * p.k > (int64_t)1 << (pl.vec == 8 ? 26 : 25)))) {
+        RdPlan mp{};
+        mp.mfma = true;
+        mp.mkind = 8;
+        mp.vec = p.k % 64 == 0 && pl.vec == 8 ? 4 : pl.vec;  // 8 and K % 64 == 0 means packed rows
+        mp.rows = 16;
+        mp.mt = p.m <= 16 ? 16 : p.m <= 32 ? 32 : 64;
+        mp.waves = 8;
+        mp.rpw = 256;
+        gemm_split(p.m, p.n, p.k, cus, 1, 1, mp);
+        mp.xfuse = true;
+        mp.workspace_bytes = mp.kslices > 1 ? (size_t)mp.kslices * p.m * p.n * 4 : 0;
+        mp.grid_x = (p.n + mp.rpw - 1) / mp.rpw;
+        mp.grid_y = (p.m + mp.mt - 1) / mp.mt;
+        if (mp.grid_x * mp.grid_y * mp.kslices <= INT32_MAX) return mp;
     }
 
     // Streaming kernel: packed 128-bit rows and k within the register budget.

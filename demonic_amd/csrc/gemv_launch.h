@@ -132,8 +132,8 @@ CsPlan plan_cs(const CsProblem &p, int num_cus);
 // when plan.slices > 1).  Returns hipSuccess or the launch error.
 hipError_t launch_rd(const RdProblem &p, const RdPlan &plan, void *workspace, hipStream_t stream);
 hipError_t launch_rd_group(const RdGroup &g, const RdPlan &plan, hipStream_t stream);
-// The gemm layout (plan.mkind == 8), and the sum of k-slice partials
-// part[slice][m][n] into p.y in slice order with the zero rule.
+// The gemm layout (plan.mkind == 8), and the sum of
+// k-slice partials part[slice][m][n] into p.y in slice order with the zero rule.
 hipError_t launch_gemm(const RdProblem &p, const RdPlan &plan, void *workspace, hipStream_t stream);
 hipError_t launch_sum_slices(const float *part, int slices, const RdProblem &p, hipStream_t stream);
 

@@ -234,7 +234,8 @@ int32_t dmc_hip_gemv_rd_grouped(int64_t count, const int64_t *x_devs, const int6
  * windows per lane (with vec < 8, the variant that reads misaligned rows with
  * unaligned 128-bit loads), 0 the general kernel, -6 / -7 / -8 the MFMA layouts
  * (wide: 256 rows per workgroup; rows16: 16 rows per block; gemm: 256 rows
- * against 16, 32 or 64 activation rows, k possibly split; mt activation rows);
+ * against 16, 32 or 64 activation rows, k possibly split; with vec < 8, or K no
+ * multiple of 64, over rows of any length and alignment; mt activation rows);
  * waves and rows_per_group (weight rows per workgroup) describe the workgroup.
  * Column-stream layout: `vec` is the row alignment as above; rows_or_rw <= 0 is
  * the streaming kernel (512 columns per workgroup, or with -G row groups per

@@ -51,3 +51,35 @@ def test_a_lone_cancelling_output_takes_the_chain(hip, slices, monkeypatch):
     check(y, y_ref, what="lone zero")
     for r in (0, 70, 79):
         check_bound(y[r], y_ref[r], x[r], W.bf16_to_f32(w), what=f"lone zero row {r}")
+
+
+def planted(m, k, n, seed):
+    """Edge data, with special values, zero rows and underflow where they fit; (x, w [n,k], reference)."""
+    x, w = case(m, k, n, seed=seed, edge=True)
+    if k > 2 and n > 4 and m > 3:
+        x[0, k - 1], w[1, k - 1], w[n - 1, k - 1] = np.inf, 0x7F80, 0x3F80  # in the last chunk and the last element
+        x[1, 0], w[1, 0] = np.float32(1e-45), 0xFF80
+        w[2, :], x[2, :] = 0, 0
+        x[3, :], w[3, :] = np.float32(-1e-38), 0x0001
+    return x, w, oracle.matmul_bf16_t(x, w)
+
+
+@pytest.mark.parametrize("offset", [0, 2])
+@pytest.mark.parametrize("m,k,n", [(5, 65, 257), (16, 4097, 300), (17, 1003, 256), (33, 4104, 255), (64, 63, 513),
+                                   (65, 130, 1030), (200, 2050, 259), (7, 1, 6), (6, 8191, 130)])
+def test_rows_of_any_length_and_alignment(hip, m, k, n, offset, monkeypatch):
+    """The gemm layout on rows whose length is no multiple of 64, W at the end
+    of its region and 0 or 2 bytes into it: nothing past K takes part (the next
+    row starts with what it likes, the last row ends the region)."""
+    monkeypatch.setenv("DMC_HIP_RD_GEMM_ROWS", "2")
+    x, w, y_ref = planted(m, k, n, seed=m + k + n)
+    buf = np.zeros(w.size + offset // 2, np.uint16)
+    buf[offset // 2:] = w.reshape(-1)
+    with hip.DeviceBuffer.from_numpy(buf) as dw, hip.DeviceBuffer.from_numpy(x) as dx, \
+            hip.DeviceBuffer(4 * m * n) as dy:
+        p = hip.plan("rd", m, k, n, x_addr=dx.addr, w_addr=dw.addr + offset)
+        assert (p.slices, p.mt, p.rows_per_group) == (-8, 16 if m <= 16 else 32 if m <= 32 else 64, 256), p
+        hip.gemv_rd(dx, dw.addr + offset, dy, m, k, n)
+        hip.synchronize()
+        y = dy.download(np.float32, (m, n))
+    check_or_bound(y, y_ref, x, W.bf16_to_f32(w), f"gemm rows {m}x{k}x{n}+{offset}")
