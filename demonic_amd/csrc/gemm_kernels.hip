@@ -694,4 +694,34 @@ hipError_t launch_gemm(const RdProblem &p, const RdPlan &pl, void *workspace, hi
     return hipGetLastError();
 }
 
+hipError_t launch_gemm_cs(const CsProblem &p, const CsPlan &pl, void *workspace, hipStream_t s) {
+    const int64_t nchunks = (p.k + 63) / 64;
+    const int64_t kc = pl.kslice / 64;
+    if (p.k < 1 || pl.cb != 256 || pl.waves != 8 || pl.kslice % 64 != 0 || kc < 1 || pl.slices < 1 ||
+        pl.slices * kc < nchunks || (pl.slices > 1 && !workspace) || pl.grid_x * 256 < p.n || p.batch > 65535 ||
+        (p.k + 64) * p.n * 2 > INT32_MAX || p.m * p.k * 4 > INT32_MAX || !aligned(p.w, 2) || !aligned(p.x, 4))
+        return hipErrorInvalidValue;
+    float *const part = pl.slices > 1 ? static_cast<float *>(workspace) : nullptr;
+    const int64_t gy = (p.m + pl.mt - 1) / pl.mt;
+    const int64_t wgs = pl.grid_x * gy * pl.slices;
+    if (wgs > INT32_MAX) return hipErrorInvalidValue;
+    const dim3 grid((unsigned)wgs, (unsigned)p.batch);
+#define DMC_GEMM_CS(MT)                                                                                        \
+    hipLaunchKernelGGL((gemv_mfma_gemm_kernel<8, MT, kSrcCols, true>), grid, dim3(512), 0, s, p.w, p.x,            \
+                       (const uint16_t *)nullptr, p.y, part, (int)p.n, (int)p.k, (int)p.m, (int)kc, (int)pl.grid_x, \
+                       (int)gy, gy > 1 ? 1 : 0, p.rs, p.ls)
+    if (pl.mt == 32) DMC_GEMM_CS(32);
+    else if (pl.mt == 64) DMC_GEMM_CS(64);
+    else return hipErrorInvalidValue;
+#undef DMC_GEMM_CS
+    if (pl.slices <= 1) return hipGetLastError();
+#define DMC_SUM_CS(Q)                                                                                          \
+    hipLaunchKernelGGL((gemm_sum_slices_kernel<Q, false>), dim3(grid_for((p.m * p.n / Q + 255) / 256), (unsigned)p.batch), \
+                       dim3(256), 0, s, part, (int)pl.slices, p.y, p.w, p.x, (int)p.m, (int)p.n, (int)p.k, p.n, p.rs, p.ls)
+    if (p.n % 4 == 0) DMC_SUM_CS(4);
+    else DMC_SUM_CS(1);
+#undef DMC_SUM_CS
+    return hipGetLastError();
+}
+
 }  // namespace dmc

@@ -3130,7 +3130,7 @@ RdPlan plan_rd_group(const RdGroup &g, int num_cus) {
     return pl;
 }
 
-CsPlan plan_cs(const CsProblem &p, int num_cus) {
+static CsPlan plan_cs_fma(const CsProblem &p, int num_cus) {
     CsPlan pl{};
     for (int v : {8, 4, 2, 1}) {
         if (p.n % v == 0 && (p.batch <= 1 || p.rs % v == 0) && aligned(p.w, 2 * v)) {
@@ -3230,6 +3230,46 @@ CsPlan plan_cs(const CsProblem &p, int num_cus) {
         pl.slices = (kmax + pl.kslice - 1) / pl.kslice;
     }
     pl.workspace_bytes = pl.slices > 1 ? (size_t)pl.slices * batch * p.m * p.n * 4 : 0;
+    return pl;
+}
+
+CsPlan plan_cs(const CsProblem &p, int num_cus) {
+    const CsPlan fma = plan_cs_fma(p, num_cus);
+    // From 17 activation rows: the gemm layout over columns (the FMA kernels
+    // stream W once per 4 rows).  Same box, these / here, us: C2 up m = 17 / 33
+    // / 64 170 / 485 / 3675 against 33 / 42 / 46, down m = 64 3742 / 42; odd N,
+    // [11007,4097] m = 32 414 / 38; the smallest, [512,512] m = 17 / 64 31 / 96
+    // against 14 / 18; per-head batches, W [32,4096,128] m = 17 182 / 21.5.
+    const int env = env_int("DMC_HIP_CS_GEMM", 1);  // 0: never; 2: wherever it applies
+    const int64_t cus = num_cus > 0 ? num_cus : 256, batch = std::max<int64_t>(p.batch, 1);
+    if (env == 0 || p.m < (env == 2 ? 1 : 17) || p.k < 1 || batch > 65535 ||
+        (p.k + 64) * p.n * 2 > INT32_MAX || p.m * p.k * 4 > INT32_MAX)
+        return fma;
+    RdPlan g{};
+    g.mt = p.m <= 32 ? 32 : 64;
+    g.waves = 8;
+    g.rpw = 256;
+    gemm_split(p.m, p.n, p.k, std::max<int64_t>(1, cus / batch), 1, 1, g);
+    // The partial sums stay within the fixed scratch of the no-allocation
+    // entry, whose limit is judged by the FMA plan (workspace_bytes).
+    const int64_t out = batch * p.m * p.n * 4;
+    while (g.kslices > 1 && g.kslices * out > (int64_t)noalloc_scratch_bytes()) {
+        const int64_t nchunks = (p.k + 63) / 64, s = g.kslices - 1;
+        g.kchunks = (int)((nchunks + s - 1) / s);
+        g.kslices = (int)((nchunks + g.kchunks - 1) / g.kchunks);
+    }
+    CsPlan pl = fma;
+    pl.gemm = true;
+    pl.stream = pl.unaligned = false;
+    pl.rw = -256;
+    pl.mt = g.mt;
+    pl.cb = 256;
+    pl.waves = 8;
+    pl.kslice = (int64_t)g.kchunks * 64;
+    pl.slices = g.kslices;
+    pl.grid_x = (p.n + 255) / 256;
+    pl.workspace_bytes = std::max<size_t>(fma.workspace_bytes, pl.slices > 1 ? (size_t)pl.slices * out : 0);
+    if (pl.grid_x * ((p.m + pl.mt - 1) / pl.mt) * pl.slices > INT32_MAX) return fma;
     return pl;
 }
 
@@ -3400,6 +3440,7 @@ hipError_t launch_rd(const RdProblem &p, const RdPlan &pl, void *workspace, hipS
 
 hipError_t launch_cs(const CsProblem &p, const CsPlan &pl, void *workspace, hipStream_t s) {
     if (p.m <= 0 || p.n <= 0 || p.batch <= 0) return hipSuccess;
+    if (pl.gemm) return launch_gemm_cs(p, pl, workspace, s);
     const int64_t zmax_s = 32768;  // grid.z limit, with margin
     if (pl.stream) {
         float *P = pl.slices > 1 || pl.unaligned ? static_cast<float *>(workspace) : nullptr;

@@ -100,6 +100,7 @@ struct CsPlan {
     int cb;         // output columns per workgroup
     int waves;      // waves per workgroup
     bool stream;    // streaming kernel
+    bool gemm = false;  // the gemm layout over columns: cb = 256, kslice a multiple of 64
     bool unaligned; // streaming over rows at any 2-byte alignment (the last k row in the slice pass)
     int64_t kslice; // k rows per workgroup (split-K)
     int64_t slices; // number of k slices (1 = no reduction across workgroups)
@@ -132,9 +133,10 @@ CsPlan plan_cs(const CsProblem &p, int num_cus);
 // when plan.slices > 1).  Returns hipSuccess or the launch error.
 hipError_t launch_rd(const RdProblem &p, const RdPlan &plan, void *workspace, hipStream_t stream);
 hipError_t launch_rd_group(const RdGroup &g, const RdPlan &plan, hipStream_t stream);
-// The gemm layout (plan.mkind == 8), and the sum of
+// The gemm layout (plan.mkind == 8; over columns: CsPlan::gemm), and the sum of
 // k-slice partials part[slice][m][n] into p.y in slice order with the zero rule.
 hipError_t launch_gemm(const RdProblem &p, const RdPlan &plan, void *workspace, hipStream_t stream);
+hipError_t launch_gemm_cs(const CsProblem &p, const CsPlan &plan, void *workspace, hipStream_t stream);
 hipError_t launch_sum_slices(const float *part, int slices, const RdProblem &p, hipStream_t stream);
 
 hipError_t launch_cs(const CsProblem &p, const CsPlan &plan, void *workspace, hipStream_t stream);

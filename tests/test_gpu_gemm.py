@@ -83,3 +83,27 @@ def test_rows_of_any_length_and_alignment(hip, m, k, n, offset, monkeypatch):
         hip.synchronize()
         y = dy.download(np.float32, (m, n))
     check_or_bound(y, y_ref, x, W.bf16_to_f32(w), f"gemm rows {m}x{k}x{n}+{offset}")
+
+
+@pytest.mark.parametrize("offset", [0, 2])
+@pytest.mark.parametrize("m,k,n,batch", [(17, 65, 257, 1), (33, 4097, 300, 1), (64, 63, 255, 1), (65, 1000, 513, 1),
+                                         (20, 128, 64, 3), (40, 70, 131, 2), (18, 1, 9, 1), (130, 2048, 1024, 1)])
+def test_columns_on_the_gemm_layout(hip, m, k, n, batch, offset, monkeypatch):
+    """W [k,n] per batch slice on the gemm layout: partial column blocks, odd N
+    (the last element shares a dword with what follows the matrix), K tails,
+    several slices of k and of the batch, W 0 or 2 bytes into its region."""
+    monkeypatch.setenv("DMC_HIP_CS_GEMM", "2")
+    zs = [planted(m, k, n, seed=m + k + n + z) for z in range(batch)]
+    x = np.stack([z[0] for z in zs])
+    wt = np.stack([np.ascontiguousarray(z[1].T) for z in zs])
+    buf = np.zeros(wt.size + offset // 2, np.uint16)
+    buf[offset // 2:] = wt.reshape(-1)
+    with hip.DeviceBuffer.from_numpy(buf) as dw, hip.DeviceBuffer.from_numpy(x) as dx, \
+            hip.DeviceBuffer(4 * batch * m * n) as dy:
+        p = hip.plan("cs", m, k, n, batch=batch, rs=k * n, x_addr=dx.addr, w_addr=dw.addr + offset)
+        assert p.rows_or_rw == -256, p
+        hip.gemv_cs(dx, dw.addr + offset, dy, m, k, n, batch, m * k, k * n)
+        hip.synchronize()
+        y = dy.download(np.float32, (batch, m, n))
+    for z, (xz, wz, y_ref) in enumerate(zs):
+        check_or_bound(y[z], y_ref, xz, W.bf16_to_f32(wz), f"gemm cols {m}x{k}x{n} slice {z}")
