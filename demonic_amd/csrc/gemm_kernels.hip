@@ -338,7 +338,7 @@ gemv_mfma_gemm_kernel(const uint16_t *__restrict__ W, const float *__restrict__ 
     // Chunk c is in LDS buffer BUF and its first step's operands in registers;
     // chunk c + 1 is in `r`, loaded a chunk ago.
     Regs r;
-    auto chunk = [&](int c, auto BUF, auto TERMS) __attribute__((always_inline)) {
+    auto chunk = [&](int c, auto BUF, auto TERMS, auto AT) __attribute__((always_inline)) {
         constexpr int buf = decltype(BUF)::value;
 #pragma unroll
         for (int s = 0; s < NS; ++s) {
@@ -347,7 +347,7 @@ gemv_mfma_gemm_kernel(const uint16_t *__restrict__ W, const float *__restrict__ 
                 if ((s + 1) % RM == 0) read_a(buf, (s + 1) / RM);
                 read_x(buf, (s + 1) / RM, (s + 1) % RM, (s + 1) & 1);
             }
-            if (s == NS - 2) {
+            if (s == decltype(AT)::value) {
                 store(r, c + 1, buf ^ 1, TERMS);
                 load(c + 2, r);
             }
@@ -393,7 +393,7 @@ gemv_mfma_gemm_kernel(const uint16_t *__restrict__ W, const float *__restrict__ 
                     part[i][j][v] = 0.0f;
                 }
     };
-    auto stream = [&](auto TERMS) __attribute__((always_inline)) {
+    auto stream = [&](auto TERMS, auto AT) __attribute__((always_inline)) {
 #pragma unroll
         for (int i = 0; i < RM; ++i)
 #pragma unroll
@@ -414,8 +414,8 @@ gemv_mfma_gemm_kernel(const uint16_t *__restrict__ W, const float *__restrict__ 
         int c = 0;
         int until = fold;
         for (; c + 1 < nch; c += 2) {
-            chunk(c, std::integral_constant<int, 0>{}, TERMS);
-            chunk(c + 1, std::integral_constant<int, 1>{}, TERMS);
+            chunk(c, std::integral_constant<int, 0>{}, TERMS, AT);
+            chunk(c + 1, std::integral_constant<int, 1>{}, TERMS, AT);
             if constexpr (kTwoLevel) {
                 if (c + 2 >= until) {
                     fold_parts();
@@ -423,7 +423,7 @@ gemv_mfma_gemm_kernel(const uint16_t *__restrict__ W, const float *__restrict__ 
                 }
             }
         }
-        if (c < nch) chunk(c, std::integral_constant<int, 0>{}, TERMS);
+        if (c < nch) chunk(c, std::integral_constant<int, 0>{}, TERMS, AT);
         if constexpr (kTwoLevel) {
             fold_parts();
 #pragma unroll
@@ -434,7 +434,14 @@ gemv_mfma_gemm_kernel(const uint16_t *__restrict__ W, const float *__restrict__ 
                     for (int v = 0; v < 4; ++v) acc[i][j][v] = add_lost(total[i][j][v], lost[i][j][v]);
         }
     };
-    stream(std::integral_constant<int, 3>{});
+    // Waves w and w + 4 share a SIMD: they stage (split or transpose, store) in
+    // different steps, so that one's vector work runs under the other's MFMAs.
+    // Same box, in the same step / staggered, us: C2 up m = 512 168 / 164, down
+    // m = 2048 604 / 581, columns up m = 64 47.5 / 44.0; packed 64-row tiles
+    // lose 2% where a slice has few chunks (C2 up m = 64 40.2 / 40.7).
+    constexpr bool kStagger = MT == 128 || (SRC == kSrcCols && MT == 64);
+    if (!kStagger || wave >= 4) stream(std::integral_constant<int, 3>{}, std::integral_constant<int, NS - 2>{});
+    else stream(std::integral_constant<int, 3>{}, std::integral_constant<int, 0>{});
 
     // The activation rows' largest magnitudes (this slice's k), in LDS bytes
     // that the stream is done with.
@@ -523,7 +530,7 @@ gemv_mfma_gemm_kernel(const uint16_t *__restrict__ W, const float *__restrict__ 
     const bool again = *any_s != 0;
     __syncthreads();
     if (!again) return;
-    stream(std::integral_constant<int, 1>{});
+    stream(std::integral_constant<int, 1>{}, std::integral_constant<int, NS - 2>{});
 #pragma unroll
     for (int mf = 0; mf < RM; ++mf) {
         const int ml = (wm * RM + mf) * 16 + i16;
