@@ -508,7 +508,7 @@ gemv_mfma_gemm_kernel(const uint16_t *__restrict__ W, const float *__restrict__ 
                 const uint16_t *const wu = readlane_ptr(wr, __builtin_ctzll(who));
                 const bool nz = SRC == kSrcPacked ? wave_row_nonzero(wu, K / 8, 0x7fff7fffu)
                                                : wave_weights_nonzero(wu, wstep, K);
-                const float v = wave_chains(ask && nz, 0.0f, wr, wstep, xr, K);
+                const float v = wave_chains<MT == 16 ? 2 : 4>(ask && nz, 0.0f, wr, wstep, xr, K);
                 if (ask) *o = v;
             }
         }
@@ -633,7 +633,7 @@ gemm_sum_slices_kernel(const float *__restrict__ P, int slices, float *__restric
                     const bool nz = PACKED ? wave_row_nonzero(wu, K / 8, 0x7fff7fffu) : wave_weights_nonzero(wu, wstep, K);
                     if ((int)(threadIdx.x & 63) == j) chain = nz;
                 }
-                s[e] = wave_chains(chain, z ? 0.0f : s[e], w, wstep, X + (int64_t)m * K, K);
+                s[e] = wave_chains<2>(chain, z ? 0.0f : s[e], w, wstep, X + (int64_t)m * K, K);
             }
         }
         *reinterpret_cast<vec *>(Y + i) = s;

@@ -157,7 +157,7 @@ __device__ bool wave_any_product(const float *x, const uint16_t *w, int64_t wste
 // ordinary data (full cancellation) is rare per output, ~3e-8, but a prefill
 // has millions of outputs: a few calls in a hundred at 1M, one in four at 8M.
 // Elements past K multiply +0 by -0: adding -0 keeps the accumulator.
-__device__ __attribute__((noinline)) float wave_chain(const uint16_t *w, int64_t wstep, const float *x, int K) {
+__device__ __forceinline__ float wave_chain(const uint16_t *w, int64_t wstep, const float *x, int K) {
     const int lane = threadIdx.x & 63;
     if (K <= 0) return 0.0f;
     const bool packed = wstep <= 1 && K <= (1 << 28);
@@ -209,13 +209,79 @@ __device__ __attribute__((noinline)) float wave_chain(const uint16_t *w, int64_t
     return acc;
 }
 
-// The chains of the lanes that ask for one (w, x per lane): a few one after
-// another by the whole wave, many one per lane.
+// Wave-uniform, for an output whose split sum is exactly zero: can the
+// reference chain end at -0?  A product x * w is a multiple of 2^(ex + ew - 284)
+// (biased exponents; 23 and 7 fraction bits).  Where that is at least 2^-149
+// for the least nonzero |x| and |w| of the two rows, every sum of the chain is
+// a multiple of the least subnormal, none underflows, and a chain that ends at
+// zero ends at +0 (an exact cancellation, or it never left +0).  So +0 is the
+// answer where the reference is zero, and where its roundings leave a residue,
+// +0 is as close to the exact sum as any other order's.  One pass over the
+// rows, against the chain's K dependent steps (4 us against 31 at K = 14336).
+template <int U>  // 512 * U elements a round: 12 registers each
+__device__ __forceinline__ bool wave_zero_is_plus(const uint16_t *w, int64_t wstep, const float *x, int K) {
+    const int lane = threadIdx.x & 63;
+    if (K <= 0) return true;
+    uint32_t xm = ~0u, wm = ((uint32_t)w[(int64_t)(K - 1) * wstep] & 0x7fffu) - 1u;  // least magnitude - 1: zeros on top
+    if (wstep <= 1 && K <= (1 << 28)) {
+        const uintptr_t wb = reinterpret_cast<uintptr_t>(w);
+        const uint32_t wd = (uint32_t)(wb & 3);
+        const __amdgpu_buffer_rsrc_t xr = weight_rsrc(x, (uint32_t)K * 4u);  // past K: zeros, which do not count
+        const __amdgpu_buffer_rsrc_t wr = weight_rsrc(reinterpret_cast<const void *>(wb - wd), wd + 2u * (uint32_t)K);
+        for (int k0 = 0; k0 < K; k0 += 512 * U) {
+            u32x4 xa[U], xc[U], wv[U];
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                const uint32_t e = (uint32_t)(k0 + (u * 64 + lane) * 8);
+                xa[u] = __builtin_amdgcn_raw_buffer_load_b128(xr, e * 4u, 0, 0);
+                xc[u] = __builtin_amdgcn_raw_buffer_load_b128(xr, e * 4u + 16u, 0, 0);
+                wv[u] = __builtin_amdgcn_raw_buffer_load_b128(wr, wd + e * 2u, 0, 0);
+            }
+#pragma unroll
+            for (int u = 0; u < U; ++u)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    xm = min(xm, min((xa[u][i] & 0x7fffffffu) - 1u, (xc[u][i] & 0x7fffffffu) - 1u));
+                    wm = min(wm, min((wv[u][i] & 0x7fffu) - 1u, (wv[u][i] >> 16 & 0x7fffu) - 1u));
+                }
+        }
+    } else {
+        for (int k0 = 0; k0 < K; k0 += 64 * U) {
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                const int k = min(k0 + u * 64 + lane, K - 1);
+                xm = min(xm, (__float_as_uint(x[k]) & 0x7fffffffu) - 1u);
+                wm = min(wm, ((uint32_t)w[(int64_t)k * wstep] & 0x7fffu) - 1u);
+            }
+        }
+    }
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) {
+        xm = min(xm, (uint32_t)__shfl_xor((int)xm, o));
+        wm = min(wm, (uint32_t)__shfl_xor((int)wm, o));
+    }
+    const uint32_t ex = (xm + 1) >> 23, ew = (wm + 1) >> 7;
+    return xm == ~0u || wm == ~0u || (ex >= 1 && ew >= 1 && ex + ew >= 135);
+}
+
+// The reference's values for the lanes whose sums are exactly zero (`ask`; w, x
+// per lane): +0 where it cannot be -0, else the chain, a few one after another
+// by the whole wave, many one per lane.  U = 0: the chain always (the FMA
+// kernels, whose outputs are few and whose registers are full).
+template <int U>
 __device__ __forceinline__ float wave_chains(bool ask, float s, const uint16_t *w, int64_t wstep, const float *x, int K) {
-    uint64_t todo = __builtin_amdgcn_ballot_w64(ask);
-    if (__builtin_popcountll(todo) > 6) return ask ? chain_strided(w, wstep, x, K) : s;
-    for (; todo; todo &= todo - 1) {
+    uint64_t chains = U > 0 ? 0 : __builtin_amdgcn_ballot_w64(ask);
+    if constexpr (U > 0) for (uint64_t todo = __builtin_amdgcn_ballot_w64(ask); todo; todo &= todo - 1) {
         const int j = __builtin_ctzll(todo);
+        if (wave_zero_is_plus<U>(readlane_ptr(w, j), wstep, readlane_ptr(x, j), K)) {
+            if ((int)(threadIdx.x & 63) == j) s = 0.0f;
+        } else {
+            chains |= 1ull << j;
+        }
+    }
+    if (__builtin_popcountll(chains) > 6) return (chains >> (threadIdx.x & 63)) & 1 ? chain_strided(w, wstep, x, K) : s;
+    for (; chains; chains &= chains - 1) {
+        const int j = __builtin_ctzll(chains);
         const float v = wave_chain(readlane_ptr(w, j), wstep, readlane_ptr(x, j), K);
         if ((int)(threadIdx.x & 63) == j) s = v;
     }
@@ -249,7 +315,7 @@ __device__ float settle_zero(float s, bool zero, const float *x, const uint16_t 
         const bool hit = wave_any_product(readlane_ptr(x, j), readlane_ptr(w, j), wstep, K);
         if (lane == j) chain = hit;
     }
-    return wave_chains(chain, zero ? 0.0f : s, w, wstep, x, K);
+    return wave_chains<0>(chain, zero ? 0.0f : s, w, wstep, x, K);
 }
 
 // ---- RD skinny M on MFMA: W [N,K] x X [M,K], K % 64 == 0 ---------------------------
@@ -473,7 +539,7 @@ __device__ void settle_zeros(f32x4 (&s)[T], const bool (&live)[T][4], const int 
     for (int t = 0; t < T; ++t)
 #pragma unroll
         for (int r = 0; r < 4; ++r)
-            s[t][r] = wave_chains(chain[t][r], s[t][r], W + (int64_t)(base[t] + 4 * g + r) * K, 1, X + (int64_t)m * K, K);
+            s[t][r] = wave_chains<2>(chain[t][r], s[t][r], W + (int64_t)(base[t] + 4 * g + r) * K, 1, X + (int64_t)m * K, K);
 }
 
 // Weight and x tiles in LDS hold rows of 128 bytes, 8 pieces of 16, back to
