@@ -623,6 +623,7 @@ gemv_rd_stream_xlds_kernel(const uint16_t *__restrict__ W, const float *__restri
 constexpr int kX14Waves = 14;
 constexpr int kX14MaxK = 2 * kX14Waves * 512;  // 14336: KV <= 2 (bf16), 4 (f32)
 constexpr int kX14MaxM = 4;
+constexpr int kGroupMaxMF32 = 8;  // f32 weights, at most two windows per lane (x: 64 registers)
 
 __device__ float chain_f32(const float *__restrict__ w, const float *__restrict__ x, int K);
 
@@ -640,7 +641,7 @@ __device__ __forceinline__ void rd_group_body(const WT *__restrict__ W, const fl
     constexpr int NT = 64 * NS, RPW = RPW_;
     static_assert(RPW % ROWS == 0, "rows per workgroup");
     static_assert(KV * NS * 64 * EW <= kX14MaxK, "windows");
-    static_assert(MT >= 1 && MT <= kX14MaxM, "activation rows");
+    static_assert(MT >= 1 && MT <= (F32 && KV <= 2 ? kGroupMaxMF32 : kX14MaxM), "activation rows");
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int rb = (int)blockIdx.x * RPW;
     const int nr = max(0, min(N, rb + RPW) - rb);
@@ -799,11 +800,11 @@ gemv_rd_stream_x4_kernel(const uint16_t *__restrict__ W, const float *__restrict
     rd_group_body<uint16_t, 1, MT, 4>(W, X, Y, N, K, ys_act, ys_row);
 }
 
-template <int MT>
+template <int KV, int MT>
 __global__ void __launch_bounds__(512)
 gemv_rd_stream_x8f_kernel(const float *__restrict__ W, const float *__restrict__ X, float *__restrict__ Y, int N,
                           int K, int64_t ys_act, int64_t ys_row) {
-    rd_group_body<float, 2, MT, 8>(W, X, Y, N, K, ys_act, ys_row);
+    rd_group_body<float, KV, MT, 8>(W, X, Y, N, K, ys_act, ys_row);
 }
 
 // One 8-wave group per CU: RPW rows per workgroup (N = RPW * CUs), ROWS per
@@ -3490,6 +3491,40 @@ hipError_t launch_cs(const CsProblem &p, const CsPlan &pl, void *workspace, hipS
 
 // ---- f32 weights, row-dot ------------------------------------------------------
 
+// Five and more activation rows on 16-byte f32 rows of K <= 14336: the group
+// kernels with up to 8 rows' x in registers (4 where a lane holds 3 or 4
+// windows), W read once per 8 (4) rows, evenly split; the streaming kernel
+// reads it once per 4 rows up to K = 4096, per 2 up to 8192 and per row beyond.
+// HBM bounds both.  Same box, streaming / here, us: W[14336,4096] m = 5 / 8 /
+// 16 84.7 / 82.9 / 164 against 40.2 / 41.9 / 83.2, [4096,14336] m = 5 / 8 / 16
+// 164 / 260 / 516 against 72 / 73 / 147, [4096,4096] m = 8 25.9 / 13.2,
+// [8192,2048] m = 8 25.2 / 13.6, [2000,12000] m = 8 109 / 45.  Not on short
+// rows, whose lanes would idle ([8192,1024] m = 16 22.6 / 22.7, [30000,512]
+// 22.2 / 29.8), nor on few workgroups ([1024,4096] m = 8 8.1 / 10.2;
+// [600,14336] m = 6 32.1 / 42.0).  Above 8 rows a matrix of up to 64 MiB keeps
+// its plan of 4 rows per workgroup, whose passes meet it in the last-level
+// cache ([4096,4096] m = 16 49 us).
+static bool f32_group_rows(const F32Problem &p, int64_t cus, F32Plan &pl) {
+    const int env = env_int("DMC_HIP_F32_GROUP_M", 1);  // 0: never; 2: wherever it applies
+    if (env == 0 || p.m <= kX14MaxM || p.k < 4 || p.k > kX14MaxK || p.k % 4 != 0 || p.ldw != p.k || p.ldx != p.k ||
+        !aligned(p.w, 16) || !aligned(p.x, 16) || env_int("DMC_HIP_F32_STREAM", 1) == 0)
+        return false;
+    const int64_t g16 = (p.n + 15) / 16;
+    if (env != 2 && (p.k <= 1024 || g16 < (p.k <= 4096 ? cus / 2 : cus / 4) ||
+                     (p.m > kGroupMaxMF32 && p.n * p.k * 4 <= (int64_t)64 << 20)))
+        return false;
+    const int waves = p.k <= 4096 ? 8 : kX14Waves;
+    pl.waves = waves;
+    pl.kvec = (int)((p.k + waves * 256 - 1) / (waves * 256));
+    const int most = pl.kvec <= 2 ? kGroupMaxMF32 : kX14MaxM;
+    pl.grid_y = (p.m + most - 1) / most;
+    pl.mt = (int)((p.m + pl.grid_y - 1) / pl.grid_y);
+    pl.rows = pl.mt <= 2 ? 2 : 1;
+    pl.rpw = 16;
+    pl.grid_x = g16;
+    return true;
+}
+
 F32Plan plan_f32(const F32Problem &p, int num_cus) {
     F32Plan pl{};
     const int64_t cus = num_cus > 0 ? num_cus : 256;
@@ -3522,6 +3557,7 @@ F32Plan plan_f32(const F32Problem &p, int num_cus) {
             return pl;
         }
     }
+    if (f32_group_rows(p, cus, pl)) return pl;
     // One group of 8 waves for 2048 < K <= 4096 (two windows of 4 weights per
     // lane, x in registers, zeros settled after the stream): at 3 or 4
     // activation rows, and where the 8-wave streaming kernel's last window
@@ -3622,48 +3658,48 @@ hipError_t launch_f32(const F32Problem &p, const F32Plan &pl, hipStream_t s) {
     if (p.k < 0 || p.m > INT32_MAX || p.n > INT32_MAX || p.k > INT32_MAX || pl.grid_x < 1 || pl.grid_y < 1 ||
         pl.grid_y > 65535 || pl.grid_x > INT32_MAX || pl.grid_x * pl.rpw < p.n || pl.grid_y * pl.mt < p.m)
         return hipErrorInvalidValue;
-    if (pl.kvec == 2 && pl.waves == 8 && pl.rpw == 16) {
-        if (pl.mt != p.m || p.m < 1 || p.m > kX14MaxM || p.k > 4096 || p.k < 1 || p.k % 4 != 0 || p.ldw != p.k ||
-            p.ldx != p.k || !aligned(p.w, 16) || !aligned(p.x, 16) || pl.grid_x != (p.n + 15) / 16 || pl.grid_y != 1)
+    if (pl.kvec > 0 && pl.rpw == 16) {
+        // The group kernels: 16 weight rows per workgroup, mt activation rows'
+        // x in registers, one launch per mt of them.
+        if ((pl.waves != 8 && pl.waves != kX14Waves) || pl.kvec > 4 || (pl.waves == 8 && pl.kvec > 2) || pl.mt < 1 ||
+            pl.mt > (pl.kvec <= 2 ? kGroupMaxMF32 : kX14MaxM) || (int64_t)pl.kvec * pl.waves * 256 < p.k ||
+            p.k > kX14MaxK || p.k < 1 || p.k % 4 != 0 || p.ldw != p.k || p.ldx != p.k || !aligned(p.w, 16) ||
+            !aligned(p.x, 16) || pl.grid_x != (p.n + 15) / 16)
             return hipErrorInvalidValue;
-#define DMC_F32X8(MT)                                                                                        \
-    hipLaunchKernelGGL((gemv_rd_stream_x8f_kernel<MT>), dim3((unsigned)pl.grid_x), dim3(512), 0, s, p.w, p.x, \
-                       p.y, (int)p.n, (int)p.k, p.ys_act, p.ys_row)
-        switch ((int)p.m) {
-        case 1: DMC_F32X8(1); break;
-        case 2: DMC_F32X8(2); break;
-        case 3: DMC_F32X8(3); break;
-        default: DMC_F32X8(4); break;
+        for (int64_t m0 = 0; m0 < p.m; m0 += pl.mt) {
+            const int mc = (int)std::min<int64_t>(pl.mt, p.m - m0);
+            const float *const x = p.x + m0 * p.ldx;
+            float *const y = p.y + m0 * p.ys_act;
+            const dim3 grid((unsigned)pl.grid_x), block(64 * pl.waves);
+#define DMC_F32G(KERNEL, ...)                                                                                 \
+    hipLaunchKernelGGL((KERNEL<__VA_ARGS__>), grid, block, 0, s, p.w, x, y, (int)p.n, (int)p.k, p.ys_act, p.ys_row); \
+    break
+#define DMC_F32G4(BASE, KERNEL, ...)                                                                          \
+    case BASE + 1: DMC_F32G(KERNEL, __VA_ARGS__, 1);                                                          \
+    case BASE + 2: DMC_F32G(KERNEL, __VA_ARGS__, 2);                                                          \
+    case BASE + 3: DMC_F32G(KERNEL, __VA_ARGS__, 3);                                                          \
+    case BASE + 4: DMC_F32G(KERNEL, __VA_ARGS__, 4);
+#define DMC_F32G8(BASE, KERNEL, ...)                                                                          \
+    DMC_F32G4(BASE, KERNEL, __VA_ARGS__)                                                                      \
+    case BASE + 5: DMC_F32G(KERNEL, __VA_ARGS__, 5);                                                          \
+    case BASE + 6: DMC_F32G(KERNEL, __VA_ARGS__, 6);                                                          \
+    case BASE + 7: DMC_F32G(KERNEL, __VA_ARGS__, 7);                                                          \
+    case BASE + 8: DMC_F32G(KERNEL, __VA_ARGS__, 8);
+            switch (pl.waves * 100 + pl.kvec * 10 + mc) {
+                DMC_F32G8(810, gemv_rd_stream_x8f_kernel, 1)
+                DMC_F32G8(820, gemv_rd_stream_x8f_kernel, 2)
+                DMC_F32G8(100 * kX14Waves + 20, gemv_rd_stream_x14_kernel, float, 2)
+                DMC_F32G4(100 * kX14Waves + 30, gemv_rd_stream_x14_kernel, float, 3)
+                DMC_F32G4(100 * kX14Waves + 40, gemv_rd_stream_x14_kernel, float, 4)
+            default: return hipErrorInvalidValue;
+            }
+#undef DMC_F32G8
+#undef DMC_F32G4
+#undef DMC_F32G
+            const hipError_t e = hipGetLastError();
+            if (e != hipSuccess) return e;
         }
-#undef DMC_F32X8
-        return hipGetLastError();
-    }
-    if (pl.kvec > 0 && pl.waves == kX14Waves) {
-        // The 14-wave kernel: 16 rows per workgroup, x straight into registers.
-        if (pl.rpw != 16 || pl.mt != p.m || p.m < 1 || p.m > kX14MaxM || pl.kvec < 2 || pl.kvec > 4 ||
-            (int64_t)pl.kvec * kX14Waves * 256 < p.k || p.k > kX14MaxK || p.k % 4 != 0 || p.ldw != p.k ||
-            p.ldx != p.k || !aligned(p.w, 16) || !aligned(p.x, 16) || pl.grid_x != (p.n + 15) / 16 || pl.grid_y != 1)
-            return hipErrorInvalidValue;
-#define DMC_F32X14(KV, MT)                                                                                  \
-    hipLaunchKernelGGL((gemv_rd_stream_x14_kernel<float, KV, MT>), dim3((unsigned)pl.grid_x),              \
-                       dim3(64 * kX14Waves), 0, s, p.w, p.x, p.y, (int)p.n, (int)p.k, p.ys_act, p.ys_row)
-        switch (pl.kvec * 10 + (int)p.m) {
-        case 21: DMC_F32X14(2, 1); break;
-        case 22: DMC_F32X14(2, 2); break;
-        case 23: DMC_F32X14(2, 3); break;
-        case 24: DMC_F32X14(2, 4); break;
-        case 31: DMC_F32X14(3, 1); break;
-        case 32: DMC_F32X14(3, 2); break;
-        case 33: DMC_F32X14(3, 3); break;
-        case 34: DMC_F32X14(3, 4); break;
-        case 41: DMC_F32X14(4, 1); break;
-        case 42: DMC_F32X14(4, 2); break;
-        case 43: DMC_F32X14(4, 3); break;
-        case 44: DMC_F32X14(4, 4); break;
-        default: return hipErrorInvalidValue;
-        }
-#undef DMC_F32X14
-        return hipGetLastError();
+        return hipSuccess;
     }
     if (pl.kvec > 0) {
         // The shapes the streaming kernel assumes (plan_f32's conditions).
