@@ -717,7 +717,8 @@ hipError_t launch_gemm_cs(const CsProblem &p, const CsPlan &pl, void *workspace,
     hipLaunchKernelGGL((gemv_mfma_gemm_kernel<8, MT, kSrcCols, true>), grid, dim3(512), 0, s, p.w, p.x,            \
                        (const uint16_t *)nullptr, p.y, part, (int)p.n, (int)p.k, (int)p.m, (int)kc, (int)pl.grid_x, \
                        (int)gy, gy > 1 ? 1 : 0, p.rs, p.ls)
-    if (pl.mt == 32) DMC_GEMM_CS(32);
+    if (pl.mt == 16) DMC_GEMM_CS(16);
+    else if (pl.mt == 32) DMC_GEMM_CS(32);
     else if (pl.mt == 64) DMC_GEMM_CS(64);
     else return hipErrorInvalidValue;
 #undef DMC_GEMM_CS

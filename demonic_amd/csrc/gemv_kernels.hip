@@ -3236,18 +3236,28 @@ static CsPlan plan_cs_fma(const CsProblem &p, int num_cus) {
 
 CsPlan plan_cs(const CsProblem &p, int num_cus) {
     const CsPlan fma = plan_cs_fma(p, num_cus);
-    // From 17 activation rows: the gemm layout over columns (the FMA kernels
+    // At many activation rows: the gemm layout over columns (the FMA kernels
     // stream W once per 4 rows).  Same box, these / here, us: C2 up m = 17 / 33
     // / 64 170 / 485 / 3675 against 33 / 42 / 46, down m = 64 3742 / 42; odd N,
     // [11007,4097] m = 32 414 / 38; the smallest, [512,512] m = 17 / 64 31 / 96
     // against 14 / 18; per-head batches, W [32,4096,128] m = 17 182 / 21.5.
+    // 5 to 16 rows on 16-row tiles, where W is large: C2 up m = 5 / 8 / 16 62 /
+    // 65 / 142 against 28.4 / 28.4 / 29.3, down m = 16 221 / 29.5, [32000,1024]
+    // m = 8 43 / 20, [4097,11008] m = 8 67 / 29.5, W [32,4096,128] m = 8 23 /
+    // 14, [32,128,4096] m = 8 43 / 19; 32-row tiles: 33 to 35 on C2.  A small W
+    // is the last-level cache's and its two launches count ([1024,4096] m = 8
+    // 16 / 19); a single matrix of up to 32 MiB keeps the FMA kernels' plan
+    // whole (their 4 rows per workgroup).  At 4 rows the FMA kernels' one pass is
+    // level: C2 up 33.8 / 28.2, down 25.9 / 27.9, [4097,11008] 25.7 / 29.2.
     const int env = env_int("DMC_HIP_CS_GEMM", 1);  // 0: never; 2: wherever it applies
     const int64_t cus = num_cus > 0 ? num_cus : 256, batch = std::max<int64_t>(p.batch, 1);
-    if (env == 0 || p.m < (env == 2 ? 1 : 17) || p.k < 1 || batch > 65535 ||
+    const int64_t bytes = batch * p.k * p.n * 2, large = (int64_t)32 << 20;
+    const int64_t least = env == 2 ? 1 : bytes > large || (batch > 1 && bytes == large) ? 5 : 17;
+    if (env == 0 || p.m < least || p.k < 1 || batch > 65535 ||
         (p.k + 64) * p.n * 2 > INT32_MAX || p.m * p.k * 4 > INT32_MAX)
         return fma;
     RdPlan g{};
-    g.mt = p.m <= 32 ? 32 : 64;
+    g.mt = p.m <= 16 ? 16 : p.m <= 32 ? 32 : 64;
     g.waves = 8;
     g.rpw = 256;
     gemm_split(p.m, p.n, p.k, std::max<int64_t>(1, cus / batch), 1, 1, g);

@@ -87,7 +87,8 @@ def test_rows_of_any_length_and_alignment(hip, m, k, n, offset, monkeypatch):
 
 @pytest.mark.parametrize("offset", [0, 2])
 @pytest.mark.parametrize("m,k,n,batch", [(17, 65, 257, 1), (33, 4097, 300, 1), (64, 63, 255, 1), (65, 1000, 513, 1),
-                                         (20, 128, 64, 3), (40, 70, 131, 2), (18, 1, 9, 1), (130, 2048, 1024, 1)])
+                                         (20, 128, 64, 3), (40, 70, 131, 2), (18, 1, 9, 1), (130, 2048, 1024, 1),
+                                         (16, 129, 259, 1), (5, 4097, 300, 1), (7, 64, 130, 3), (1, 66, 1, 1)])
 def test_columns_on_the_gemm_layout(hip, m, k, n, batch, offset, monkeypatch):
     """W [k,n] per batch slice on the gemm layout: partial column blocks, odd N
     (the last element shares a dword with what follows the matrix), K tails,
@@ -101,7 +102,7 @@ def test_columns_on_the_gemm_layout(hip, m, k, n, batch, offset, monkeypatch):
     with hip.DeviceBuffer.from_numpy(buf) as dw, hip.DeviceBuffer.from_numpy(x) as dx, \
             hip.DeviceBuffer(4 * batch * m * n) as dy:
         p = hip.plan("cs", m, k, n, batch=batch, rs=k * n, x_addr=dx.addr, w_addr=dw.addr + offset)
-        assert p.rows_or_rw == -256, p
+        assert p.rows_or_rw == -256 and p.mt == (16 if m <= 16 else 32 if m <= 32 else 64), p
         hip.gemv_cs(dx, dw.addr + offset, dy, m, k, n, batch, m * k, k * n)
         hip.synchronize()
         y = dy.download(np.float32, (batch, m, n))
