@@ -161,6 +161,7 @@ struct Ctx {
     Buf dx, dy, ws;         // device scratch (reuse is stream-ordered)
     Buf dwf, dwt;           // f32 route: a weight staged for one call, and its transpose
     int live_graphs = 0;    // executable graphs not yet destroyed
+    bool capturing = false; // between capture_begin and capture_end: the workspace cannot grow
     std::vector<void *> retired_ws;  // outgrown workspaces a live graph may still use
     Buf hx, hy;             // pinned staging
     size_t hx_off = 0, hy_off = 0;
@@ -301,6 +302,9 @@ int ensure_dev(Buf &b, size_t need) {
     b.cap = cap;
     return DMC_HIP_OK;
 }
+
+// The most workspace a plan may ask for: what is there, while capturing.
+int64_t ws_cap(const Ctx &c) { return c.capturing ? (int64_t)c.ws.cap : INT64_MAX; }
 
 int flush_locked();
 
@@ -1162,7 +1166,7 @@ int32_t dmc_hip_gemv_cs(int64_t x_dev, int64_t w_dev, int64_t y_dev, int64_t m, 
     Ctx &c = ctx();
     dmc::CsProblem p{reinterpret_cast<const uint16_t *>(w_dev), reinterpret_cast<const float *>(x_dev),
                      reinterpret_cast<float *>(y_dev), m, k, n, batch, ls, rs};
-    const dmc::CsPlan pl = dmc::plan_cs(p, c.cus);
+    const dmc::CsPlan pl = dmc::plan_cs(p, c.cus, ws_cap(c));
     if ((rc = ensure_dev(c.ws, pl.workspace_bytes))) return rc;
     hipError_t e = dmc::launch_cs(p, pl, c.ws.p, c.stream);
     if (e != hipSuccess) return hip_fail(e, "kernel launch");
@@ -1209,7 +1213,7 @@ int32_t dmc_hip_gemv_rd(int64_t x_dev, int64_t w_dev, int64_t y_dev, int64_t m, 
     Ctx &c = ctx();
     dmc::RdProblem p{reinterpret_cast<const uint16_t *>(w_dev), k, reinterpret_cast<const float *>(x_dev),
                      k, reinterpret_cast<float *>(y_dev), n, m, k, n};
-    const dmc::RdPlan pl = dmc::plan_rd(p, c.cus);
+    const dmc::RdPlan pl = dmc::plan_rd(p, c.cus, ws_cap(c));
     if ((rc = ensure_dev(c.ws, pl.workspace_bytes))) return rc;
     hipError_t e = dmc::launch_rd(p, pl, pl.workspace_bytes ? c.ws.p : nullptr, c.stream);
     if (e != hipSuccess) return hip_fail(e, "kernel launch");
@@ -1279,7 +1283,7 @@ int32_t dmc_hip_gemv_rd_grouped(int64_t count, const int64_t *x_devs, const int6
         for (int i = 0; i < g.count; ++i) {  // outside the streaming kernel's range: one launch each
             if (g.n[i] == 0) continue;
             dmc::RdProblem p{g.w[i], k, g.x[i], k, g.y[i], g.n[i], m, k, g.n[i]};
-            const dmc::RdPlan pl = dmc::plan_rd(p, c.cus);
+            const dmc::RdPlan pl = dmc::plan_rd(p, c.cus, ws_cap(c));
             if ((rc = ensure_dev(c.ws, pl.workspace_bytes))) return rc;
             hipError_t e = dmc::launch_rd(p, pl, pl.workspace_bytes ? c.ws.p : nullptr, c.stream);
             if (e != hipSuccess) return hip_fail(e, "kernel launch");
@@ -1344,12 +1348,14 @@ int32_t dmc_hip_capture_begin(void) {
     int rc = ensure_init();
     if (rc) return rc;
     HIP_TRY(hipStreamBeginCapture(ctx().stream, hipStreamCaptureModeThreadLocal), "hipStreamBeginCapture");
+    ctx().capturing = true;
     return DMC_HIP_OK;
 }
 
 int64_t dmc_hip_capture_end(void) {
     std::lock_guard<std::mutex> lk(g_mu);
     if (ensure_init()) return 0;
+    ctx().capturing = false;
     hipGraph_t graph = nullptr;
     hipError_t e = hipStreamEndCapture(ctx().stream, &graph);
     if (e != hipSuccess) return hip_fail(e, "hipStreamEndCapture (an entry that allocates or waits was "

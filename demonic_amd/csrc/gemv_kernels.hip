@@ -2692,7 +2692,7 @@ static double gemm_split(int64_t m, int64_t n, int64_t k, int64_t cus, int pair,
            (pl.kslices > 1 ? 5 + 0.42e-6 * ((double)pl.kslices * m * n * 4) : 0);
 }
 
-RdPlan plan_rd(const RdProblem &p, int num_cus) {
+RdPlan plan_rd(const RdProblem &p, int num_cus, int64_t ws_cap) {
     RdPlan pl{};
     // Widest load the row alignment allows: every row start, every activation
     // row start and the base pointers must be aligned to the vector size.
@@ -2922,7 +2922,12 @@ RdPlan plan_rd(const RdProblem &p, int num_cus) {
             RdPlan one = mp, two = mp;
             const int wg_per_cu = mp.mt == 16 || mp.waves == 4 ? 2 : 1;
             const double t1 = gemm_split(p.m, p.n, p.k, cus, 1, wg_per_cu, one);
-            mp = can_pair && (gemm_split(p.m, p.n, p.k, cus, 2, wg_per_cu, two) < t1 || penv == 2) ? two : one;
+            const bool pair = can_pair && (gemm_split(p.m, p.n, p.k, cus, 2, wg_per_cu, two) < t1 || penv == 2);
+            auto bytes = [&](const RdPlan &g) {
+                return (g.xfuse ? 0 : ((size_t)3 * p.m * p.k * 2 + 255) / 256 * 256) +
+                       (g.kslices > 1 ? (size_t)g.kslices * p.m * p.n * 4 : 0);
+            };
+            mp = pair && (int64_t)bytes(two) <= std::max(ws_cap, (int64_t)bytes(one)) ? two : one;
             // Workgroups split their own chunks of x (no planes, no split
             // launch) at 16-row tiles (C2 down at m = 16: the split launch cost
             // 3-4 us of 37), and at 32 and 64 while the repeated split stays
@@ -2935,8 +2940,7 @@ RdPlan plan_rd(const RdProblem &p, int num_cus) {
             // Two 64-row tiles per workgroup read and split twice as much x per
             // weight, and both in the kernel hold up to gx * m = 65536 (C2 up m =
             // 512 181 / 170, down m = 2048 626 / 562).
-            const size_t planes = mp.xfuse ? 0 : ((size_t)3 * p.m * p.k * 2 + 255) / 256 * 256;
-            mp.workspace_bytes = planes + (mp.kslices > 1 ? (size_t)mp.kslices * p.m * p.n * 4 : 0);
+            mp.workspace_bytes = bytes(mp);
         } else if (mp.mkind == 6) {
             mp.rpw = kWideRows;
         } else {
@@ -3039,6 +3043,10 @@ RdPlan plan_rd(const RdProblem &p, int num_cus) {
         mp.rpw = 256;
         gemm_split(p.m, p.n, p.k, cus, 1, 1, mp);
         mp.xfuse = true;
+        if (mp.kslices * p.m * p.n * 4 > ws_cap) {  // k in one slice needs none
+            mp.kslices = 1;
+            mp.kchunks = (int)((p.k + 63) / 64);
+        }
         mp.workspace_bytes = mp.kslices > 1 ? (size_t)mp.kslices * p.m * p.n * 4 : 0;
         mp.grid_x = (p.n + mp.rpw - 1) / mp.rpw;
         mp.grid_y = (p.m + mp.mt - 1) / mp.mt;
@@ -3234,7 +3242,7 @@ static CsPlan plan_cs_fma(const CsProblem &p, int num_cus) {
     return pl;
 }
 
-CsPlan plan_cs(const CsProblem &p, int num_cus) {
+CsPlan plan_cs(const CsProblem &p, int num_cus, int64_t ws_cap) {
     const CsPlan fma = plan_cs_fma(p, num_cus);
     // At many activation rows: the gemm layout over columns (the FMA kernels
     // stream W once per 4 rows).  Same box, these / here, us: C2 up m = 17 / 33
@@ -3262,9 +3270,11 @@ CsPlan plan_cs(const CsProblem &p, int num_cus) {
     g.rpw = 256;
     gemm_split(p.m, p.n, p.k, std::max<int64_t>(1, cus / batch), 1, 1, g);
     // The partial sums stay within the fixed scratch of the no-allocation
-    // entry, whose limit is judged by the FMA plan (workspace_bytes).
+    // entry, whose limit is judged by the FMA plan (workspace_bytes), and
+    // within ws_cap.
     const int64_t out = batch * p.m * p.n * 4;
-    while (g.kslices > 1 && g.kslices * out > (int64_t)noalloc_scratch_bytes()) {
+    const int64_t most = std::min<int64_t>(noalloc_scratch_bytes(), std::max<int64_t>(ws_cap, fma.workspace_bytes));
+    while (g.kslices > 1 && g.kslices * out > most) {
         const int64_t nchunks = (p.k + 63) / 64, s = g.kslices - 1;
         g.kchunks = (int)((nchunks + s - 1) / s);
         g.kslices = (int)((nchunks + g.kchunks - 1) / g.kchunks);

@@ -122,11 +122,13 @@ struct RdGroup {
     int64_t m, k;
 };
 
-RdPlan plan_rd(const RdProblem &p, int num_cus);
+// `ws_cap`: the most workspace a plan may ask for where one that needs less
+// would do (while a graph is captured the workspace cannot grow).
+RdPlan plan_rd(const RdProblem &p, int num_cus, int64_t ws_cap = INT64_MAX);
 // Streaming plan for a group; kvec == 0 when the streaming kernel cannot take
 // it (the caller then launches the problems one by one).
 RdPlan plan_rd_group(const RdGroup &g, int num_cus);
-CsPlan plan_cs(const CsProblem &p, int num_cus);
+CsPlan plan_cs(const CsProblem &p, int num_cus, int64_t ws_cap = INT64_MAX);
 
 // Enqueue on `stream`.  `workspace` must hold plan.workspace_bytes (row-dot:
 // the gemm layout's x planes and partial sums; column-stream: the partial sums

@@ -3,6 +3,10 @@ two 64-row activation tiles per workgroup at the edges of both, special values
 in the weights and in the activations (which send a tile through its second,
 hi-term pass), and outputs whose exact zero sends one wave through the
 reference chain."""
+import pathlib
+import subprocess
+import sys
+
 import numpy as np
 import pytest
 
@@ -108,3 +112,42 @@ def test_columns_on_the_gemm_layout(hip, m, k, n, batch, offset, monkeypatch):
         y = dy.download(np.float32, (batch, m, n))
     for z, (xz, wz, y_ref) in enumerate(zs):
         check_or_bound(y[z], y_ref, xz, W.bf16_to_f32(wz), f"gemm cols {m}x{k}x{n} slice {z}")
+
+
+FIRST_CALL_CAPTURED = """
+import sys
+import pathlib
+import subprocess
+import sys
+
+import numpy as np
+sys.path[:0] = [{root!r}, {root!r} + "/tests"]
+import demonic_amd as hip, oracle
+from demonic_amd import workloads as W
+from parity import check
+from test_gpu_parity import case
+assert hip.available()
+for m, k, n, columns in ((5, 4097, 3000, False), (40, 4097, 2000, False), (64, 1024, 8192, True)):
+    x, w = case(m, k, n, seed=m, scale=0.02)
+    y_ref = oracle.matmul_bf16_t(x, w)
+    with hip.DeviceBuffer.from_numpy(np.ascontiguousarray(w.T) if columns else w) as dw, \\
+            hip.DeviceBuffer.from_numpy(x) as dx, hip.DeviceBuffer(4 * m * n) as dy:
+        with hip.Graph() as g:
+            (hip.gemv_cs if columns else hip.gemv_rd)(dx, dw, dy, m, k, n)
+        for rep in range(3):
+            dy.upload(np.full(m * n, np.nan, np.float32))
+            g.launch()
+            hip.synchronize()
+            check(dy.download(np.float32, (m, n)), y_ref, what="captured first")
+    print("ok", m, k, n, flush=True)
+"""
+
+
+def test_a_first_call_inside_a_capture(hip):
+    """A process whose first GEMV is made while capturing, when the workspace
+    cannot grow: rows of any length and columns take k in one slice, as these
+    shapes' FMA kernels needed no workspace either."""
+    root = str(pathlib.Path(__file__).resolve().parent.parent)
+    r = subprocess.run([sys.executable, "-c", FIRST_CALL_CAPTURED.format(root=root)], capture_output=True, text=True,
+                       timeout=100)
+    assert r.returncode == 0 and r.stdout.count("ok") == 3, r.stdout + r.stderr
