@@ -209,21 +209,37 @@ __device__ __forceinline__ float wave_chain(const uint16_t *w, int64_t wstep, co
     return acc;
 }
 
-// Wave-uniform, for an output whose split sum is exactly zero: can the
-// reference chain end at -0?  A product x * w is a multiple of 2^(ex + ew - 284)
-// (biased exponents; 23 and 7 fraction bits).  Where that is at least 2^-149
-// for the least nonzero |x| and |w| of the two rows, every sum of the chain is
-// a multiple of the least subnormal, none underflows, and a chain that ends at
-// zero ends at +0 (an exact cancellation, or it never left +0).  So +0 is the
-// answer where the reference is zero, and where its roundings leave a residue,
-// +0 is as close to the exact sum as any other order's.  One pass over the
-// rows, against the chain's K dependent steps (4 us against 31 at K = 14336).
+// Wave-uniform, for an output whose split sum is exactly zero: is it settled
+// that +0 stands for the reference chain?  A product x * w is a multiple of
+// 2^(ex + ew - 284) (biased exponents; 23 and 7 fraction bits).  Where that is
+// at least 2^-149 for the least nonzero |x| and |w| of the two rows, every sum
+// of the chain is a multiple of the least subnormal, none underflows, and a
+// chain that ends at zero ends at +0 (an exact cancellation, or it never left
+// +0).  And where K products of the greatest |x| and |w| cannot reach inf, nor
+// can the chain on its way (|x| < 2^(ex - 126), |w| < 2^(ew - 126), and its
+// roundings grow a sum less than 4-fold up to K = 2^24).  So +0 is the answer
+// where the reference is zero, and where its roundings leave a residue, +0 is
+// as close to the exact sum as any other order's.  One pass over the rows,
+// against the chain's K dependent steps (4 us against 31 at K = 14336).
 template <int U>  // 512 * U elements a round: 12 registers each
 __device__ __forceinline__ bool wave_zero_is_plus(const uint16_t *w, int64_t wstep, const float *x, int K) {
     const int lane = threadIdx.x & 63;
     if (K <= 0) return true;
-    uint32_t xm = ~0u, wm = ((uint32_t)w[(int64_t)(K - 1) * wstep] & 0x7fffu) - 1u;  // least magnitude - 1: zeros on top
-    if (wstep <= 1 && K <= (1 << 28)) {
+    if (K > 1 << 24) return false;
+    const uint32_t wl = (uint32_t)w[(int64_t)(K - 1) * wstep] & 0x7fffu;
+    // least magnitude - 1 (zeros on top), greatest magnitude
+    uint32_t xm = ~0u, wm = wl - 1u, xt = 0, wt = wl;
+    auto put_x = [&](uint32_t v) {
+        v &= 0x7fffffffu;
+        xm = min(xm, v - 1u);
+        xt = max(xt, v);
+    };
+    auto put_w = [&](uint32_t v) {
+        v &= 0x7fffu;
+        wm = min(wm, v - 1u);
+        wt = max(wt, v);
+    };
+    if (wstep <= 1) {
         const uintptr_t wb = reinterpret_cast<uintptr_t>(w);
         const uint32_t wd = (uint32_t)(wb & 3);
         const __amdgpu_buffer_rsrc_t xr = weight_rsrc(x, (uint32_t)K * 4u);  // past K: zeros, which do not count
@@ -241,8 +257,10 @@ __device__ __forceinline__ bool wave_zero_is_plus(const uint16_t *w, int64_t wst
             for (int u = 0; u < U; ++u)
 #pragma unroll
                 for (int i = 0; i < 4; ++i) {
-                    xm = min(xm, min((xa[u][i] & 0x7fffffffu) - 1u, (xc[u][i] & 0x7fffffffu) - 1u));
-                    wm = min(wm, min((wv[u][i] & 0x7fffu) - 1u, (wv[u][i] >> 16 & 0x7fffu) - 1u));
+                    put_x(xa[u][i]);
+                    put_x(xc[u][i]);
+                    put_w(wv[u][i]);
+                    put_w(wv[u][i] >> 16);
                 }
         }
     } else {
@@ -250,8 +268,8 @@ __device__ __forceinline__ bool wave_zero_is_plus(const uint16_t *w, int64_t wst
 #pragma unroll
             for (int u = 0; u < U; ++u) {
                 const int k = min(k0 + u * 64 + lane, K - 1);
-                xm = min(xm, (__float_as_uint(x[k]) & 0x7fffffffu) - 1u);
-                wm = min(wm, ((uint32_t)w[(int64_t)k * wstep] & 0x7fffu) - 1u);
+                put_x(__float_as_uint(x[k]));
+                put_w((uint32_t)w[(int64_t)k * wstep]);
             }
         }
     }
@@ -259,9 +277,12 @@ __device__ __forceinline__ bool wave_zero_is_plus(const uint16_t *w, int64_t wst
     for (int o = 32; o > 0; o >>= 1) {
         xm = min(xm, (uint32_t)__shfl_xor((int)xm, o));
         wm = min(wm, (uint32_t)__shfl_xor((int)wm, o));
+        xt = max(xt, (uint32_t)__shfl_xor((int)xt, o));
+        wt = max(wt, (uint32_t)__shfl_xor((int)wt, o));
     }
     const uint32_t ex = (xm + 1) >> 23, ew = (wm + 1) >> 7;
-    return xm == ~0u || wm == ~0u || (ex >= 1 && ew >= 1 && ex + ew >= 135);
+    const uint32_t lg = 32 - __builtin_clz((uint32_t)K);  // K < 2^lg
+    return xt == 0 || wt == 0 || (ex >= 1 && ew >= 1 && ex + ew >= 135 && (xt >> 23) + (wt >> 7) + lg <= 377);
 }
 
 // The reference's values for the lanes whose sums are exactly zero (`ask`; w, x

@@ -12,8 +12,8 @@ import pytest
 
 import oracle
 from demonic_amd import workloads as W
-from parity import check, check_bound, check_or_bound
-from test_gpu_parity import case, run_rd
+from parity import check, check_bound, check_classes, check_or_bound
+from test_gpu_parity import case, run_cs_dev, run_rd
 
 pytestmark = pytest.mark.gpu
 
@@ -38,23 +38,54 @@ def test_one_and_two_activation_tiles(hip, m, k, n, pair, fuse, monkeypatch):
     check_or_bound(run_rd(hip, x, w), y_ref, x, W.bf16_to_f32(w), f"gemm pair={pair} fuse={fuse} {m}x{k}x{n}")
 
 
-@pytest.mark.parametrize("slices", [1, 4])
-def test_a_lone_cancelling_output_takes_the_chain(hip, slices, monkeypatch):
-    """One output in 80 x 300 whose sum is exactly zero, K long enough for
-    several rounds of the wave's chain: the reference's bits."""
-    m, k, n = 80, 3008, 300
-    monkeypatch.setenv("DMC_HIP_RD_MFMA_KIND", "8")
-    monkeypatch.setenv("DMC_HIP_GEMM_MAX_SLICES", str(slices))
+ROUTES = [  # (environment, K, W stored [k,n])
+    pytest.param({"DMC_HIP_RD_MFMA_KIND": "8", "DMC_HIP_GEMM_MAX_SLICES": "1"}, 3008, False, id="gemm"),
+    pytest.param({"DMC_HIP_RD_MFMA_KIND": "8", "DMC_HIP_GEMM_MAX_SLICES": "4"}, 3008, False, id="gemm-slices"),
+    pytest.param({"DMC_HIP_RD_MFMA_KIND": "7"}, 3008, False, id="rows16"),
+    pytest.param({"DMC_HIP_RD_MFMA_KIND": "6"}, 3008, False, id="wide"),
+    pytest.param({"DMC_HIP_RD_GEMM_ROWS": "2", "DMC_HIP_GEMM_MAX_SLICES": "1"}, 3001, False, id="rows"),
+    pytest.param({"DMC_HIP_RD_GEMM_ROWS": "2"}, 3001, False, id="rows-slices"),
+    pytest.param({"DMC_HIP_CS_GEMM": "2", "DMC_HIP_GEMM_MAX_SLICES": "1"}, 3001, True, id="columns"),
+    pytest.param({"DMC_HIP_CS_GEMM": "2"}, 3001, True, id="columns-slices"),
+]
+
+
+def on_route(hip, x, w, columns):
+    return run_cs_dev(hip, x, w) if columns else run_rd(hip, x, w)
+
+
+@pytest.mark.parametrize("env,k,columns", ROUTES)
+def test_zero_sums_take_the_reference_chain(hip, env, k, columns, monkeypatch):
+    """Sums that come out exactly zero, alone in 80 x 300 and many in one wave,
+    K long enough for several rounds of the wave's chain:
+    - full cancellation of ordinary products (the reference: +0);
+    - products that all underflow, positive and then, past k = 2000, negative,
+      in a row that is not all tiny since its largest element meets a weight
+      of 0 (the reference chain: -0);
+    - products that cancel after the chain has overflowed (the reference: inf)."""
+    m, n = 80, 300
+    for name, value in env.items():
+        monkeypatch.setenv(name, value)
     x, w = case(m, k, n, seed=5, scale=0.02)
+    x[:, :4] = 0.25
     x[70] = 1
-    w[200, : k // 2], w[200, k // 2:] = 0x3F80, 0xBF80
-    y_ref = oracle.matmul_bf16_t(x, w)
-    assert y_ref[70, 200] == 0
-    y = run_rd(hip, x, w)
-    assert y[70, 200].view(np.uint32) == y_ref[70, 200].view(np.uint32)
-    check(y, y_ref, what="lone zero")
-    for r in (0, 70, 79):
-        check_bound(y[r], y_ref[r], x[r], W.bf16_to_f32(w), what=f"lone zero row {r}")
+    half = k // 2
+    w[200] = 0
+    w[200, :half], w[200, half:2 * half] = 0x3F80, 0xBF80
+    x[30] = np.float32(1e-38)
+    x[30, 0], x[30, 2000:] = 1, np.float32(-1e-38)
+    w[100], w[100, 0] = 0x0001, 0
+    w[240:260], w[240:260, 0] = 0x0001, 0
+    w[50] = 0
+    w[50, 0:2], w[50, 2:4] = 0x7F62, 0xFF62  # 3e38 twice, -3e38 twice
+    with np.errstate(over="ignore"):
+        y_ref = oracle.matmul_bf16_t(x, w)
+    assert y_ref[70, 200] == 0 and np.isposinf(y_ref[70, 50])
+    assert all(y_ref[30, c] == 0 and np.signbit(y_ref[30, c]) for c in [100, *range(240, 260)])
+    y = on_route(hip, x, w, columns)
+    for r, c in ((70, 200), (70, 50), (30, 100), (30, 240), (30, 259)):
+        assert y[r, c].view(np.uint32) == y_ref[r, c].view(np.uint32), (r, c, y[r, c], y_ref[r, c])
+    check_or_bound(y, y_ref, x, W.bf16_to_f32(w), what="zero sums")
 
 
 def planted(m, k, n, seed):
