@@ -781,6 +781,10 @@ template <typename WT, int KV, int MT>
 __global__ void __launch_bounds__(64 * kX14Waves)
 gemv_rd_stream_x14_kernel(const WT *__restrict__ W, const float *__restrict__ X, float *__restrict__ Y, int N, int K,
                           int64_t ys_act, int64_t ys_row) {
+    if constexpr (sizeof(WT) == 4) {  // activation rows MT * blockIdx.y on
+        X += (int64_t)blockIdx.y * MT * K;
+        Y += (int64_t)blockIdx.y * MT * ys_act;
+    }
     rd_group_body<WT, KV, MT, kX14Waves>(W, X, Y, N, K, ys_act, ys_row);
 }
 
@@ -804,6 +808,8 @@ template <int KV, int MT>
 __global__ void __launch_bounds__(512)
 gemv_rd_stream_x8f_kernel(const float *__restrict__ W, const float *__restrict__ X, float *__restrict__ Y, int N,
                           int K, int64_t ys_act, int64_t ys_row) {
+    X += (int64_t)blockIdx.y * MT * K;  // activation rows MT * blockIdx.y on
+    Y += (int64_t)blockIdx.y * MT * ys_act;
     rd_group_body<float, KV, MT, 8>(W, X, Y, N, K, ys_act, ys_row);
 }
 
@@ -3516,8 +3522,8 @@ hipError_t launch_cs(const CsProblem &p, const CsPlan &pl, void *workspace, hipS
 // windows), W read once per 8 (4) rows, evenly split; the streaming kernel
 // reads it once per 4 rows up to K = 4096, per 2 up to 8192 and per row beyond.
 // HBM bounds both.  Same box, streaming / here, us: W[14336,4096] m = 5 / 8 /
-// 16 84.7 / 82.9 / 164 against 40.2 / 41.9 / 83.2, [4096,14336] m = 5 / 8 / 16
-// 164 / 260 / 516 against 72 / 73 / 147, [4096,4096] m = 8 25.9 / 13.2,
+// 16 84.7 / 82.9 / 164 against 40.2 / 41.9 / 76, [4096,14336] m = 5 / 8 / 16
+// 164 / 260 / 516 against 72 / 73 / 139, [4096,4096] m = 8 25.9 / 13.2,
 // [8192,2048] m = 8 25.2 / 13.6, [2000,12000] m = 8 109 / 45.  Not on short
 // rows, whose lanes would idle ([8192,1024] m = 16 22.6 / 22.7, [30000,512]
 // 22.2 / 29.8), nor on few workgroups ([1024,4096] m = 8 8.1 / 10.2;
@@ -3537,6 +3543,7 @@ static bool f32_group_rows(const F32Problem &p, int64_t cus, F32Plan &pl) {
     pl.waves = waves;
     pl.kvec = (int)((p.k + waves * 256 - 1) / (waves * 256));
     const int most = pl.kvec <= 2 ? kGroupMaxMF32 : kX14MaxM;
+    if ((p.m + most - 1) / most > 65535) return false;  // the grid's second extent: the general kernel holds 16 rows
     pl.grid_y = (p.m + most - 1) / most;
     pl.mt = (int)((p.m + pl.grid_y - 1) / pl.grid_y);
     pl.rows = pl.mt <= 2 ? 2 : 1;
@@ -3680,17 +3687,22 @@ hipError_t launch_f32(const F32Problem &p, const F32Plan &pl, hipStream_t s) {
         return hipErrorInvalidValue;
     if (pl.kvec > 0 && pl.rpw == 16) {
         // The group kernels: 16 weight rows per workgroup, mt activation rows'
-        // x in registers, one launch per mt of them.
+        // x in registers.
         if ((pl.waves != 8 && pl.waves != kX14Waves) || pl.kvec > 4 || (pl.waves == 8 && pl.kvec > 2) || pl.mt < 1 ||
             pl.mt > (pl.kvec <= 2 ? kGroupMaxMF32 : kX14MaxM) || (int64_t)pl.kvec * pl.waves * 256 < p.k ||
             p.k > kX14MaxK || p.k < 1 || p.k % 4 != 0 || p.ldw != p.k || p.ldx != p.k || !aligned(p.w, 16) ||
             !aligned(p.x, 16) || pl.grid_x != (p.n + 15) / 16)
             return hipErrorInvalidValue;
-        for (int64_t m0 = 0; m0 < p.m; m0 += pl.mt) {
+        // The whole groups in one launch, what is left in a second.  A launch
+        // per group / so, us: W[14336,4096] m = 16 / 64 86.6 / 350 against 76.3 /
+        // 291, [4096,14336] m = 16 147 / 139, [30000,8192] m = 13 677 / 641.
+        for (int64_t m0 = 0; m0 < p.m;) {
             const int mc = (int)std::min<int64_t>(pl.mt, p.m - m0);
+            const int64_t groups = (p.m - m0) / mc;
             const float *const x = p.x + m0 * p.ldx;
             float *const y = p.y + m0 * p.ys_act;
-            const dim3 grid((unsigned)pl.grid_x), block(64 * pl.waves);
+            m0 += groups * mc;
+            const dim3 grid((unsigned)pl.grid_x, (unsigned)groups), block(64 * pl.waves);
 #define DMC_F32G(KERNEL, ...)                                                                                 \
     hipLaunchKernelGGL((KERNEL<__VA_ARGS__>), grid, block, 0, s, p.w, x, y, (int)p.n, (int)p.k, p.ys_act, p.ys_row); \
     break

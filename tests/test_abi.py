@@ -697,6 +697,16 @@ def test_f32_activation_rows_per_workgroup(monkeypatch):
     assert d.plan_f32(16, 4097, 64, x_addr=256, w_addr=256).mt == 16      # general
 
 
+@pytest.mark.parametrize("k,n,most", [(4096, 14336, 8), (7168, 14336, 8), (14336, 14336, 4)])
+def test_f32_group_rows_stay_within_a_grid(k, n, most):
+    """The group kernels' activation groups are a grid's second extent, at most
+    65535; more rows than that go to the general kernel, which holds 16."""
+    p = d.plan_f32(65535 * most, k, n, x_addr=256, w_addr=256)
+    assert (p.rows_per_group, p.mt, p.grid_y) == (16, most, 65535), p
+    p = d.plan_f32(65535 * most + 1, k, n, x_addr=256, w_addr=256)
+    assert (p.kvec, p.mt) == (0, 16) and p.grid_y <= 65535, p
+
+
 def test_f32_entries_reject_gemm_shapes_before_touching_a_device():
     lib = _lib.load()
     l = np.ones((17, 8), np.float32)

@@ -1,6 +1,6 @@
 """GPU parity of the f32 group kernels at 5 and more activation rows: W read
 once per 8 rows (4 where a lane holds 3 or 4 windows), the rows split evenly
-over the launches."""
+over the groups."""
 import numpy as np
 import pytest
 
@@ -11,7 +11,7 @@ from test_gpu_f32 import edge
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("m", [5, 8, 9, 17])
+@pytest.mark.parametrize("m", [5, 8, 9, 17, 40])
 @pytest.mark.parametrize("n,k", [(33, 4), (300, 2048), (17, 2052), (40, 4096), (16, 4100), (35, 7168), (18, 7172),
                                  (50, 14336)])
 def test_group_rows_f32(hip, n, k, m, monkeypatch):
