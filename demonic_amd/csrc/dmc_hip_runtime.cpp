@@ -161,7 +161,6 @@ struct Ctx {
     Buf dx, dy, ws;         // device scratch (reuse is stream-ordered)
     Buf dwf, dwt;           // f32 route: a weight staged for one call, and its transpose
     int live_graphs = 0;    // executable graphs not yet destroyed
-    bool capturing = false; // between capture_begin and capture_end: the workspace cannot grow
     std::vector<void *> retired_ws;  // outgrown workspaces a live graph may still use
     Buf hx, hy;             // pinned staging
     size_t hx_off = 0, hy_off = 0;
@@ -303,8 +302,22 @@ int ensure_dev(Buf &b, size_t need) {
     return DMC_HIP_OK;
 }
 
-// The most workspace a plan may ask for: what is there, while capturing.
-int64_t ws_cap(const Ctx &c) { return c.capturing ? (int64_t)c.ws.cap : INT64_MAX; }
+// The workspace at no less than `need` bytes if there is memory for it; else it
+// stays as it is.  Drained and retired as in ensure_dev.
+void reserve_ws(size_t need) {
+    Ctx &c = ctx();
+    void *p = nullptr;
+    if (need <= c.ws.cap) return;
+    if (hipMalloc(&p, need) != hipSuccess || hipStreamSynchronize(c.stream) != hipSuccess) {
+        (void)hipGetLastError();
+        if (p) (void)hipFree(p);
+        return;
+    }
+    if (c.ws.p && c.live_graphs > 0) c.retired_ws.push_back(c.ws.p);
+    else if (c.ws.p) (void)hipFree(c.ws.p);
+    c.ws.p = p;
+    c.ws.cap = need;
+}
 
 int flush_locked();
 
@@ -1166,7 +1179,7 @@ int32_t dmc_hip_gemv_cs(int64_t x_dev, int64_t w_dev, int64_t y_dev, int64_t m, 
     Ctx &c = ctx();
     dmc::CsProblem p{reinterpret_cast<const uint16_t *>(w_dev), reinterpret_cast<const float *>(x_dev),
                      reinterpret_cast<float *>(y_dev), m, k, n, batch, ls, rs};
-    const dmc::CsPlan pl = dmc::plan_cs(p, c.cus, ws_cap(c));
+    const dmc::CsPlan pl = dmc::plan_cs(p, c.cus);
     if ((rc = ensure_dev(c.ws, pl.workspace_bytes))) return rc;
     hipError_t e = dmc::launch_cs(p, pl, c.ws.p, c.stream);
     if (e != hipSuccess) return hip_fail(e, "kernel launch");
@@ -1193,11 +1206,12 @@ int32_t dmc_hip_gemv_cs_noalloc(int64_t x_dev, int64_t w_dev, int64_t y_dev, int
     dmc::CsProblem p{reinterpret_cast<const uint16_t *>(w_dev), reinterpret_cast<const float *>(x_dev),
                      reinterpret_cast<float *>(y_dev), m, k, n, batch, ls, rs};
     const dmc::CsPlan pl = dmc::plan_cs(p, c.cus);
-    if (pl.workspace_bytes > dmc::noalloc_scratch_bytes())
+    const size_t need = std::max(pl.noalloc_bytes, pl.workspace_bytes);
+    if (need > dmc::noalloc_scratch_bytes())
         return fail(DMC_HIP_EINVAL,
                     "dmc_hip_gemv_cs_noalloc: this shape needs %zu bytes of split-k scratch, the fixed maximum is "
                     "%zu (use dmc_hip_gemv_cs)",
-                    pl.workspace_bytes, dmc::noalloc_scratch_bytes());
+                    need, dmc::noalloc_scratch_bytes());
     hipError_t e = dmc::launch_cs(p, pl, it->second, c.stream);
     if (e != hipSuccess) return hip_fail(e, "kernel launch");
     return DMC_HIP_OK;
@@ -1213,7 +1227,7 @@ int32_t dmc_hip_gemv_rd(int64_t x_dev, int64_t w_dev, int64_t y_dev, int64_t m, 
     Ctx &c = ctx();
     dmc::RdProblem p{reinterpret_cast<const uint16_t *>(w_dev), k, reinterpret_cast<const float *>(x_dev),
                      k, reinterpret_cast<float *>(y_dev), n, m, k, n};
-    const dmc::RdPlan pl = dmc::plan_rd(p, c.cus, ws_cap(c));
+    const dmc::RdPlan pl = dmc::plan_rd(p, c.cus);
     if ((rc = ensure_dev(c.ws, pl.workspace_bytes))) return rc;
     hipError_t e = dmc::launch_rd(p, pl, pl.workspace_bytes ? c.ws.p : nullptr, c.stream);
     if (e != hipSuccess) return hip_fail(e, "kernel launch");
@@ -1283,7 +1297,7 @@ int32_t dmc_hip_gemv_rd_grouped(int64_t count, const int64_t *x_devs, const int6
         for (int i = 0; i < g.count; ++i) {  // outside the streaming kernel's range: one launch each
             if (g.n[i] == 0) continue;
             dmc::RdProblem p{g.w[i], k, g.x[i], k, g.y[i], g.n[i], m, k, g.n[i]};
-            const dmc::RdPlan pl = dmc::plan_rd(p, c.cus, ws_cap(c));
+            const dmc::RdPlan pl = dmc::plan_rd(p, c.cus);
             if ((rc = ensure_dev(c.ws, pl.workspace_bytes))) return rc;
             hipError_t e = dmc::launch_rd(p, pl, pl.workspace_bytes ? c.ws.p : nullptr, c.stream);
             if (e != hipSuccess) return hip_fail(e, "kernel launch");
@@ -1347,15 +1361,18 @@ int32_t dmc_hip_capture_begin(void) {
     std::lock_guard<std::mutex> lk(g_mu);
     int rc = ensure_init();
     if (rc) return rc;
-    HIP_TRY(hipStreamBeginCapture(ctx().stream, hipStreamCaptureModeThreadLocal), "hipStreamBeginCapture");
-    ctx().capturing = true;
+    // The workspace cannot grow while capturing: room now for the k slices of
+    // any gemm-layout plan, so that a shape's first call may be a recorded one.
+    // (Without that much memory, calls that need it are refused one by one.)
+    Ctx &c = ctx();
+    reserve_ws(dmc::max_split_bytes(c.cus));
+    HIP_TRY(hipStreamBeginCapture(c.stream, hipStreamCaptureModeThreadLocal), "hipStreamBeginCapture");
     return DMC_HIP_OK;
 }
 
 int64_t dmc_hip_capture_end(void) {
     std::lock_guard<std::mutex> lk(g_mu);
     if (ensure_init()) return 0;
-    ctx().capturing = false;
     hipGraph_t graph = nullptr;
     hipError_t e = hipStreamEndCapture(ctx().stream, &graph);
     if (e != hipSuccess) return hip_fail(e, "hipStreamEndCapture (an entry that allocates or waits was "

@@ -2698,7 +2698,12 @@ static double gemm_split(int64_t m, int64_t n, int64_t k, int64_t cus, int pair,
            (pl.kslices > 1 ? 5 + 0.42e-6 * ((double)pl.kslices * m * n * 4) : 0);
 }
 
-RdPlan plan_rd(const RdProblem &p, int num_cus, int64_t ws_cap) {
+// At most 2 * wg_per_cu workgroups per CU hold a slice's sums of rpw weight rows
+// by mt * pair activation rows each: two tiles of 256 x 64 on one workgroup per
+// CU is the largest of the forms (the others: half of that).
+size_t max_split_bytes(int num_cus) { return (size_t)2 * std::max(1, num_cus) * 256 * 128 * 4; }
+
+RdPlan plan_rd(const RdProblem &p, int num_cus) {
     RdPlan pl{};
     // Widest load the row alignment allows: every row start, every activation
     // row start and the base pointers must be aligned to the vector size.
@@ -2933,7 +2938,7 @@ RdPlan plan_rd(const RdProblem &p, int num_cus, int64_t ws_cap) {
                 return (g.xfuse ? 0 : ((size_t)3 * p.m * p.k * 2 + 255) / 256 * 256) +
                        (g.kslices > 1 ? (size_t)g.kslices * p.m * p.n * 4 : 0);
             };
-            mp = pair && (int64_t)bytes(two) <= std::max(ws_cap, (int64_t)bytes(one)) ? two : one;
+            mp = pair ? two : one;
             // Workgroups split their own chunks of x (no planes, no split
             // launch) at 16-row tiles (C2 down at m = 16: the split launch cost
             // 3-4 us of 37), and at 32 and 64 while the repeated split stays
@@ -3049,10 +3054,6 @@ RdPlan plan_rd(const RdProblem &p, int num_cus, int64_t ws_cap) {
         mp.rpw = 256;
         gemm_split(p.m, p.n, p.k, cus, 1, 1, mp);
         mp.xfuse = true;
-        if (mp.kslices * p.m * p.n * 4 > ws_cap) {  // k in one slice needs none
-            mp.kslices = 1;
-            mp.kchunks = (int)((p.k + 63) / 64);
-        }
         mp.workspace_bytes = mp.kslices > 1 ? (size_t)mp.kslices * p.m * p.n * 4 : 0;
         mp.grid_x = (p.n + mp.rpw - 1) / mp.rpw;
         mp.grid_y = (p.m + mp.mt - 1) / mp.mt;
@@ -3248,8 +3249,9 @@ static CsPlan plan_cs_fma(const CsProblem &p, int num_cus) {
     return pl;
 }
 
-CsPlan plan_cs(const CsProblem &p, int num_cus, int64_t ws_cap) {
-    const CsPlan fma = plan_cs_fma(p, num_cus);
+CsPlan plan_cs(const CsProblem &p, int num_cus) {
+    CsPlan fma = plan_cs_fma(p, num_cus);
+    fma.noalloc_bytes = fma.workspace_bytes;
     // At many activation rows: the gemm layout over columns (the FMA kernels
     // stream W once per 4 rows).  Same box, these / here, us: C2 up m = 17 / 33
     // / 64 170 / 485 / 3675 against 33 / 42 / 46, down m = 64 3742 / 42; odd N,
@@ -3276,11 +3278,9 @@ CsPlan plan_cs(const CsProblem &p, int num_cus, int64_t ws_cap) {
     g.rpw = 256;
     gemm_split(p.m, p.n, p.k, std::max<int64_t>(1, cus / batch), 1, 1, g);
     // The partial sums stay within the fixed scratch of the no-allocation
-    // entry, whose limit is judged by the FMA plan (workspace_bytes), and
-    // within ws_cap.
+    // entry, which refuses by the FMA plan's bytes (noalloc_bytes).
     const int64_t out = batch * p.m * p.n * 4;
-    const int64_t most = std::min<int64_t>(noalloc_scratch_bytes(), std::max<int64_t>(ws_cap, fma.workspace_bytes));
-    while (g.kslices > 1 && g.kslices * out > most) {
+    while (g.kslices > 1 && g.kslices * out > (int64_t)noalloc_scratch_bytes()) {
         const int64_t nchunks = (p.k + 63) / 64, s = g.kslices - 1;
         g.kchunks = (int)((nchunks + s - 1) / s);
         g.kslices = (int)((nchunks + g.kchunks - 1) / g.kchunks);
@@ -3295,7 +3295,7 @@ CsPlan plan_cs(const CsProblem &p, int num_cus, int64_t ws_cap) {
     pl.kslice = (int64_t)g.kchunks * 64;
     pl.slices = g.kslices;
     pl.grid_x = (p.n + 255) / 256;
-    pl.workspace_bytes = std::max<size_t>(fma.workspace_bytes, pl.slices > 1 ? (size_t)pl.slices * out : 0);
+    pl.workspace_bytes = pl.slices > 1 ? (size_t)pl.slices * out : 0;
     if (pl.grid_x * ((p.m + pl.mt - 1) / pl.mt) * pl.slices > INT32_MAX) return fma;
     return pl;
 }

@@ -106,6 +106,7 @@ struct CsPlan {
     int64_t slices; // number of k slices (1 = no reduction across workgroups)
     int64_t grid_x;
     size_t workspace_bytes;  // partial sums when slices > 1
+    size_t noalloc_bytes;    // what the no-allocation entry judges a shape by: the FMA kernels' workspace
 };
 
 // Up to kMaxGroup independent row-dot problems that share m and k (and x's
@@ -122,13 +123,16 @@ struct RdGroup {
     int64_t m, k;
 };
 
-// `ws_cap`: the most workspace a plan may ask for where one that needs less
-// would do (while a graph is captured the workspace cannot grow).
-RdPlan plan_rd(const RdProblem &p, int num_cus, int64_t ws_cap = INT64_MAX);
+// A plan depends on the problem and the device alone, never on earlier calls or
+// on a capture in progress: the same call gives the same bits, recorded or run.
+RdPlan plan_rd(const RdProblem &p, int num_cus);
 // Streaming plan for a group; kvec == 0 when the streaming kernel cannot take
 // it (the caller then launches the problems one by one).
 RdPlan plan_rd_group(const RdGroup &g, int num_cus);
-CsPlan plan_cs(const CsProblem &p, int num_cus, int64_t ws_cap = INT64_MAX);
+CsPlan plan_cs(const CsProblem &p, int num_cus);
+// The most that the gemm layout's k slices take in partial sums (not x's
+// planes), whatever the problem: 64 MiB on 256 CUs.
+size_t max_split_bytes(int num_cus);
 
 // Enqueue on `stream`.  `workspace` must hold plan.workspace_bytes (row-dot:
 // the gemm layout's x planes and partial sums; column-stream: the partial sums

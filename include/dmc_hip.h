@@ -285,8 +285,10 @@ int32_t dmc_hip_bf16_transpose_2d(int64_t src_dev, int64_t dst_dev, int64_t m, i
  * recorded instead of run, provided that any plan whose dmc_hip_plan
  * workspace_bytes > 0 (column-stream split-K partials; row-dot k-slice
  * partials on the rows16 and gemm layouts, or x's bf16 planes) already fits
- * the library workspace, i.e. after one uncaptured call of the same shape;
- * capture_end returns an
+ * the library workspace: 64 MiB, which capture_begin reserves and which hold
+ * the k-slice partials of any gemm-layout plan, or more after one uncaptured
+ * call of a shape that needs more.  A recorded call's results are the uncaptured
+ * call's, bit for bit.  capture_end returns an
  * executable graph (0 on error: an entry that allocates or waits was called
  * while capturing) that graph_launch replays on the library stream.  While
  * any graph is alive, a workspace outgrown by a later call stays allocated

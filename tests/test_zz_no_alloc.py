@@ -29,13 +29,15 @@ def run(hip, entry, x, wt, m, k, n, batch, ls, rs):
         return dy.download(np.float32, (batch * m * n,))
 
 
-@pytest.mark.parametrize("shapes", [[(2, 4096, 14336, 1), (1, 1000, 515, 3)]])
+@pytest.mark.parametrize("shapes", [[(2, 4096, 14336, 1), (1, 1000, 515, 3)],
+                                    [(64, 4096, 1024, 1), (20, 2000, 259, 3)]])  # FMA kernels; gemm layout
 def test_noalloc_matches_gemv_cs_on_consecutive_calls(hip, shapes):
     lib = _lib.load()
     assert hip.available()
     for m, k, n, batch in shapes:   # the second call is smaller, with odd N (the unaligned kernel)
         p = hip.plan("cs", m, k, n, batch=batch, rs=k * n)
         assert 0 < p.workspace_bytes <= LIMIT, p   # the split-k partials do use the scratch
+        assert (p.rows_or_rw == -256) == (m >= 17), p
         rng = np.random.default_rng(m * 1000 + n)
         x = rng.standard_normal(batch * m * k).astype(np.float32)
         wt = W.bf16_rne(np.float32(0.02) * rng.standard_normal(batch * k * n).astype(np.float32))
