@@ -93,18 +93,6 @@ __device__ __forceinline__ int swz_cols(int r, int p) {
     return r * 128 + ((p ^ (((r >> 1) ^ (r >> 4 & 1)) & 7)) << 4);
 }
 
-// Does some weight of a row (wstep 1) or a column (wstep N) differ from +-0?  Wave-uniform; the rare path.
-__device__ bool wave_weights_nonzero(const uint16_t *w, int64_t wstep, int K) {
-    constexpr int U = 16;
-    for (int k0 = 0; k0 < K; k0 += 64 * U) {
-        uint32_t hit = 0;
-#pragma unroll
-        for (int u = 0; u < U; ++u) hit |= w[(int64_t)min(k0 + u * 64 + (int)(threadIdx.x & 63), K - 1) * wstep];
-        if (__builtin_amdgcn_ballot_w64((hit & 0x7fffu) != 0) != 0) return true;
-    }
-    return false;
-}
-
 // s += p, and what the rounding of that sum lost.
 __device__ __forceinline__ float add_exact(float &s, float p) {
     const float t = s + p, b = t - s;
@@ -500,17 +488,8 @@ gemv_mfma_gemm_kernel(const uint16_t *__restrict__ W, const float *__restrict__ 
                                     : chain_strided(wr + 64 * c0 * wstep, wstep, xr + 64 * c0,
                                                     min(64 * nch, K - 64 * c0));
             if (zero && xm == 0) *o = 0.0f;  // an activation row of +-0
-            // Zeros of the other rows: +0 where the weight row holds only +-0, else the chain.
-            for (int gq = 0; gq < 4; ++gq) {
-                const bool ask = zero && xm != 0 && g == gq;
-                const uint64_t who = __builtin_amdgcn_ballot_w64(ask);
-                if (who == 0) continue;
-                const uint16_t *const wu = readlane_ptr(wr, __builtin_ctzll(who));
-                const bool nz = SRC == kSrcPacked ? wave_row_nonzero(wu, K / 8, 0x7fff7fffu)
-                                               : wave_weights_nonzero(wu, wstep, K);
-                const float v = wave_chains<MT == 16 ? 2 : 4>(ask && nz, 0.0f, wr, wstep, xr, K);
-                if (ask) *o = v;
-            }
+            const bool ask = zero && xm != 0;
+            if (__builtin_amdgcn_ballot_w64(ask) != 0) settle_zeros(o, ask ? 1u : 0u, xr, wr, 0, wstep, K);
         }
     }
     // Outputs that are not finite: a weight or an activation is inf or NaN
@@ -583,10 +562,9 @@ gemm_sum_slices_kernel(const float *__restrict__ P, int slices, float *__restric
         W += blockIdx.y * w_batch;
         X += blockIdx.y * x_batch;
     }
-    for (int64_t i0 = Q * ((int64_t)blockIdx.x * 256 + threadIdx.x / 64 * 64); i0 < count;
-         i0 += Q * (int64_t)gridDim.x * 256) {  // wave-uniform
-        const int64_t own = i0 + Q * (threadIdx.x & 63);
-        const int64_t i = own < count ? own : count - Q;  // lanes past the end repeat the last outputs
+    const int64_t first = Q * ((int64_t)blockIdx.x * 256 + threadIdx.x), step = Q * (int64_t)gridDim.x * 256;
+    bool zero = false;
+    for (int64_t i = first; i < count; i += step) {
         vec s = *reinterpret_cast<const vec *>(P + i);
         float lost[Q] = {};  // !PACKED: what the sum's roundings lost
 #pragma unroll 8
@@ -607,36 +585,22 @@ gemm_sum_slices_kernel(const float *__restrict__ P, int slices, float *__restric
 #pragma unroll
             for (int e = 0; e < Q; ++e) s[e] = add_lost(s[e], lost[e]);
         }
-        bool zero = false;
+        *reinterpret_cast<vec *>(Y + i) = s;
 #pragma unroll
         for (int e = 0; e < Q; ++e) zero |= s[e] == 0.0f;
-        // Rare: the wave settles its lanes' zeros together, each activation row scanned once.
-        if (__builtin_amdgcn_ballot_w64(zero) != 0) {
-            const int m = (int)(i / N), n = (int)(i - (int64_t)m * N);
-            bool xnz = false;
-            for (uint64_t todo = __builtin_amdgcn_ballot_w64(zero); todo;) {
-                const int mj = __builtin_amdgcn_readlane(m, __builtin_ctzll(todo));
-                const float *const xr = X + (int64_t)mj * K;
-                const bool nz = PACKED ? wave_row_nonzero(xr, K / 4, 0x7fffffffu) : wave_any_product(xr, nullptr, 0, K);
-                const bool same = zero && m == mj;
-                if (same) xnz = nz;
-                todo &= ~__builtin_amdgcn_ballot_w64(same);
-            }
+    }
+    // Rare: the wave settles its lanes' zeros together, over the outputs again.
+    if (__builtin_amdgcn_ballot_w64(zero) == 0) return;
+#pragma nounroll
+    for (int64_t i = first; __builtin_amdgcn_ballot_w64(i < count) != 0; i += step) {
+        const int64_t at = i < count ? i : 0;
+        const vec s = *reinterpret_cast<const vec *>(Y + at);
+        uint32_t zeros = 0;
 #pragma unroll
-            for (int e = 0; e < Q; ++e) {
-                const bool z = s[e] == 0.0f;
-                const uint16_t *const w = W + (int64_t)(n + e) * (wstep == 1 ? K : 1);
-                bool chain = false;
-                for (uint64_t todo = __builtin_amdgcn_ballot_w64(z && xnz); todo; todo &= todo - 1) {
-                    const int j = __builtin_ctzll(todo);
-                    const uint16_t *const wu = readlane_ptr(w, j);
-                    const bool nz = PACKED ? wave_row_nonzero(wu, K / 8, 0x7fff7fffu) : wave_weights_nonzero(wu, wstep, K);
-                    if ((int)(threadIdx.x & 63) == j) chain = nz;
-                }
-                s[e] = wave_chains<2>(chain, z ? 0.0f : s[e], w, wstep, X + (int64_t)m * K, K);
-            }
-        }
-        *reinterpret_cast<vec *>(Y + i) = s;
+        for (int e = 0; e < Q; ++e) zeros |= (i < count && s[e] == 0.0f ? 1u : 0u) << e;
+        const int64_t m = at / N, n = at - m * N;
+        if (__builtin_amdgcn_ballot_w64(zeros != 0) != 0)
+            settle_zeros(Y + at, zeros, X + m * K, W + n * (wstep == 1 ? K : 1), wstep == 1 ? K : 1, wstep, K);
     }
 }
 

@@ -148,172 +148,12 @@ __device__ bool wave_any_product(const float *x, const uint16_t *w, int64_t wste
     return false;
 }
 
-// The reference chain of one output by a whole wave (w, wstep, x, K wave-
-// uniform; wstep <= 1 means packed weights): the lanes load 512 elements at a
-// time, 8 each, the next 512 while these are summed, and the accumulator goes
-// from lane to lane, 8 dependent fmas and one readlane per lane.  A lane on
-// its own waits for memory every 8 elements: the chain of one output of
-// K = 14336 took 560 us that way, against 45 us here.  An exact zero from
-// ordinary data (full cancellation) is rare per output, ~3e-8, but a prefill
-// has millions of outputs: a few calls in a hundred at 1M, one in four at 8M.
-// Elements past K multiply +0 by -0: adding -0 keeps the accumulator.
-__device__ __forceinline__ float wave_chain(const uint16_t *w, int64_t wstep, const float *x, int K) {
-    const int lane = threadIdx.x & 63;
-    if (K <= 0) return 0.0f;
-    const bool packed = wstep <= 1 && K <= (1 << 28);
-    const uintptr_t wb = reinterpret_cast<uintptr_t>(w);
-    const uint32_t wd = packed ? (uint32_t)(wb & 3) : 0;  // 0 or 2
-    const __amdgpu_buffer_rsrc_t xr = weight_rsrc(x, packed ? (uint32_t)K * 4u : 0u);
-    const __amdgpu_buffer_rsrc_t wr =
-        weight_rsrc(reinterpret_cast<const void *>(wb - wd), packed ? wd + 2u * (uint32_t)K : 0u);
-    const uint32_t wlast = w[(int64_t)(K - 1) * wstep];  // its dword may straddle the range's end
-    struct Block {
-        float x[8], w[8];
-    };
-    auto load = [&](int k0, Block &b) {
-        const int e0 = k0 + lane * 8;
-        if (packed) {
-            const u32x4 xa = __builtin_amdgcn_raw_buffer_load_b128(xr, (uint32_t)e0 * 4u, 0, 0);
-            const u32x4 xc = __builtin_amdgcn_raw_buffer_load_b128(xr, (uint32_t)e0 * 4u + 16u, 0, 0);
-            const u32x4 wv = __builtin_amdgcn_raw_buffer_load_b128(wr, wd + (uint32_t)e0 * 2u, 0, 0);
-#pragma unroll
-            for (int e = 0; e < 8; ++e) {
-                b.x[e] = __uint_as_float(e < 4 ? xa[e] : xc[e - 4]);
-                uint32_t bits = (wv[e >> 1] >> (16 * (e & 1))) & 0xffffu;
-                bits = e0 + e == K - 1 ? wlast : bits;
-                b.w[e] = __uint_as_float((e0 + e < K ? bits : 0x8000u) << 16);
-            }
-        } else {
-#pragma unroll
-            for (int e = 0; e < 8; ++e) {
-                const int k = min(e0 + e, K - 1);
-                b.x[e] = e0 + e < K ? x[k] : 0.0f;
-                b.w[e] = __uint_as_float((e0 + e < K ? (uint32_t)w[(int64_t)k * wstep] : 0x8000u) << 16);
-            }
-        }
-    };
-    float acc = 0.0f;
-    Block cur, next;
-    load(0, cur);
-    for (int k0 = 0; k0 < K; k0 += 512) {
-        load(min(k0 + 512, K), next);
-        const int n = min(64, (K - k0 + 7) / 8);
-        for (int l = 0; l < n; ++l) {
-            float t = acc;
-#pragma unroll
-            for (int e = 0; e < 8; ++e) t = fmaf(cur.x[e], cur.w[e], t);
-            acc = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(t), l));
-        }
-        cur = next;
-    }
-    return acc;
-}
-
-// Wave-uniform, for an output whose split sum is exactly zero: is it settled
-// that +0 stands for the reference chain?  A product x * w is a multiple of
-// 2^(ex + ew - 284) (biased exponents; 23 and 7 fraction bits).  Where that is
-// at least 2^-149 for the least nonzero |x| and |w| of the two rows, every sum
-// of the chain is a multiple of the least subnormal, none underflows, and a
-// chain that ends at zero ends at +0 (an exact cancellation, or it never left
-// +0).  And where K products of the greatest |x| and |w| cannot reach inf, nor
-// can the chain on its way (|x| < 2^(ex - 126), |w| < 2^(ew - 126), and its
-// roundings grow a sum less than 4-fold up to K = 2^24).  So +0 is the answer
-// where the reference is zero, and where its roundings leave a residue, +0 is
-// as close to the exact sum as any other order's.  One pass over the rows,
-// against the chain's K dependent steps (4 us against 31 at K = 14336).
-template <int U>  // 512 * U elements a round: 12 registers each
-__device__ __forceinline__ bool wave_zero_is_plus(const uint16_t *w, int64_t wstep, const float *x, int K) {
-    const int lane = threadIdx.x & 63;
-    if (K <= 0) return true;
-    if (K > 1 << 24) return false;
-    const uint32_t wl = (uint32_t)w[(int64_t)(K - 1) * wstep] & 0x7fffu;
-    // least magnitude - 1 (zeros on top), greatest magnitude
-    uint32_t xm = ~0u, wm = wl - 1u, xt = 0, wt = wl;
-    auto put_x = [&](uint32_t v) {
-        v &= 0x7fffffffu;
-        xm = min(xm, v - 1u);
-        xt = max(xt, v);
-    };
-    auto put_w = [&](uint32_t v) {
-        v &= 0x7fffu;
-        wm = min(wm, v - 1u);
-        wt = max(wt, v);
-    };
-    if (wstep <= 1) {
-        const uintptr_t wb = reinterpret_cast<uintptr_t>(w);
-        const uint32_t wd = (uint32_t)(wb & 3);
-        const __amdgpu_buffer_rsrc_t xr = weight_rsrc(x, (uint32_t)K * 4u);  // past K: zeros, which do not count
-        const __amdgpu_buffer_rsrc_t wr = weight_rsrc(reinterpret_cast<const void *>(wb - wd), wd + 2u * (uint32_t)K);
-        for (int k0 = 0; k0 < K; k0 += 512 * U) {
-            u32x4 xa[U], xc[U], wv[U];
-#pragma unroll
-            for (int u = 0; u < U; ++u) {
-                const uint32_t e = (uint32_t)(k0 + (u * 64 + lane) * 8);
-                xa[u] = __builtin_amdgcn_raw_buffer_load_b128(xr, e * 4u, 0, 0);
-                xc[u] = __builtin_amdgcn_raw_buffer_load_b128(xr, e * 4u + 16u, 0, 0);
-                wv[u] = __builtin_amdgcn_raw_buffer_load_b128(wr, wd + e * 2u, 0, 0);
-            }
-#pragma unroll
-            for (int u = 0; u < U; ++u)
-#pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    put_x(xa[u][i]);
-                    put_x(xc[u][i]);
-                    put_w(wv[u][i]);
-                    put_w(wv[u][i] >> 16);
-                }
-        }
-    } else {
-        for (int k0 = 0; k0 < K; k0 += 64 * U) {
-#pragma unroll
-            for (int u = 0; u < U; ++u) {
-                const int k = min(k0 + u * 64 + lane, K - 1);
-                put_x(__float_as_uint(x[k]));
-                put_w((uint32_t)w[(int64_t)k * wstep]);
-            }
-        }
-    }
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) {
-        xm = min(xm, (uint32_t)__shfl_xor((int)xm, o));
-        wm = min(wm, (uint32_t)__shfl_xor((int)wm, o));
-        xt = max(xt, (uint32_t)__shfl_xor((int)xt, o));
-        wt = max(wt, (uint32_t)__shfl_xor((int)wt, o));
-    }
-    const uint32_t ex = (xm + 1) >> 23, ew = (wm + 1) >> 7;
-    const uint32_t lg = 32 - __builtin_clz((uint32_t)K);  // K < 2^lg
-    return xt == 0 || wt == 0 || (ex >= 1 && ew >= 1 && ex + ew >= 135 && (xt >> 23) + (wt >> 7) + lg <= 377);
-}
-
-// The reference's values for the lanes whose sums are exactly zero (`ask`; w, x
-// per lane): +0 where it cannot be -0, else the chain, a few one after another
-// by the whole wave, many one per lane.  U = 0: the chain always (the FMA
-// kernels, whose outputs are few and whose registers are full).
-template <int U>
-__device__ __forceinline__ float wave_chains(bool ask, float s, const uint16_t *w, int64_t wstep, const float *x, int K) {
-    uint64_t chains = U > 0 ? 0 : __builtin_amdgcn_ballot_w64(ask);
-    if constexpr (U > 0) for (uint64_t todo = __builtin_amdgcn_ballot_w64(ask); todo; todo &= todo - 1) {
-        const int j = __builtin_ctzll(todo);
-        if (wave_zero_is_plus<U>(readlane_ptr(w, j), wstep, readlane_ptr(x, j), K)) {
-            if ((int)(threadIdx.x & 63) == j) s = 0.0f;
-        } else {
-            chains |= 1ull << j;
-        }
-    }
-    if (__builtin_popcountll(chains) > 6) return (chains >> (threadIdx.x & 63)) & 1 ? chain_strided(w, wstep, x, K) : s;
-    for (; chains; chains &= chains - 1) {
-        const int j = __builtin_ctzll(chains);
-        const float v = wave_chain(readlane_ptr(w, j), wstep, readlane_ptr(x, j), K);
-        if ((int)(threadIdx.x & 63) == j) s = v;
-    }
-    return s;
-}
-
-// The zero rule for the outputs this wave holds, one per lane: `zero` marks a
-// lane whose output s is exactly 0 and is stored; x is its activation row,
-// w its first weight, wstep the elements between consecutive k.  All 64 lanes
-// call it (wave-uniform control flow): rows are scanned by the whole wave,
-// one output at a time, and the chains (if any) run one per lane.
+// The zero rule for the general row-dot kernel's outputs this wave holds, one
+// per lane: `zero` marks a lane whose output s is exactly 0 and is stored; x is
+// its activation row, w its first weight, wstep the elements between
+// consecutive k.  All 64 lanes call it (wave-uniform control flow): rows are
+// scanned by the whole wave, one output at a time, and the chains (if any) run
+// one per lane.
 __device__ float settle_zero(float s, bool zero, const float *x, const uint16_t *w, int64_t wstep, int K) {
     uint64_t pend = __builtin_amdgcn_ballot_w64(zero);
     if (pend == 0) return s;
@@ -336,7 +176,203 @@ __device__ float settle_zero(float s, bool zero, const float *x, const uint16_t 
         const bool hit = wave_any_product(readlane_ptr(x, j), readlane_ptr(w, j), wstep, K);
         if (lane == j) chain = hit;
     }
-    return wave_chains<0>(chain, zero ? 0.0f : s, w, wstep, x, K);
+    if (zero) s = chain ? chain_strided(w, wstep, x, K) : 0.0f;
+    return s;
+}
+
+// ---- zero outputs of the MFMA kernels ------------------------------------------
+//
+// Out of the kernels' code (settle_zeros is not inlined): expanded at their
+// unrolled outputs, this rare path set their registers (gemm_sum_slices_kernel:
+// 149 VGPRs, 3 waves per SIMD, and 199 SGPRs spilled, against 8 waves and none).
+
+// Least and greatest magnitude of a row: lo - 1 (zeros wrap to the top), hi.
+struct Range {
+    uint32_t lo1 = ~0u, hi = 0;
+    __device__ __forceinline__ void put(uint32_t v) {
+        lo1 = min(lo1, v - 1u);
+        hi = max(hi, v);
+    }
+    __device__ __forceinline__ void over_wave() {
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1) {
+            lo1 = min(lo1, (uint32_t)__shfl_xor((int)lo1, o));
+            hi = max(hi, (uint32_t)__shfl_xor((int)hi, o));
+        }
+    }
+};
+
+// The wave's ranges of an activation row and of a weight row or column, K <=
+// 2^24, 16-byte loads at the rows' own alignments (exact on gfx950; a dword past
+// the row's end comes back as zeros, which do not count, and the last weight,
+// which may share one, is read alone).
+__device__ __noinline__ Range wave_range(const float *x, int K) {
+    Range r;
+    const __amdgpu_buffer_rsrc_t xr = weight_rsrc(x, (uint32_t)K * 4u);
+#pragma nounroll
+    for (int k0 = 0; k0 < K; k0 += 1024) {
+        u32x4 v[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+            v[u] = __builtin_amdgcn_raw_buffer_load_b128(xr, (uint32_t)(k0 + (u * 64 + (threadIdx.x & 63)) * 4) * 4u, 0, 0);
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) r.put(v[u][i] & 0x7fffffffu);
+    }
+    r.over_wave();
+    return r;
+}
+
+__device__ __noinline__ Range wave_range(const uint16_t *w, int64_t wstep, int K) {
+    const int lane = threadIdx.x & 63;
+    Range r;
+    r.put((uint32_t)w[(int64_t)(K - 1) * wstep] & 0x7fffu);
+    if (wstep <= 1) {
+        const uintptr_t wb = reinterpret_cast<uintptr_t>(w);
+        const uint32_t wd = (uint32_t)(wb & 3);
+        const __amdgpu_buffer_rsrc_t wr = weight_rsrc(reinterpret_cast<const void *>(wb - wd), wd + 2u * (uint32_t)K);
+#pragma nounroll
+        for (int k0 = 0; k0 < K; k0 += 2048) {
+            u32x4 v[4];
+#pragma unroll
+            for (int u = 0; u < 4; ++u)
+                v[u] = __builtin_amdgcn_raw_buffer_load_b128(wr, wd + (uint32_t)(k0 + (u * 64 + lane) * 8) * 2u, 0, 0);
+#pragma unroll
+            for (int u = 0; u < 4; ++u)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    r.put(v[u][i] & 0x7fffu);
+                    r.put(v[u][i] >> 16 & 0x7fffu);
+                }
+        }
+    } else {
+#pragma nounroll
+        for (int k0 = 0; k0 < K; k0 += 64 * 8) {
+            uint32_t v[8];
+#pragma unroll
+            for (int u = 0; u < 8; ++u) v[u] = w[(int64_t)min(k0 + u * 64 + lane, K - 1) * wstep];
+#pragma unroll
+            for (int u = 0; u < 8; ++u) r.put(v[u] & 0x7fffu);
+        }
+    }
+    r.over_wave();
+    return r;
+}
+
+// For an output whose split sum is exactly zero, from the ranges of its two
+// rows: is it settled that +0 stands for the reference chain?  A product x * w
+// is a multiple of 2^(ex + ew - 284) (biased exponents; 23 and 7 fraction bits).
+// Where that is at least 2^-149 for the least nonzero |x| and |w|, every sum of
+// the chain is a multiple of the least subnormal, none underflows, and a chain
+// that ends at zero ends at +0 (an exact cancellation, or it never left +0).
+// And where K products of the greatest |x| and |w| cannot reach inf, nor can
+// the chain on its way (|x| < 2^(ex - 126), |w| < 2^(ew - 126), and its
+// roundings grow a sum less than 4-fold up to K = 2^24).  So +0 is the answer
+// where the reference is zero, and where its roundings leave a residue, +0 is
+// as close to the exact sum as any other order's.
+__device__ __forceinline__ bool zero_is_plus(const Range &x, const Range &w, int K) {
+    const uint32_t ex = (x.lo1 + 1) >> 23, ew = (w.lo1 + 1) >> 7;
+    const uint32_t lg = 32 - __builtin_clz((uint32_t)K);  // K < 2^lg
+    return x.hi == 0 || w.hi == 0 ||
+           (ex >= 1 && ew >= 1 && ex + ew >= 135 && (x.hi >> 23) + (w.hi >> 7) + lg <= 377);
+}
+
+// The reference chain of one output by a whole wave (w, x, K wave-uniform;
+// packed weights, K <= 2^24): the lanes load 512 elements at a time, 8 each, the
+// next 512 while these are summed, and the accumulator goes from lane to lane, 8
+// dependent fmas and one readlane per lane.  A lane on its own waits for memory
+// every 8 elements: the chain of one output of K = 14336 took 560 us that way,
+// against 31 us here.  Elements past K multiply +0 by -0: adding -0 keeps the
+// accumulator.
+__device__ __noinline__ float wave_chain(const uint16_t *w, const float *x, int K) {
+    const int lane = threadIdx.x & 63;
+    const uintptr_t wb = reinterpret_cast<uintptr_t>(w);
+    const uint32_t wd = (uint32_t)(wb & 3);  // 0 or 2
+    const __amdgpu_buffer_rsrc_t xr = weight_rsrc(x, (uint32_t)K * 4u);
+    const __amdgpu_buffer_rsrc_t wr = weight_rsrc(reinterpret_cast<const void *>(wb - wd), wd + 2u * (uint32_t)K);
+    const uint32_t wlast = w[K - 1];  // its dword may straddle the range's end
+    u32x4 x0, x1, wv, nx0, nx1, nwv;
+    auto load = [&](int k0) __attribute__((always_inline)) {
+        const uint32_t e0 = (uint32_t)(k0 + lane * 8);
+        nx0 = __builtin_amdgcn_raw_buffer_load_b128(xr, e0 * 4u, 0, 0);
+        nx1 = __builtin_amdgcn_raw_buffer_load_b128(xr, e0 * 4u + 16u, 0, 0);
+        nwv = __builtin_amdgcn_raw_buffer_load_b128(wr, wd + e0 * 2u, 0, 0);
+    };
+    float acc = 0.0f;
+    load(0);
+#pragma nounroll
+    for (int k0 = 0; k0 < K; k0 += 512) {
+        x0 = nx0, x1 = nx1, wv = nwv;
+        load(k0 + 512);
+        const int left = K - k0 - lane * 8;  // elements of this lane's 8 (x past K is 0)
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+            const uint32_t lo = 2 * v >= left ? 0x8000u : 2 * v + 1 == left ? wlast : wv[v] & 0xffffu;
+            const uint32_t hi = 2 * v + 1 >= left ? 0x8000u : 2 * v + 2 == left ? wlast : wv[v] >> 16;
+            wv[v] = lo | hi << 16;
+        }
+        const int n = min(64, (K - k0 + 7) / 8);
+#pragma nounroll
+        for (int l = 0; l < n; ++l) {
+            float t = acc;
+#pragma unroll
+            for (int e = 0; e < 8; ++e)
+                t = fmaf(__uint_as_float(e < 4 ? x0[e] : x1[e - 4]), e & 1 ? widen_hi(wv[e >> 1]) : widen_lo(wv[e >> 1]),
+                         t);
+            acc = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(t), l));
+        }
+    }
+    return acc;
+}
+
+// One per lane.
+__device__ __noinline__ float lane_chain(const uint16_t *w, int64_t wstep, const float *x, int K) {
+    return chain_strided(w, wstep, x, K);
+}
+
+// The reference's values for outputs whose sums are exactly zero: a lane's are
+// y[e] where bit e of `zeros` is set (e < 4), of its activation row x and the
+// weights w + e * wpitch, wstep elements between consecutive k.  All 64 lanes
+// call this.  The ranges of each distinct activation and weight row are taken
+// once by the whole wave and settle almost every zero (zero_is_plus); the chains
+// left, if any, run one after another by the whole wave where they are few and
+// the weights packed, else one per lane.
+__device__ __forceinline__ void settle_zeros(float *y, uint32_t zeros, const float *x, const uint16_t *w, int64_t wpitch,
+                                          int64_t wstep, int K) {
+    const bool ranges = K <= 1 << 24;
+    Range rx;
+    if (ranges)
+        for (uint64_t todo = __builtin_amdgcn_ballot_w64(zeros != 0); todo;) {
+            const float *const xj = readlane_ptr(x, __builtin_ctzll(todo));
+            const Range r = wave_range(xj, K);
+            if (x == xj) rx = r;
+            todo &= ~__builtin_amdgcn_ballot_w64(x == xj);
+        }
+#pragma nounroll
+    for (int e = 0; e < 4; ++e, w += wpitch) {
+        const bool zero = (zeros >> e & 1) != 0;
+        bool plus = ranges && rx.hi == 0;  // an activation row of +-0
+        if (ranges)
+            for (uint64_t todo = __builtin_amdgcn_ballot_w64(zero && !plus); todo;) {
+                const uint16_t *const wj = readlane_ptr(w, __builtin_ctzll(todo));
+                const Range r = wave_range(wj, wstep, K);
+                if (w == wj) plus |= zero_is_plus(rx, r, K);
+                todo &= ~__builtin_amdgcn_ballot_w64(w == wj);
+            }
+        float v = 0.0f;
+        uint64_t chains = __builtin_amdgcn_ballot_w64(zero && !plus);
+        if (wstep > 1 || !ranges || __builtin_popcountll(chains) > 6) {
+            if (zero && !plus) v = lane_chain(w, wstep, x, K);
+        } else {
+            for (; chains; chains &= chains - 1) {
+                const int j = __builtin_ctzll(chains);
+                const float c = wave_chain(readlane_ptr(w, j), readlane_ptr(x, j), K);
+                if ((int)(threadIdx.x & 63) == j) v = c;
+            }
+        }
+        if (zero) y[e] = v;
+    }
 }
 
 // ---- RD skinny M on MFMA: W [N,K] x X [M,K], K % 64 == 0 ---------------------------
@@ -363,10 +399,9 @@ __device__ float settle_zero(float s, bool zero, const float *x, const uint16_t 
 // Zeros: the MFMA rounds a nonzero sum smaller than half the least f32
 // subnormal to +0 whatever its sign, where the reference's fmaf gives the
 // signed zero (every product underflowing negative ends at -0).  So an output
-// that comes out exactly zero is settled by the reference's own rule: +0 when
-// its activation row or its weight row holds only zeros (every product is an
-// exact zero and the chain never leaves +0), otherwise the chain itself,
-// fmaf over ascending k from +0 (rare: underflow or exact cancellation).
+// that comes out exactly zero is settled at the end (settle_zeros above): +0
+// where the two rows' magnitudes leave the chain no room to underflow or
+// overflow, otherwise the chain itself, fmaf over ascending k from +0.
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
@@ -500,68 +535,6 @@ constexpr uint32_t kTinyHiBits = 0x0d80u;
 
 __device__ __forceinline__ uint32_t hi_max(uint32_t mx) { return max(mx & 0xffffu, mx >> 16); }
 __device__ __forceinline__ bool tiny_row(uint32_t mx) { return mx != 0 && mx < kTinyHiBits; }
-
-// Wave-uniform: does the row hold an element other than +-0?  (bytes: 16 * n16)
-__device__ bool wave_row_nonzero(const void *row, int n16, uint32_t mask) {
-    const u32x4 *p = reinterpret_cast<const u32x4 *>(row);
-    uint32_t acc = 0;
-    for (int c = threadIdx.x & 63; c < n16; c += 64) {
-        const u32x4 v = p[c];
-        acc |= (v[0] | v[1] | v[2] | v[3]) & mask;
-    }
-    return __builtin_amdgcn_ballot_w64(acc != 0) != 0;
-}
-
-// One wave's outputs after the zero rule above.  Lane l holds s[t][r] for
-// weight row base[t] + 4(l/16) + r of W and activation row m of X; `live`
-// marks the ones it stores.  All 64 lanes call this; the rows are walked
-// wave-uniformly.  Rare path: entered only when some output is exactly zero.
-template <int T>
-__device__ void settle_zeros(f32x4 (&s)[T], const bool (&live)[T][4], const int (&base)[T], const uint16_t *W,
-                             const float *X, int K, int m) {
-    const int g = (threadIdx.x & 63) >> 4;
-    bool zero[T][4];
-    bool any = false;
-#pragma unroll
-    for (int t = 0; t < T; ++t)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            zero[t][r] = live[t][r] && s[t][r] == 0.0f;
-            any |= zero[t][r];
-        }
-    if (__builtin_amdgcn_ballot_w64(any) == 0) return;
-    // Is this lane's activation row nonzero?  Lanes j = 0..15 hold every row
-    // the wave has.
-    bool xnz = false;
-    for (int j = 0; j < 16; ++j) {
-        const int mj = __builtin_amdgcn_readlane(m, j);
-        if (__builtin_amdgcn_ballot_w64(any && m == mj) != 0) {
-            const bool nz = wave_row_nonzero(X + (int64_t)mj * K, K / 4, 0x7fffffffu);
-            if (m == mj) xnz = nz;
-        }
-    }
-    // Zero outputs become +0, or the chain's value where both rows are nonzero.
-    bool chain[T][4];
-#pragma unroll
-    for (int t = 0; t < T; ++t)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            chain[t][r] = false;
-            if (zero[t][r]) s[t][r] = 0.0f;
-            for (int gq = 0; gq < 4; ++gq) {
-                const bool ask = zero[t][r] && xnz && g == gq;
-                if (__builtin_amdgcn_ballot_w64(ask) == 0) continue;
-                const int row = base[t] + 4 * gq + r;
-                const bool nz = wave_row_nonzero(W + (int64_t)row * K, K / 8, 0x7fff7fffu);
-                if (ask) chain[t][r] = nz;
-            }
-        }
-#pragma unroll
-    for (int t = 0; t < T; ++t)
-#pragma unroll
-        for (int r = 0; r < 4; ++r)
-            s[t][r] = wave_chains<2>(chain[t][r], s[t][r], W + (int64_t)(base[t] + 4 * g + r) * K, 1, X + (int64_t)m * K, K);
-}
 
 // Weight and x tiles in LDS hold rows of 128 bytes, 8 pieces of 16, back to
 // back, with piece p of row r stored at position p ^ ((r / 2) mod 8).  A
