@@ -57,7 +57,9 @@ namespace {
 // 7e-7).  They keep that: every k-block of 32 is summed from zero (lo, mid, hi:
 // one rounding at full size), the blocks are added up in f32, and those sums
 // once more every `fold` chunks, these and the k slices with the rounding
-// errors of their sums kept.
+// errors of their sums kept.  And they keep x's 24 bits where three bf16 terms
+// do not, |x| < 2^-110: a tile that holds such elements is streamed once more for
+// what the terms left (kRest).
 //
 // When the tiles would leave the device short of workgroups, k is split over
 // `slices` workgroups of kc chunks each, whose partial sums go to
@@ -70,9 +72,13 @@ enum Src { kSrcPacked, kSrcRows, kSrcCols };
 constexpr uint32_t kDeadChunk = 0x7fff0000u;  // scalar offset of a chunk past the last (no 32-bit wrap with kDeadLane)
 
 // The three bf16 terms of eight values by truncation alone: split3's terms for
-// every finite |x| >= 2^-133 and 0.  Of a smaller x nothing is left, and an inf
-// leaves a NaN in mid: rows that hold those are settled after the stream.
-__device__ __forceinline__ void split8_finite(const float (&v)[8], u32x4 (&t)[3]) {
+// every finite |x| >= 2^-133 and 0.  Of a smaller x nothing is left, which
+// matters where the row is not large either (tiny rows, settled after the
+// stream) and where its larger elements meet weights of 0 or the small ones
+// large weights: `cut` collects, in its low half, whether any element had more
+// than the terms hold (kRest below).  An inf leaves a NaN in mid: settled after
+// the stream too.
+__device__ __forceinline__ void split8_finite(const float (&v)[8], u32x4 (&t)[3], uint32_t &cut) {
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
         const uint32_t u0 = __float_as_uint(v[2 * q]), u1 = __float_as_uint(v[2 * q + 1]);
@@ -84,6 +90,28 @@ __device__ __forceinline__ void split8_finite(const float (&v)[8], u32x4 (&t)[3]
         t[0][q] = (u0 >> 16) | (u1 & 0xffff0000u);
         t[1][q] = (b10 >> 16) | (b11 & 0xffff0000u);
         t[2][q] = (b20 >> 16) | (b21 & 0xffff0000u);
+        cut |= b20 | b21;
+    }
+}
+
+// What three terms leave of eight values, times 2^64: nothing of |x| >= 2^-110,
+// else a multiple of 2^-85 under 2^-69, 16 bits, which two terms hold exactly.
+__device__ __forceinline__ void split8_rest(const float (&v)[8], u32x4 (&t)[3]) {
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+        uint32_t h[2], m[2];
+#pragma unroll
+        for (int e = 0; e < 2; ++e) {
+            float r = v[2 * q + e];
+            const bool fin = (__float_as_uint(r) & 0x7f800000u) != 0x7f800000u;
+#pragma unroll
+            for (int i = 0; i < 3; ++i) r -= __uint_as_float(__float_as_uint(r) & 0xffff0000u);
+            r = fin ? r * 0x1p64f : 0.0f;
+            h[e] = __float_as_uint(r) & 0xffff0000u;
+            m[e] = __float_as_uint(r - __uint_as_float(h[e]));
+        }
+        t[0][q] = (h[0] >> 16) | h[1];
+        t[1][q] = (m[0] >> 16) | (m[1] & 0xffff0000u);
     }
 }
 
@@ -102,6 +130,10 @@ __device__ __forceinline__ float add_exact(float &s, float p) {
 }
 // (Sums that are not finite have no meaningful loss.)
 __device__ __forceinline__ float add_lost(float s, float e) { return fabsf(s) < __builtin_inff() ? s + e : s; }
+
+// Passes over the tile: the products (three terms), what the terms leave of x
+// (two, times 2^64), and the hi term alone (the classes of what is not finite).
+constexpr int kAll = 3, kRest = 2, kHi = 1;
 
 template <int NWV, int MT, int SRC, bool FUSE>
 __global__ void __launch_bounds__(64 * NWV) __attribute__((amdgpu_waves_per_eu(MT == 16 && SRC == kSrcPacked ? 4 : 2)))
@@ -223,6 +255,7 @@ gemv_mfma_gemm_kernel(const uint16_t *__restrict__ W, const float *__restrict__ 
     uint32_t xmx[XI];  // the largest |x| staged (f32 bits; the hi term's with planes), per lane
 #pragma unroll
     for (int j = 0; j < XI; ++j) xmx[j] = 0;
+    uint32_t cut = 0;
     // Chunk c's staged registers into LDS buffer `buf`.
     auto store = [&](Regs &r, int c, int buf, auto TERMS) __attribute__((always_inline)) {
         constexpr int terms = decltype(TERMS)::value;
@@ -285,17 +318,19 @@ gemv_mfma_gemm_kernel(const uint16_t *__restrict__ W, const float *__restrict__ 
                     v[e] = __uint_as_float(r.x[j][0][e]);
                     v[4 + e] = __uint_as_float(r.x[j][1][e]);
                 }
-                if constexpr (terms == 1) {
+                if constexpr (terms == kHi) {
                     split8(v, t[0], t[1], t[2]);
+                } else if constexpr (terms == kRest) {
+                    split8_rest(v, t);
                 } else {
-                    split8_finite(v, t);
+                    split8_finite(v, t, cut);
 #pragma unroll
                     for (int e = 0; e < 8; ++e) xmx[j] = max(xmx[j], __float_as_uint(v[e]) & 0x7fffffffu);
                 }
             } else {
 #pragma unroll
                 for (int q = 0; q < 3; ++q) t[q] = r.x[j][q];
-                if constexpr (terms == 3) {
+                if constexpr (terms == kAll) {
 #pragma unroll
                     for (int e = 0; e < 4; ++e) xmx[j] = max_mag(xmx[j], t[0][e]);
                 }
@@ -422,31 +457,112 @@ gemv_mfma_gemm_kernel(const uint16_t *__restrict__ W, const float *__restrict__ 
                     for (int v = 0; v < 4; ++v) acc[i][j][v] = add_lost(total[i][j][v], lost[i][j][v]);
         }
     };
+    // The pass over what the terms left of x, rare: one LDS buffer and one set of
+    // operands (registers), the next chunk's loads under this one's MFMAs.
+    auto stream_rest = [&]() __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < RM; ++i)
+#pragma unroll
+            for (int j = 0; j < RN; ++j)
+#pragma unroll
+                for (int v = 0; v < 4; ++v) total[i][j][v] = lost[i][j][v] = part[i][j][v] = 0.0f;
+        load(0, r);
+        int until = fold;
+#pragma nounroll
+        for (int c = 0; c < nch; ++c) {
+            lds_barrier();  // every wave is done with the buffer
+            store(r, c, 0, std::integral_constant<int, kRest>{});
+            load(c + 1, r);
+            lds_barrier();
+#pragma unroll
+            for (int kb = 0; kb < 2; ++kb) {
+                read_a(0, kb);
+#pragma unroll
+                for (int mf = 0; mf < RM; ++mf) {
+                    read_x(0, kb, mf, 0);
+                    f32x4 blk[RN];
+#pragma unroll
+                    for (int j = 0; j < RN; ++j) {
+                        blk[j] = mfma_bf16(a[kb][j], xo[0][1], f32x4{0.0f, 0.0f, 0.0f, 0.0f});
+                        blk[j] = mfma_bf16(a[kb][j], xo[0][0], blk[j]);
+                    }
+#pragma unroll
+                    for (int j = 0; j < RN; ++j)
+#pragma unroll
+                        for (int v = 0; v < 4; ++v) part[mf][j][v] += blk[j][v];
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+            }
+            if (c + 1 >= until) {
+                fold_parts();
+                until = c + 1 + fold;
+            }
+        }
+        fold_parts();
+#pragma unroll
+        for (int i = 0; i < RM; ++i)
+#pragma unroll
+            for (int j = 0; j < RN; ++j)
+#pragma unroll
+                for (int v = 0; v < 4; ++v) acc[i][j][v] = add_lost(total[i][j][v], lost[i][j][v]);
+    };
     // Waves w and w + 4 share a SIMD: they stage (split or transpose, store) in
     // different steps, so that one's vector work runs under the other's MFMAs.
     // Same box, in the same step / staggered, us: C2 up m = 512 168 / 164, down
     // m = 2048 604 / 581, columns up m = 64 47.5 / 44.0; packed 64-row tiles
     // lose 2% where a slice has few chunks (C2 up m = 64 40.2 / 40.7).
     constexpr bool kStagger = MT == 128 || (SRC == kSrcCols && MT == 64);
-    if (!kStagger || wave >= 4) stream(std::integral_constant<int, 3>{}, std::integral_constant<int, NS - 2>{});
-    else stream(std::integral_constant<int, 3>{}, std::integral_constant<int, 0>{});
+    if (!kStagger || wave >= 4) stream(std::integral_constant<int, kAll>{}, std::integral_constant<int, NS - 2>{});
+    else stream(std::integral_constant<int, kAll>{}, std::integral_constant<int, 0>{});
 
+    float *const out = (P ? P + (int64_t)bz * M * N : Y) + row0;
     // The activation rows' largest magnitudes (this slice's k), in LDS bytes
-    // that the stream is done with.
+    // that the stream is done with, and whether the terms left some of x.
     uint32_t *const xmax_s = reinterpret_cast<uint32_t *>(&xp[0][0][0][0][0]);
-    __syncthreads();
-    for (int i = tid; i < MT; i += 64 * NWV) xmax_s[i] = 0;
-    __syncthreads();
+    uint32_t *const any_s = xmax_s + MT;
+    auto row_maxima = [&]() __attribute__((always_inline)) {
+        __syncthreads();
+        for (int i = tid; i <= MT; i += 64 * NWV) xmax_s[i] = 0;
+        __syncthreads();
 #pragma unroll
-    for (int j = 0; j < XI; ++j) {
-        const int it = wave * XI + j;
-        if (it < 2 * XT) atomicMax(&xmax_s[(it >> 1) * 16 + i16], FUSE ? xmx[j] : hi_max(xmx[j]) << 16);
+        for (int j = 0; j < XI; ++j) {
+            const int it = wave * XI + j;
+            if (it < 2 * XT) atomicMax(&xmax_s[(it >> 1) * 16 + i16], FUSE ? xmx[j] : hi_max(xmx[j]) << 16);
+        }
+        if (kTwoLevel && (cut & 0xffffu) != 0) *any_s = 1;
+        __syncthreads();
+    };
+    row_maxima();
+    if constexpr (kTwoLevel) {
+        // Rare: the tile is streamed once more for what the terms left of x, so
+        // that these forms keep the 24 bits that the f32 FMA kernels keep.  With
+        // and without such elements (the FMA kernels the same), us: columns
+        // [4096,14336] m = 5 / 17 / 64 50 / 66 / 100 against 27.7 / 34.2 / 45.0
+        // (61 / 172 / 3680), [11008,4097] m = 3 / 33 42 / 75 against 21.3 / 35.5
+        // (48 / 494).
+        if (*any_s != 0) {
+            auto each = [&](auto body) __attribute__((always_inline)) {
+#pragma unroll
+                for (int f = 0; f < RM * RN * 4; ++f) {
+                    const int mf = f / (RN * 4), j = f / 4 % RN, n = (wn * RN + j) * 16 + g * 4 + f % 4;
+                    const int ml = (wm * RM + mf) * 16 + i16;
+                    if (m0 + ml < M && n < nrows)
+                        acc[mf][j][f % 4] = body(out[(int64_t)(m0 + ml) * N + n], acc[mf][j][f % 4]);
+                }
+            };
+            each([](float &o, float v) { return o = v; });
+            __syncthreads();
+            stream_rest();
+            each([](float &o, float v) {
+                return fabsf(v) < __builtin_inff() && v != 0.0f ? o + v * 0x1p-64f : o;
+            });
+            cut = 0;
+            row_maxima();
+        }
     }
-    __syncthreads();
     // Outputs: lane l holds weight rows 4(l/16) + v of a tile, activation row
     // l%16.  They are stored as they are; the rare ones that the sums do not
     // settle (a tiny row, an exact zero, a value that is not finite) are redone.
-    float *const out = (P ? P + (int64_t)bz * M * N : Y) + row0;
     bool rare = false, big = false;  // big: some output is not finite
 #pragma unroll
     for (int mf = 0; mf < RM; ++mf) {
@@ -501,7 +617,6 @@ gemv_mfma_gemm_kernel(const uint16_t *__restrict__ W, const float *__restrict__ 
     // streamed again with it and those outputs take its result where that is
     // not finite either.  (Screening W in the loop and clearing such weights
     // for mid and lo cost 12-18% of it, for weights that hold none.)
-    uint32_t *const any_s = xmax_s + MT;
     if (tid == 0) *any_s = 0;
     __syncthreads();
     if (big) *any_s = 1;
@@ -509,7 +624,7 @@ gemv_mfma_gemm_kernel(const uint16_t *__restrict__ W, const float *__restrict__ 
     const bool again = *any_s != 0;
     __syncthreads();
     if (!again) return;
-    stream(std::integral_constant<int, 1>{}, std::integral_constant<int, NS - 2>{});
+    stream(std::integral_constant<int, kHi>{}, std::integral_constant<int, NS - 2>{});
 #pragma unroll
     for (int mf = 0; mf < RM; ++mf) {
         const int ml = (wm * RM + mf) * 16 + i16;

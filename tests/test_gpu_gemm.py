@@ -88,6 +88,41 @@ def test_zero_sums_take_the_reference_chain(hip, env, k, columns, monkeypatch):
     check_or_bound(y, y_ref, x, W.bf16_to_f32(w), what="zero sums")
 
 
+@pytest.mark.parametrize("env,k,columns", ROUTES[4:])
+def test_small_elements_beside_large_ones_keep_their_bits(hip, env, k, columns, monkeypatch):
+    """Activation elements down to the least subnormal in rows whose largest
+    element meets a weight of 0, and small elements against large weights: f32
+    keeps all 24 bits of them (three bf16 terms alone lose those under 2^-133)."""
+    m, n = 40, 300
+    for name, value in env.items():
+        monkeypatch.setenv(name, value)
+    rng = np.random.default_rng(11)
+    x, w = case(m, k, n, seed=6, scale=0.02)
+    for r, top in ((3, -112), (17, -125), (33, -136)):
+        x[r] = np.ldexp(rng.standard_normal(k), top).astype(np.float32)
+        x[r, 5] = 1
+    x[34], x[34, 0], x[34, 1] = 0, 1, np.ldexp(np.float32(1), -140)
+    x[35, 9], x[36, 2] = np.inf, np.nan  # whole rows that are not finite, in the same tiles
+    w[::3, 5] = 0
+    w[::3, 6:] = W.bf16_rne(np.ldexp(rng.standard_normal((n + 2) // 3 * (k - 6)), 60).astype(np.float32)).reshape(-1, k - 6)
+    w[7], w[7, 0], w[7, 1] = 0, 0x2180, 0x7F00  # 2^-60 and 2^127: 2^-13 with row 34
+    w[8, 3] = 0x7F80
+    y_ref = oracle.matmul_bf16_t(x, w)
+    assert abs(y_ref[34, 7] - 2.0 ** -13) < 1e-9
+    y = on_route(hip, x, w, columns)
+    wf = W.bf16_to_f32(w)
+    check_classes(y, y_ref, "mixed rows")
+    fin = np.all(np.isfinite(wf), axis=1)
+    for r in np.flatnonzero(np.all(np.isfinite(x), axis=1)):
+        check_bound(y[r, fin], y_ref[r, fin], x[r], wf[fin], what=f"mixed row {r}")
+    for r in (3, 17, 33):  # every product carries the same 24 bits: a few roundings away
+        cols = np.flatnonzero(w[:, 5] == 0)
+        want = wf[cols].astype(np.float64) @ x[r].astype(np.float64)
+        size = np.abs(wf[cols].astype(np.float64)) @ np.abs(x[r].astype(np.float64))
+        # 3 roundings per k-block, at most 12 per sum of blocks, 1 for the small parts
+        assert np.all(np.abs(y[r, cols] - want) <= 16 * 2.0 ** -24 * size + 2.0 ** -148), r
+
+
 def planted(m, k, n, seed):
     """Edge data, with special values, zero rows and underflow where they fit; (x, w [n,k], reference)."""
     x, w = case(m, k, n, seed=seed, edge=True)
