@@ -128,8 +128,10 @@ __device__ __forceinline__ float add_exact(float &s, float p) {
     s = t;
     return e;
 }
-// (Sums that are not finite have no meaningful loss.)
-__device__ __forceinline__ float add_lost(float s, float e) { return fabsf(s) < __builtin_inff() ? s + e : s; }
+// (Sums that are not finite have no meaningful loss, and without one a sum keeps its bits, a -0 too.)
+__device__ __forceinline__ float add_lost(float s, float e) {
+    return fabsf(s) < __builtin_inff() && fabsf(e) > 0.0f ? s + e : s;
+}
 
 // Passes over the tile: the products (three terms), what the terms leave of x
 // (two, times 2^64), and the hi term alone (the classes of what is not finite).
@@ -582,32 +584,140 @@ gemv_mfma_gemm_kernel(const uint16_t *__restrict__ W, const float *__restrict__ 
             }
 #pragma unroll
             for (int v = 0; v < 4; ++v) {
-                rare |= !P && n + v < nrows && acc[mf][j][v] == 0.0f;
+                rare |= n + v < nrows && acc[mf][j][v] == 0.0f;
                 big |= n + v < nrows && !(fabsf(acc[mf][j][v]) < __builtin_inff());
             }
         }
     }
-    if (__builtin_amdgcn_ballot_w64(rare) != 0) {
+    // The lane's outputs of `mask` (bit f, in the order above), some lane's at a
+    // time: body(is it this lane's, activation row of the tile, address, w, x).
+    auto each_output = [&](uint64_t mask, auto body) __attribute__((always_inline)) {
 #pragma nounroll
+        for (int f = 0; f < RM * RN * 4; ++f) {
+            const bool mine = (mask >> f & 1) != 0;
+            if (__builtin_amdgcn_ballot_w64(mine) == 0) continue;
+            const int mf = f / (RN * 4), n = (wn * RN + f / 4 % RN) * 16 + g * 4 + f % 4;
+            const int ml = (wm * RM + mf) * 16 + i16;
+            body(mine, ml, out + (int64_t)(m0 + ml) * N + n, wrow0 + min(n, nrows - 1) * wpitch,
+                 X + (int64_t)min(m0 + ml, M - 1) * K);
+        }
+    };
+    // An exact zero that stands for the reference's +0: a k slice marks it -0,
+    // which its sums never are, so that the sum over the slices is -0 exactly
+    // where every slice says so.
+    const float plus = P ? -0.0f : 0.0f;
+    uint64_t zeros = 0;  // ... and those that are not settled yet
+    if (__builtin_amdgcn_ballot_w64(rare) != 0) {
+        uint64_t tiny = 0, none = 0;  // outputs of tiny activation rows; zeros of rows of +-0
+#pragma unroll
         for (int f = 0; f < RM * RN * 4; ++f) {
             const int mf = f / (RN * 4), n = (wn * RN + f / 4 % RN) * 16 + g * 4 + f % 4;
             const int ml = (wm * RM + mf) * 16 + i16;
-            const bool live = m0 + ml < M && n < nrows;
             const uint32_t xm = xmax_s[ml];
-            const float *const xr = X + (int64_t)min(m0 + ml, M - 1) * K;
-            const uint16_t *const wr = wrow0 + min(n, nrows - 1) * wpitch;
-            float *const o = out + (int64_t)(m0 + ml) * N + n;
-            const bool tiny = live && xm != 0 && xm < kTinyHiBits << 16;
-            const bool zero = live && !tiny && !P && *o == 0.0f;
-            if (tiny)  // this slice's chain
-                *o = SRC == kSrcPacked ? reference_chain(wr + 64 * c0, xr + 64 * c0, 64 * nch)
-                                    : chain_strided(wr + 64 * c0 * wstep, wstep, xr + 64 * c0,
-                                                    min(64 * nch, K - 64 * c0));
-            if (zero && xm == 0) *o = 0.0f;  // an activation row of +-0
-            const bool ask = zero && xm != 0;
-            if (__builtin_amdgcn_ballot_w64(ask) != 0) settle_zeros(o, ask ? 1u : 0u, xr, wr, 0, wstep, K);
+            const uint64_t bit = m0 + ml < M && n < nrows ? 1ull << f : 0;
+            const bool zero = acc[mf][f / 4 % RN][f % 4] == 0.0f;
+            if (xm == 0) none |= zero ? bit : 0;
+            else if (xm < kTinyHiBits << 16) tiny |= bit;
+            else zeros |= zero ? bit : 0;
         }
+        each_output(none, [&](bool mine, int, float *o, const uint16_t *, const float *) {
+            if (mine) *o = plus;
+        });
+        each_output(tiny, [&](bool mine, int, float *o, const uint16_t *wr, const float *xr) {
+            if (mine)  // this slice's chain (+0.0f: no -0 that would be taken for the mark)
+                *o = (SRC == kSrcPacked ? reference_chain(wr + 64 * c0, xr + 64 * c0, 64 * nch)
+                                        : chain_strided(wr + 64 * c0 * wstep, wstep, xr + 64 * c0,
+                                                        min(64 * nch, K - 64 * c0))) + (P ? 0.0f : -0.0f);
+        });
     }
+    uint32_t *const zeros_s = any_s + 1;
+    if (tid == 0) *any_s = *zeros_s = 0;
+    __syncthreads();
+    if (big) *any_s = 1;
+    if (zeros) atomicAdd(zeros_s, (uint32_t)__builtin_popcountll(zeros));
+    __syncthreads();
+    const bool again = *any_s != 0;
+    const int open = (int)*zeros_s;
+    __syncthreads();
+    if (!again && open == 0) return;
+    if (open != 0) {
+        // Exact zeros, of weight rows or columns that hold only +-0 (padding,
+        // pruning) or of products that cancel.  One pass over the tile takes the
+        // range of its weights and of each activation row, which settles them
+        // all (zero_is_plus), but for a tile whose weights or x reach down to
+        // underflow or up to inf.  What is left, and a few zeros alone against
+        // many chunks (a range of two rows takes 4 us, a chunk here about 0.5),
+        // is settled one by one, by the sum over the slices if k is split.
+        // Scanning rows and columns for each zero took longer than the product,
+        // most so for columns, 2N bytes between elements; with 256 zero columns,
+        // so / here (without them), us: columns [4096,14336] m = 5 / 64 1166 /
+        // 1252 against 0 / 0 (27.7 / 45).
+        const bool ranges = open * 8 > nch && K <= 1 << 24;
+        Range w;
+        uint32_t *const xlo_s = zeros_s + 1, *const w_s = xlo_s + MT;
+        if (ranges) {
+            constexpr int kSets = MT == 16 ? 2 : 4;
+            for (int i = tid; i < MT; i += 64 * NWV) xlo_s[i] = ~0u;
+            if (tid == 0) w_s[0] = ~0u, w_s[1] = 0;
+            __syncthreads();
+            uint32_t xlo[XI];
+#pragma unroll
+            for (int j = 0; j < XI; ++j) xlo[j] = ~0u;
+            if (SRC != kSrcPacked) w.put(wlast & 0x7fffu);  // (cut by the matrix's end)
+#pragma nounroll
+            for (int c = 0; c < nch; c += kSets) {
+                Regs q[kSets];
+#pragma unroll
+                for (int u = 0; u < kSets; ++u) load(c + u, q[u]);
+#pragma unroll
+                for (int u = 0; u < kSets; ++u) {
+#pragma unroll
+                    for (int j = 0; j < 4; ++j)
+#pragma unroll
+                        for (int v = 0; v < 4; ++v) {
+                            w.put(q[u].w[j][v] & 0x7fffu);
+                            w.put(q[u].w[j][v] >> 16 & 0x7fffu);
+                        }
+#pragma unroll
+                    for (int j = 0; j < XI; ++j)
+#pragma unroll
+                        for (int v = 0; v < 4; ++v) {
+                            const u32x4 *const x = q[u].x[j];
+                            if constexpr (FUSE) {
+                                xlo[j] = min(xlo[j], min((x[0][v] & 0x7fffffffu) - 1u, (x[1][v] & 0x7fffffffu) - 1u));
+                            } else {  // the hi term has x's exponent
+                                xlo[j] = min(xlo[j], min((x[0][v] << 16 & 0x7fffffffu) - 1u, (x[0][v] & 0x7fff0000u) - 1u));
+                            }
+                        }
+                }
+            }
+            w.over_wave();
+            if (lane == 0) {
+                atomicMin(&w_s[0], w.lo1);
+                atomicMax(&w_s[1], w.hi);
+            }
+#pragma unroll
+            for (int j = 0; j < XI; ++j) {
+                const int it = wave * XI + j;
+                if (it < 2 * XT) atomicMin(&xlo_s[(it >> 1) * 16 + i16], xlo[j]);
+            }
+            __syncthreads();
+            w.lo1 = w_s[0];
+            w.hi = w_s[1];
+        }
+        if (ranges || !P)
+            each_output(zeros, [&](bool mine, int ml, float *o, const uint16_t *wr, const float *xr) {
+                Range x;
+                x.lo1 = ranges ? xlo_s[ml] : 0u;
+                x.hi = xmax_s[ml];
+                const bool settled = ranges && zero_is_plus(x, w, K);
+                if (mine && settled) *o = plus;
+                const bool ask = !P && mine && !settled;
+                if (__builtin_amdgcn_ballot_w64(ask) != 0) settle_zeros(o, ask ? 1u : 0u, xr, wr, 0, wstep, K);
+            });
+        __syncthreads();
+    }
+    if (!again) return;
     // Outputs that are not finite: a weight or an activation is inf or NaN
     // (then every output of its row is inf or NaN in the reference), or a sum
     // overflowed.  Their class may be wrong: mid and lo are 0 against an inf
@@ -617,13 +727,6 @@ gemv_mfma_gemm_kernel(const uint16_t *__restrict__ W, const float *__restrict__ 
     // streamed again with it and those outputs take its result where that is
     // not finite either.  (Screening W in the loop and clearing such weights
     // for mid and lo cost 12-18% of it, for weights that hold none.)
-    if (tid == 0) *any_s = 0;
-    __syncthreads();
-    if (big) *any_s = 1;
-    __syncthreads();
-    const bool again = *any_s != 0;
-    __syncthreads();
-    if (!again) return;
     stream(std::integral_constant<int, kHi>{}, std::integral_constant<int, NS - 2>{});
 #pragma unroll
     for (int mf = 0; mf < RM; ++mf) {
@@ -657,11 +760,11 @@ split_x_planes_kernel(const float *__restrict__ X, uint16_t *__restrict__ XS, in
     }
 }
 
-// y[m][n] = P[0][m][n] + P[1][m][n] + ... in slice order, then the zero rule
-// of settle_zeros for one output: an exact zero is +0 when the activation row
-// or the weight row holds only +-0, else the reference chain's value.  Q
-// outputs per thread (4 where N is a multiple of 4, so that they share an
-// activation row): 16-byte loads, up to 8 slices' in flight.
+// y[m][n] = P[0][m][n] + P[1][m][n] + ... in slice order.  A partial of -0 says
+// that its slice's products sum to a zero that stands for the reference's +0: a
+// sum of -0 is +0; any other zero sum is settled (settle_zeros).  Q outputs per
+// thread (4 where N is a multiple of 4, so that they share an activation row):
+// 16-byte loads, up to 8 slices' in flight.
 // PACKED: W as in kSrcPacked, else rows (wstep 1) or columns (wstep N, batch slice
 // blockIdx.y) of any size.
 template <int Q, bool PACKED>
@@ -700,9 +803,14 @@ gemm_sum_slices_kernel(const float *__restrict__ P, int slices, float *__restric
 #pragma unroll
             for (int e = 0; e < Q; ++e) s[e] = add_lost(s[e], lost[e]);
         }
-        *reinterpret_cast<vec *>(Y + i) = s;
 #pragma unroll
-        for (int e = 0; e < Q; ++e) zero |= s[e] == 0.0f;
+        for (int e = 0; e < Q; ++e) {
+            // -0: every slice marked its zero as settled; +0: open, marked -0 in Y meanwhile.
+            const bool open = s[e] == 0.0f && !__builtin_signbit(s[e]);
+            zero |= open;
+            s[e] = s[e] == 0.0f ? (open ? -0.0f : 0.0f) : s[e];
+        }
+        *reinterpret_cast<vec *>(Y + i) = s;
     }
     // Rare: the wave settles its lanes' zeros together, over the outputs again.
     if (__builtin_amdgcn_ballot_w64(zero) == 0) return;
@@ -712,7 +820,7 @@ gemm_sum_slices_kernel(const float *__restrict__ P, int slices, float *__restric
         const vec s = *reinterpret_cast<const vec *>(Y + at);
         uint32_t zeros = 0;
 #pragma unroll
-        for (int e = 0; e < Q; ++e) zeros |= (i < count && s[e] == 0.0f ? 1u : 0u) << e;
+        for (int e = 0; e < Q; ++e) zeros |= (i < count && s[e] == 0.0f && __builtin_signbit(s[e]) ? 1u : 0u) << e;
         const int64_t m = at / N, n = at - m * N;
         if (__builtin_amdgcn_ballot_w64(zeros != 0) != 0)
             settle_zeros(Y + at, zeros, X + m * K, W + n * (wstep == 1 ? K : 1), wstep == 1 ? K : 1, wstep, K);

@@ -1426,7 +1426,7 @@ gemv_rd_mfma_rows16_kernel(const uint16_t *__restrict__ W, const float *__restri
                 float *ps = P + (int64_t)blockIdx.z * M * N + (int64_t)(m0 + i16) * N + row0 + g * 4;
 #pragma unroll
                 for (int r = 0; r < 4; ++r)
-                    if (live[0][r]) ps[r] = s[0][r];
+                    if (live[0][r]) ps[r] = s[0][r] + 0.0f;  // no -0: a mark there
             } else {
                 float *const y = Y + (int64_t)(m0 + i16) * N + row0 + g * 4;
                 uint32_t zeros = 0;

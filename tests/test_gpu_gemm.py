@@ -180,6 +180,50 @@ def test_columns_on_the_gemm_layout(hip, m, k, n, batch, offset, monkeypatch):
         check_or_bound(y[z], y_ref, xz, W.bf16_to_f32(wz), f"gemm cols {m}x{k}x{n} slice {z}")
 
 
+@pytest.mark.parametrize("m,k,n,batch,shared", [(20, 300, 70, 3, True), (130, 200, 300, 2, True),
+                                                (130, 1000, 259, 3, False)])
+def test_columns_of_padded_batches_and_a_shared_x(hip, m, k, n, batch, shared, monkeypatch):
+    """Weight slices further apart than k * n, one activation matrix for all
+    slices (ls = 0) or one each, and several activation tiles per slice (their
+    own order of tiles over the XCDs)."""
+    monkeypatch.setenv("DMC_HIP_CS_GEMM", "2")
+    rng = np.random.default_rng(m + k + n)
+    rs = k * n + 37
+    buf = W.bf16_rne(rng.standard_normal(batch * rs).astype(np.float32))
+    x = rng.standard_normal((1 if shared else batch, m, k)).astype(np.float32)
+    with hip.DeviceBuffer.from_numpy(buf) as dw, hip.DeviceBuffer.from_numpy(x) as dx, \
+            hip.DeviceBuffer(4 * batch * m * n) as dy:
+        assert hip.plan("cs", m, k, n, batch=batch, rs=rs, x_addr=dx.addr, w_addr=dw.addr).rows_or_rw == -256
+        hip.gemv_cs(dx, dw, dy, m, k, n, batch, 0 if shared else m * k, rs)
+        hip.synchronize()
+        y = dy.download(np.float32, (batch, m, n))
+    for z in range(batch):
+        wz = np.ascontiguousarray(buf[z * rs:z * rs + k * n].reshape(k, n).T)
+        check(y[z], oracle.matmul_bf16_t(x[0 if shared else z], wz), what=f"slice {z}")
+
+
+@pytest.mark.parametrize("m,k,n", [(33, 257, 300), (40, 4097, 600), (17, 1000, 259)])
+def test_columns_that_hold_zeros(hip, m, k, n, monkeypatch):
+    """Whole weight columns of zeros, unequal blocks of zeros that an activation
+    row's few nonzero elements never meet, and small integers, whose sums
+    cancel often: +0 as in the reference, one slice of k and several."""
+    monkeypatch.setenv("DMC_HIP_CS_GEMM", "2")
+    rng = np.random.default_rng(m + n)
+    x, w = case(m, k, n, seed=m + k, scale=0.02)
+    w[n // 3:] = 0
+    w[0], w[n - 1, 0] = 0, 0x8000
+    w[1, k // 2:] = 0
+    x[2], x[2, k - 1] = 0, 3  # one-hot
+    x[3], x[4] = 0, -0.0
+    x[5:12] = rng.integers(-1, 2, (7, k))
+    w[2:60] = W.bf16_rne(rng.integers(-1, 2, (58, k)).astype(np.float32))
+    y_ref = oracle.matmul_bf16_t(x, w)
+    assert y_ref[2, 1] == 0 and (y_ref[5:12, 2:60] == 0).any()
+    for slices in ("1", "64"):
+        monkeypatch.setenv("DMC_HIP_GEMM_MAX_SLICES", slices)
+        check(run_cs_dev(hip, x, w), y_ref, what=f"zeros, at most {slices} slices")
+
+
 FIRST_CALL_CAPTURED = """
 import sys
 import numpy as np
