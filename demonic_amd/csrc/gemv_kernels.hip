@@ -2711,6 +2711,44 @@ static double gemm_split(int64_t m, int64_t n, int64_t k, int64_t cus, int pair,
            (pl.kslices > 1 ? 5 + 0.42e-6 * ((double)pl.kslices * m * n * 4) : 0);
 }
 
+// The time in us of the gemm layout over rows of any length (its split in g), and
+// of the FMA kernels that take such calls (vec: the alignment's load width).
+// Both are fits to 2200 shapes on one box (2 to 512 activation rows, n 32 to
+// 32768, K 64 to 16384): rounds of workgroups x chunks at each tile height and
+// the slice pass; passes over W with the lanes' rows padded to whole windows, a
+// term in K and one in the outputs, whose reductions an 8- or 16-row FMA
+// workgroup of short rows is bound by.  Of 1161 of those shapes above the
+// multiply-adds that the rule asks for, 108 ran more than 3% slower on the gemm
+// layout; compared by these times, 16 of the 1010 that still take it.
+static double rows_gemm_us(const RdProblem &p, int64_t cus, const RdPlan &g) {
+    const int64_t tiles = (p.n + g.rpw - 1) / g.rpw * ((p.m + g.mt - 1) / g.mt);
+    const double chunks = (double)((tiles * g.kslices + cus - 1) / cus) * g.kchunks;
+    const double mb = 4e-6 * (double)g.kslices * p.m * p.n;  // partial sums
+    const bool split = g.kslices > 1;
+    switch (g.mt) {
+    case 16: return 3 + 0.95 * chunks + (split ? 1.5 + 0.3 * g.kslices + 1.6 * mb : 0);
+    case 32: return 5 + 1.35 * chunks + (split ? 1 + 0.15 * g.kslices + 0.9 * mb : 0);
+    default: return 9 + 1.6 * chunks + (split ? 0.5 + 0.1 * g.kslices + 0.85 * mb : 0);
+    }
+}
+
+static double rd_fma_us(const RdProblem &p, int vec, int64_t cus) {
+    RdPlan sp{};
+    const bool stream = vec == 8 && plan_stream(p.m, p.k, &p.n, 1, cus, sp);
+    const int mt = stream ? sp.mt : mt_for(p.m);
+    const int64_t window = stream ? 512 * sp.waves : 64 * kWaves * vec;  // k elements per load of a workgroup
+    const double w = 2e-6 * (double)p.n * ((p.k + window - 1) / window * window) * ((p.m + mt - 1) / mt);
+    const double k = 1e-3 * p.k, out = 1e-6 * (double)p.m * p.n;
+    if (stream)
+        return mt == 8   ? 2.2 + 0.295 * w + 2.6 * k
+               : mt == 4 ? 0.5 + 0.19 * w + 0.9 * k
+               : mt == 2 ? 0.5 + 0.135 * w + 0.2 * k + 150 * out
+                         : 1 + 0.1 * w;
+    const double per_mb = mt == 16 ? 1.5 : mt == 8 ? (vec == 1 ? 0.8 : 0.57) : mt == 4 ? (vec == 1 ? 0.4 : 0.26)
+                                                                               : (vec == 1 ? 0.34 : 0.18);
+    return 1 + per_mb * w + 0.3 * k + (mt == 16 ? 110 : 280) * out;
+}
+
 // At most 2 * wg_per_cu workgroups per CU hold a slice's sums of rpw weight rows
 // by mt * pair activation rows each: two tiles of 256 x 64 on one workgroup per
 // CU is the largest of the forms (the others: half of that).
@@ -3052,7 +3090,10 @@ RdPlan plan_rd(const RdProblem &p, int num_cus) {
     // decides: K odd, up to 2^25 multiply-adds ([2001,1001] m = 16 12.7
     // against 14.7; [4000,2052] m = 5, above, 19.4 / 14.3); K a multiple of 8,
     // up to 2^26 ([11008,1000] m = 3 8.1 against 13.4, [1000,4104] m = 16 19.0
-    // / 18.3), and two rows ([11008,4104] 22.1 / 24).
+    // / 18.3), and two rows ([11008,4104] 22.1 / 24).  Above that, whichever
+    // rows_gemm_us and rd_fma_us put ahead: a small W has few 256-row tiles to
+    // deal out and is in a cache for the FMA kernels' further passes ([1088,824]
+    // m = 167 16.6 against 24.9, [59,5008] m = 114 9.0 / 30.3).
     const int rows_env = env_int("DMC_HIP_RD_GEMM_ROWS", 1);  // 0: never; 2: wherever it applies
     if (rows_env != 0 && mfma_min_m > 0 && p.k >= 1 && p.ldw == p.k && p.ldx == p.k && p.ldy == p.n &&
         (int64_t)kWideRows * p.k * 2 + 16 <= INT32_MAX && p.m * p.k * 4 <= INT32_MAX &&
@@ -3067,10 +3108,11 @@ RdPlan plan_rd(const RdProblem &p, int num_cus) {
         mp.rpw = 256;
         gemm_split(p.m, p.n, p.k, cus, 1, 1, mp);
         mp.xfuse = true;
+        const bool ahead = rows_env == 2 || rows_gemm_us(p, cus, mp) < rd_fma_us(p, pl.vec, cus);
         mp.workspace_bytes = mp.kslices > 1 ? (size_t)mp.kslices * p.m * p.n * 4 : 0;
         mp.grid_x = (p.n + mp.rpw - 1) / mp.rpw;
         mp.grid_y = (p.m + mp.mt - 1) / mp.mt;
-        if (mp.grid_x * mp.grid_y * mp.kslices <= INT32_MAX) return mp;
+        if (ahead && mp.grid_x * mp.grid_y * mp.kslices <= INT32_MAX) return mp;
     }
 
     // Streaming kernel: packed 128-bit rows and k within the register budget.

@@ -697,6 +697,19 @@ def test_f32_activation_rows_per_workgroup(monkeypatch):
     assert d.plan_f32(16, 4097, 64, x_addr=256, w_addr=256).mt == 16      # general
 
 
+@pytest.mark.parametrize("m,n,k,off,gemm", [
+    (167, 1088, 824, 0, False), (111, 856, 904, 0, False), (35, 104, 9276, 0, False), (114, 59, 5008, 2, False),
+    (61, 473, 1720, 2, False), (4, 12796, 1712, 0, False), (2, 11008, 4097, 0, True), (33, 11008, 4097, 0, True),
+    (16, 4096, 4104, 0, True), (3, 11008, 4104, 0, True), (8, 1000, 4104, 0, False), (356, 7296, 7985, 0, True),
+    (40, 2000, 4097, 0, True)])
+def test_rows_of_any_length_take_the_faster_kernels(m, n, k, off, gemm):
+    """Above the least multiply-adds the gemm layout takes rows of any length
+    where its time, by the planner's estimate, is below the FMA kernels': not
+    where a small W leaves it a handful of 256-row tiles."""
+    p = d.plan("rd", m, k, n, x_addr=256, w_addr=256 + off)
+    assert (p.slices == -8) == gemm, p
+
+
 @pytest.mark.parametrize("k,n,most", [(4096, 14336, 8), (7168, 14336, 8), (14336, 14336, 4)])
 def test_f32_group_rows_stay_within_a_grid(k, n, most):
     """The group kernels' activation groups are a grid's second extent, at most
