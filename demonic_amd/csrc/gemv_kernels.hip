@@ -777,13 +777,22 @@ __device__ __forceinline__ void rd_group_body(const WT *__restrict__ W, const fl
         });
 }
 
+// f32: the first of the activation rows of group blockIdx.y.  A last group that
+// would reach past M starts earlier, and its first rows' outputs are stored
+// twice, with the same bits.
+template <int MT>
+__device__ __forceinline__ int64_t act_group(int M) {
+    return min((int64_t)blockIdx.y * MT, (int64_t)M - MT);
+}
+
 template <typename WT, int KV, int MT>
 __global__ void __launch_bounds__(64 * kX14Waves)
 gemv_rd_stream_x14_kernel(const WT *__restrict__ W, const float *__restrict__ X, float *__restrict__ Y, int N, int K,
-                          int64_t ys_act, int64_t ys_row) {
-    if constexpr (sizeof(WT) == 4) {  // activation rows MT * blockIdx.y on
-        X += (int64_t)blockIdx.y * MT * K;
-        Y += (int64_t)blockIdx.y * MT * ys_act;
+                          int64_t ys_act, int64_t ys_row, int M) {
+    if constexpr (sizeof(WT) == 4) {
+        const int64_t m0 = act_group<MT>(M);
+        X += m0 * K;
+        Y += m0 * ys_act;
     }
     rd_group_body<WT, KV, MT, kX14Waves>(W, X, Y, N, K, ys_act, ys_row);
 }
@@ -807,9 +816,10 @@ gemv_rd_stream_x4_kernel(const uint16_t *__restrict__ W, const float *__restrict
 template <int KV, int MT>
 __global__ void __launch_bounds__(512)
 gemv_rd_stream_x8f_kernel(const float *__restrict__ W, const float *__restrict__ X, float *__restrict__ Y, int N,
-                          int K, int64_t ys_act, int64_t ys_row) {
-    X += (int64_t)blockIdx.y * MT * K;  // activation rows MT * blockIdx.y on
-    Y += (int64_t)blockIdx.y * MT * ys_act;
+                          int K, int64_t ys_act, int64_t ys_row, int M) {
+    const int64_t m0 = act_group<MT>(M);
+    X += m0 * K;
+    Y += m0 * ys_act;
     rd_group_body<float, KV, MT, 8>(W, X, Y, N, K, ys_act, ys_row);
 }
 
@@ -3473,7 +3483,7 @@ hipError_t launch_rd(const RdProblem &p, const RdPlan &pl, void *workspace, hipS
             return hipErrorInvalidValue;
 #define DMC_X14(KV, MT)                                                                                      \
     hipLaunchKernelGGL((gemv_rd_stream_x14_kernel<uint16_t, KV, MT>), dim3((unsigned)pl.grid_x),               \
-                       dim3(64 * kX14Waves), 0, s, p.w, p.x, p.y, (int)p.n, (int)p.k, (int64_t)p.ldy, (int64_t)1)
+                       dim3(64 * kX14Waves), 0, s, p.w, p.x, p.y, (int)p.n, (int)p.k, (int64_t)p.ldy, (int64_t)1, (int)p.m)
         switch (pl.kvec * 10 + (int)p.m) {
         case 11: DMC_X14(1, 1); break;
         case 21: DMC_X14(2, 1); break;
@@ -3582,16 +3592,17 @@ hipError_t launch_cs(const CsProblem &p, const CsPlan &pl, void *workspace, hipS
 // [8192,2048] m = 8 25.2 / 13.6, [2000,12000] m = 8 109 / 45.  Not on short
 // rows, whose lanes would idle ([8192,1024] m = 16 22.6 / 22.7, [30000,512]
 // 22.2 / 29.8), nor on few workgroups ([1024,4096] m = 8 8.1 / 10.2;
-// [600,14336] m = 6 32.1 / 42.0).  Above 8 rows a matrix of up to 64 MiB keeps
+// [2144,1028] m = 8 7.4 / 8.0; [600,14336] m = 6 32.1 / 42.0).  Above 8 rows a matrix of up to 64 MiB keeps
 // its plan of 4 rows per workgroup, whose passes meet it in the last-level
 // cache ([4096,4096] m = 16 49 us).
 static bool f32_group_rows(const F32Problem &p, int64_t cus, F32Plan &pl) {
-    const int env = env_int("DMC_HIP_F32_GROUP_M", 1);  // 0: never; 2: wherever it applies
-    if (env == 0 || p.m <= kX14MaxM || p.k < 4 || p.k > kX14MaxK || p.k % 4 != 0 || p.ldw != p.k || p.ldx != p.k ||
-        !aligned(p.w, 16) || !aligned(p.x, 16) || env_int("DMC_HIP_F32_STREAM", 1) == 0)
+    if (p.m <= kX14MaxM || p.k < 4 || p.k > kX14MaxK || p.k % 4 != 0 || p.ldw != p.k || p.ldx != p.k ||
+        !aligned(p.w, 16) || !aligned(p.x, 16))
         return false;
     const int64_t g16 = (p.n + 15) / 16;
-    if (env != 2 && (p.k <= 1024 || g16 < (p.k <= 4096 ? cus / 2 : cus / 4) ||
+    const int env = env_int("DMC_HIP_F32_GROUP_M", 1);  // 0: never; 2: wherever it applies
+    if (env == 0 || env_int("DMC_HIP_F32_STREAM", 1) == 0) return false;
+    if (env != 2 && (p.k <= 1024 || g16 < (p.k <= 2048 ? cus * 5 / 8 : p.k <= 4096 ? cus / 2 : cus / 4) ||
                      (p.m > kGroupMaxMF32 && p.n * p.k * 4 <= (int64_t)64 << 20)))
         return false;
     const int waves = p.k <= 4096 ? 8 : kX14Waves;
@@ -3748,18 +3759,15 @@ hipError_t launch_f32(const F32Problem &p, const F32Plan &pl, hipStream_t s) {
             p.k > kX14MaxK || p.k < 1 || p.k % 4 != 0 || p.ldw != p.k || p.ldx != p.k || !aligned(p.w, 16) ||
             !aligned(p.x, 16) || pl.grid_x != (p.n + 15) / 16)
             return hipErrorInvalidValue;
-        // The whole groups in one launch, what is left in a second.  A launch
-        // per group / so, us: W[14336,4096] m = 16 / 64 86.6 / 350 against 76.3 /
-        // 291, [4096,14336] m = 16 147 / 139, [30000,8192] m = 13 677 / 641.
-        for (int64_t m0 = 0; m0 < p.m;) {
-            const int mc = (int)std::min<int64_t>(pl.mt, p.m - m0);
-            const int64_t groups = (p.m - m0) / mc;
-            const float *const x = p.x + m0 * p.ldx;
-            float *const y = p.y + m0 * p.ys_act;
-            m0 += groups * mc;
-            const dim3 grid((unsigned)pl.grid_x, (unsigned)groups), block(64 * pl.waves);
+        // One launch of the groups.  A launch per group / so, us: W[14336,4096]
+        // m = 16 / 64 86.6 / 350 against 76.3 / 291, [4096,14336] m = 16 147 /
+        // 139, [30000,8192] m = 13 677 / 641; few workgroups a group share the
+        // device, [1181,7644] m = 7 31.5 / 18.1.
+        if (pl.mt > p.m) return hipErrorInvalidValue;
+        const dim3 grid((unsigned)pl.grid_x, (unsigned)pl.grid_y), block(64 * pl.waves);
 #define DMC_F32G(KERNEL, ...)                                                                                 \
-    hipLaunchKernelGGL((KERNEL<__VA_ARGS__>), grid, block, 0, s, p.w, x, y, (int)p.n, (int)p.k, p.ys_act, p.ys_row); \
+    hipLaunchKernelGGL((KERNEL<__VA_ARGS__>), grid, block, 0, s, p.w, p.x, p.y, (int)p.n, (int)p.k, p.ys_act,    \
+                       p.ys_row, (int)p.m);                                                                   \
     break
 #define DMC_F32G4(BASE, KERNEL, ...)                                                                          \
     case BASE + 1: DMC_F32G(KERNEL, __VA_ARGS__, 1);                                                          \
@@ -3772,21 +3780,18 @@ hipError_t launch_f32(const F32Problem &p, const F32Plan &pl, hipStream_t s) {
     case BASE + 6: DMC_F32G(KERNEL, __VA_ARGS__, 6);                                                          \
     case BASE + 7: DMC_F32G(KERNEL, __VA_ARGS__, 7);                                                          \
     case BASE + 8: DMC_F32G(KERNEL, __VA_ARGS__, 8);
-            switch (pl.waves * 100 + pl.kvec * 10 + mc) {
-                DMC_F32G8(810, gemv_rd_stream_x8f_kernel, 1)
-                DMC_F32G8(820, gemv_rd_stream_x8f_kernel, 2)
-                DMC_F32G8(100 * kX14Waves + 20, gemv_rd_stream_x14_kernel, float, 2)
-                DMC_F32G4(100 * kX14Waves + 30, gemv_rd_stream_x14_kernel, float, 3)
-                DMC_F32G4(100 * kX14Waves + 40, gemv_rd_stream_x14_kernel, float, 4)
-            default: return hipErrorInvalidValue;
-            }
+        switch (pl.waves * 100 + pl.kvec * 10 + pl.mt) {
+            DMC_F32G8(810, gemv_rd_stream_x8f_kernel, 1)
+            DMC_F32G8(820, gemv_rd_stream_x8f_kernel, 2)
+            DMC_F32G8(100 * kX14Waves + 20, gemv_rd_stream_x14_kernel, float, 2)
+            DMC_F32G4(100 * kX14Waves + 30, gemv_rd_stream_x14_kernel, float, 3)
+            DMC_F32G4(100 * kX14Waves + 40, gemv_rd_stream_x14_kernel, float, 4)
+        default: return hipErrorInvalidValue;
+        }
 #undef DMC_F32G8
 #undef DMC_F32G4
 #undef DMC_F32G
-            const hipError_t e = hipGetLastError();
-            if (e != hipSuccess) return e;
-        }
-        return hipSuccess;
+        return hipGetLastError();
     }
     if (pl.kvec > 0) {
         // The shapes the streaming kernel assumes (plan_f32's conditions).

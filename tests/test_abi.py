@@ -718,6 +718,10 @@ def test_f32_group_rows_stay_within_a_grid(k, n, most):
     assert (p.rows_per_group, p.mt, p.grid_y) == (16, most, 65535), p
     p = d.plan_f32(65535 * most + 1, k, n, x_addr=256, w_addr=256)
     assert (p.kvec, p.mt) == (0, 16) and p.grid_y <= 65535, p
+    # the groups of one launch: mt rows each, the last one starting where it ends at m
+    p = d.plan_f32(7, 7644, 1181, x_addr=256, w_addr=256)
+    assert (p.rows_per_group, p.mt, p.grid_y) == (16, 4, 2), p
+    assert d.plan_f32(8, 1028, 2144, x_addr=256, w_addr=256).rows_per_group == 4  # few 16-row workgroups
 
 
 def test_f32_entries_reject_gemm_shapes_before_touching_a_device():

@@ -1,6 +1,6 @@
 """GPU parity of the f32 group kernels at 5 and more activation rows: W read
-once per 8 rows (4 where a lane holds 3 or 4 windows), the rows split evenly
-over the groups."""
+once per 8 rows (4 where a lane holds 3 or 4 windows), the rows split over
+the groups of one launch."""
 import numpy as np
 import pytest
 
