@@ -182,9 +182,10 @@ __device__ float settle_zero(float s, bool zero, const float *x, const uint16_t 
 
 // ---- zero outputs of the MFMA kernels ------------------------------------------
 //
-// Out of the kernels' code (settle_zeros is not inlined): expanded at their
-// unrolled outputs, this rare path set their registers (gemm_sum_slices_kernel:
-// 149 VGPRs, 3 waves per SIMD, and 199 SGPRs spilled, against 8 waves and none).
+// The scans and chains are functions of their own, called from rolled loops:
+// expanded at the kernels' unrolled outputs, this rare path set their registers
+// (gemm_sum_slices_kernel: 149 VGPRs, 3 waves per SIMD, and 199 SGPRs spilled,
+// against 63, 8 waves and none).
 
 // Least and greatest magnitude of a row: lo - 1 (zeros wrap to the top), hi.
 struct Range {
@@ -331,13 +332,29 @@ __device__ __noinline__ float lane_chain(const uint16_t *w, int64_t wstep, const
     return chain_strided(w, wstep, x, K);
 }
 
+// The chains of the lanes that ask (s for the others): one after another by the
+// whole wave where they are few and the weights packed, else one per lane.
+__device__ __forceinline__ float few_or_lane_chains(bool ask, float s, const uint16_t *w, const float *x, int K,
+                                                    int64_t wstep = 1) {
+    uint64_t todo = __builtin_amdgcn_ballot_w64(ask);
+    if (wstep > 1 || K > 1 << 24 || __builtin_popcountll(todo) > 6) {
+        if (ask) s = lane_chain(w, wstep, x, K);
+        return s;
+    }
+    for (; todo; todo &= todo - 1) {
+        const int j = __builtin_ctzll(todo);
+        const float c = wave_chain(readlane_ptr(w, j), readlane_ptr(x, j), K);
+        if ((int)(threadIdx.x & 63) == j) s = c;
+    }
+    return s;
+}
+
 // The reference's values for outputs whose sums are exactly zero: a lane's are
 // y[e] where bit e of `zeros` is set (e < 4), of its activation row x and the
 // weights w + e * wpitch, wstep elements between consecutive k.  All 64 lanes
 // call this.  The ranges of each distinct activation and weight row are taken
 // once by the whole wave and settle almost every zero (zero_is_plus); the chains
-// left, if any, run one after another by the whole wave where they are few and
-// the weights packed, else one per lane.
+// of the others follow.
 __device__ __forceinline__ void settle_zeros(float *y, uint32_t zeros, const float *x, const uint16_t *w, int64_t wpitch,
                                           int64_t wstep, int K) {
     const bool ranges = K <= 1 << 24;
@@ -360,17 +377,7 @@ __device__ __forceinline__ void settle_zeros(float *y, uint32_t zeros, const flo
                 if (w == wj) plus |= zero_is_plus(rx, r, K);
                 todo &= ~__builtin_amdgcn_ballot_w64(w == wj);
             }
-        float v = 0.0f;
-        uint64_t chains = __builtin_amdgcn_ballot_w64(zero && !plus);
-        if (wstep > 1 || !ranges || __builtin_popcountll(chains) > 6) {
-            if (zero && !plus) v = lane_chain(w, wstep, x, K);
-        } else {
-            for (; chains; chains &= chains - 1) {
-                const int j = __builtin_ctzll(chains);
-                const float c = wave_chain(readlane_ptr(w, j), readlane_ptr(x, j), K);
-                if ((int)(threadIdx.x & 63) == j) v = c;
-            }
-        }
+        const float v = few_or_lane_chains(zero && !plus, 0.0f, w, x, K, wstep);
         if (zero) y[e] = v;
     }
 }
@@ -399,8 +406,9 @@ __device__ __forceinline__ void settle_zeros(float *y, uint32_t zeros, const flo
 // Zeros: the MFMA rounds a nonzero sum smaller than half the least f32
 // subnormal to +0 whatever its sign, where the reference's fmaf gives the
 // signed zero (every product underflowing negative ends at -0).  So an output
-// that comes out exactly zero is settled at the end (settle_zeros above): +0
-// where the two rows' magnitudes leave the chain no room to underflow or
+// that comes out exactly zero is settled at the end: +0 where the activation or
+// the weight row holds only +-0 or (the gemm layout and the slice sum,
+// settle_zeros) the two rows' magnitudes leave the chain no room to underflow or
 // overflow, otherwise the chain itself, fmaf over ascending k from +0.
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
@@ -535,6 +543,73 @@ constexpr uint32_t kTinyHiBits = 0x0d80u;
 
 __device__ __forceinline__ uint32_t hi_max(uint32_t mx) { return max(mx & 0xffffu, mx >> 16); }
 __device__ __forceinline__ bool tiny_row(uint32_t mx) { return mx != 0 && mx < kTinyHiBits; }
+
+// Wave-uniform: does the row hold an element other than +-0?  (bytes: 16 * n16)
+__device__ bool wave_row_nonzero(const void *row, int n16, uint32_t mask) {
+    const u32x4 *p = reinterpret_cast<const u32x4 *>(row);
+    uint32_t acc = 0;
+    for (int c = threadIdx.x & 63; c < n16; c += 64) {
+        const u32x4 v = p[c];
+        acc |= (v[0] | v[1] | v[2] | v[3]) & mask;
+    }
+    return __builtin_amdgcn_ballot_w64(acc != 0) != 0;
+}
+
+// One wave's outputs after the zero rule above.  Lane l holds s[t][r] for
+// weight row base[t] + 4(l/16) + r of W and activation row m of X; `live`
+// marks the ones it stores.  All 64 lanes call this; the rows are walked
+// wave-uniformly.  Rare path: entered only when some output is exactly zero.
+// The rows16 and wide layouts' rule: +0 where the activation row or the weight row
+// holds only +-0, else the chain, always.  Their outputs are a few per wave and
+// the scans stay in the kernel (out of it, as in settle_zeros, [102144,1024] at
+// 3 activation rows took 38.0 us for 36.3).
+template <int T>
+__device__ void settle_tile_zeros(f32x4 (&s)[T], const bool (&live)[T][4], const int (&base)[T], const uint16_t *W,
+                             const float *X, int K, int m) {
+    const int g = (threadIdx.x & 63) >> 4;
+    bool zero[T][4];
+    bool any = false;
+#pragma unroll
+    for (int t = 0; t < T; ++t)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            zero[t][r] = live[t][r] && s[t][r] == 0.0f;
+            any |= zero[t][r];
+        }
+    if (__builtin_amdgcn_ballot_w64(any) == 0) return;
+    // Is this lane's activation row nonzero?  Lanes j = 0..15 hold every row
+    // the wave has.
+    bool xnz = false;
+    for (int j = 0; j < 16; ++j) {
+        const int mj = __builtin_amdgcn_readlane(m, j);
+        if (__builtin_amdgcn_ballot_w64(any && m == mj) != 0) {
+            const bool nz = wave_row_nonzero(X + (int64_t)mj * K, K / 4, 0x7fffffffu);
+            if (m == mj) xnz = nz;
+        }
+    }
+    // Zero outputs become +0, or the chain's value where both rows are nonzero.
+    bool chain[T][4];
+#pragma unroll
+    for (int t = 0; t < T; ++t)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            chain[t][r] = false;
+            if (zero[t][r]) s[t][r] = 0.0f;
+            for (int gq = 0; gq < 4; ++gq) {
+                const bool ask = zero[t][r] && xnz && g == gq;
+                if (__builtin_amdgcn_ballot_w64(ask) == 0) continue;
+                const int row = base[t] + 4 * gq + r;
+                const bool nz = wave_row_nonzero(W + (int64_t)row * K, K / 8, 0x7fff7fffu);
+                if (ask) chain[t][r] = nz;
+            }
+        }
+#pragma unroll
+    for (int t = 0; t < T; ++t)
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+            s[t][r] = few_or_lane_chains(chain[t][r], s[t][r], W + (int64_t)(base[t] + 4 * g + r) * K,
+                                         X + (int64_t)m * K, K);
+}
 
 // Weight and x tiles in LDS hold rows of 128 bytes, 8 pieces of 16, back to
 // back, with piece p of row r stored at position p ^ ((r / 2) mod 8).  A

@@ -1188,20 +1188,12 @@ gemv_rd_mfma_wide_kernel(const uint16_t *__restrict__ W, const float *__restrict
                     acc[t][r] = reference_chain(W + (int64_t)(row0 + base[t] + g * 4 + r) * K,
                                                 X + (int64_t)(m0 + i16) * K, K);
     }
+    settle_tile_zeros(acc, live, base, W + (int64_t)row0 * K, X + (int64_t)m0 * K, K, i16);
 #pragma unroll
-    for (int t = 0; t < 2; ++t) {
-        const int64_t row = row0 + base[t] + g * 4;
-        float *const y = Y + (int64_t)(m0 + i16) * N + row;
-        uint32_t zeros = 0;
+    for (int t = 0; t < 2; ++t)
 #pragma unroll
         for (int r = 0; r < 4; ++r)
-            if (live[t][r]) {
-                y[r] = acc[t][r];
-                zeros |= (acc[t][r] == 0.0f ? 1u : 0u) << r;
-            }
-        if (__builtin_amdgcn_ballot_w64(zeros != 0) != 0)
-            settle_zeros(y, zeros, X + (int64_t)(m0 + i16) * K, W + row * K, K, 1, K);
-    }
+            if (live[t][r]) Y[(int64_t)(m0 + i16) * N + row0 + base[t] + g * 4 + r] = acc[t][r];
 }
 
 // Fifth MFMA layout ("rows16"), for a few activation rows: 16 weight rows per
@@ -1421,6 +1413,7 @@ gemv_rd_mfma_rows16_kernel(const uint16_t *__restrict__ W, const float *__restri
             f32x4 s[1] = {red[t * 64 + lane]};
 #pragma unroll
             for (int w = 1; w < 8; ++w) s[0] += red[(w * T + t) * 64 + lane];
+            const int base[1] = {0};
             bool live[1][4];
 #pragma unroll
             for (int r = 0; r < 4; ++r) live[0][r] = i16 < mrows && g * 4 + r < nrows;
@@ -1438,16 +1431,10 @@ gemv_rd_mfma_rows16_kernel(const uint16_t *__restrict__ W, const float *__restri
                 for (int r = 0; r < 4; ++r)
                     if (live[0][r]) ps[r] = s[0][r] + 0.0f;  // no -0: a mark there
             } else {
-                float *const y = Y + (int64_t)(m0 + i16) * N + row0 + g * 4;
-                uint32_t zeros = 0;
+                settle_tile_zeros(s, live, base, W + (int64_t)row0 * K, X + (int64_t)m0 * K, K, i16);
 #pragma unroll
                 for (int r = 0; r < 4; ++r)
-                    if (live[0][r]) {
-                        y[r] = s[0][r];
-                        zeros |= (s[0][r] == 0.0f ? 1u : 0u) << r;
-                    }
-                if (__builtin_amdgcn_ballot_w64(zeros != 0) != 0)
-                    settle_zeros(y, zeros, X + (int64_t)(m0 + i16) * K, W + (int64_t)(row0 + g * 4) * K, K, 1, K);
+                    if (live[0][r]) Y[(int64_t)(m0 + i16) * N + row0 + g * 4 + r] = s[0][r];
             }
         }
     }
