@@ -592,6 +592,7 @@ gemv_mfma_gemm_kernel(const uint16_t *__restrict__ W, const float *__restrict__ 
     // The lane's outputs of `mask` (bit f, in the order above), some lane's at a
     // time: body(is it this lane's, activation row of the tile, address, w, x).
     auto each_output = [&](uint64_t mask, auto body) __attribute__((always_inline)) {
+        if (__builtin_amdgcn_ballot_w64(mask != 0) == 0) return;
 #pragma nounroll
         for (int f = 0; f < RM * RN * 4; ++f) {
             const bool mine = (mask >> f & 1) != 0;
