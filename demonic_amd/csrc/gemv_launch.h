@@ -59,7 +59,8 @@ struct CsProblem {
 struct RdPlan {
     bool mfma;  // skinny-M MFMA kernel
     int mkind;  // MFMA layout: 6 = 256 rows per workgroup, weights and x staged through LDS;
-                // 7 = 16 rows per workgroup read whole, waves own lines of each window
+                // 7 = 16 rows per workgroup read whole, waves own lines of each window;
+                // 8 = gemm, 32 rows per wave against mt * mtiles activation rows
     int vec;    // bf16 elements per lane per weight load (8 = 128-bit loads)
     int rows;   // weight rows per step (streaming) / per workgroup (general)
     int mt;     // activation rows per workgroup (skinny-M tile)
@@ -140,7 +141,8 @@ size_t max_split_bytes(int num_cus);
 hipError_t launch_rd(const RdProblem &p, const RdPlan &plan, void *workspace, hipStream_t stream);
 hipError_t launch_rd_group(const RdGroup &g, const RdPlan &plan, hipStream_t stream);
 // The gemm layout (plan.mkind == 8; over columns: CsPlan::gemm), and the sum of
-// k-slice partials part[slice][m][n] into p.y in slice order with the zero rule.
+// k-slice partials part[slice][m][n] into p.y in slice order with the zero rule (a
+// partial of -0 says that its zero is settled).
 hipError_t launch_gemm(const RdProblem &p, const RdPlan &plan, void *workspace, hipStream_t stream);
 hipError_t launch_gemm_cs(const CsProblem &p, const CsPlan &plan, void *workspace, hipStream_t stream);
 hipError_t launch_sum_slices(const float *part, int slices, const RdProblem &p, hipStream_t stream);

@@ -234,15 +234,16 @@ int32_t dmc_hip_gemv_rd_grouped(int64_t count, const int64_t *x_devs, const int6
  * windows per lane (with vec < 8, the variant that reads misaligned rows with
  * unaligned 128-bit loads), 0 the general kernel, -6 / -7 / -8 the MFMA layouts
  * (wide: 256 rows per workgroup; rows16: 16 rows per block; gemm: 256 rows
- * against 16, 32 or 64 activation rows, k possibly split; with vec < 8, or K no
- * multiple of 64, over rows of any length and alignment; mt activation rows);
+ * against one tile of mt = 16, 32 or 64 activation rows, or two of 64, which mt
+ * does not tell apart, k possibly split; with vec < 8, or K no multiple of 64,
+ * over rows of any length and alignment, one tile);
  * waves and rows_per_group (weight rows per workgroup) describe the workgroup.
  * Column-stream layout: `vec` is the row alignment as above; rows_or_rw <= 0 is
  * the streaming kernel (512 columns per workgroup, or with -G row groups per
  * wave 512/G, rows_per_group k rows per slice; with vec < 8 it reads
  * misaligned rows and the slice pass applies the last k row), > 0 the
  * general kernel's k rows per wave-wide load, -256 the gemm layout over
- * columns (MFMA, 256 columns against 32 or 64 activation rows per workgroup)
+ * columns (MFMA, 256 columns against 16, 32 or 64 activation rows per workgroup)
  * (rows_per_group columns per workgroup); `slices` k slices, summed by a
  * second launch into `workspace_bytes` of partials. */
 int32_t dmc_hip_plan(int32_t layout_rd, int64_t x_addr, int64_t w_addr, int64_t m, int64_t k,
